@@ -2325,6 +2325,9 @@ int ps_read_neighbors(ps_system *s, uint32_t *counts, uint32_t *table)
                 const size_t at = (((size_t)(i >> 6) * kq + (k >> 2)) * 64 + (i & 63)) * 4 + (k & 3);
                 uint32_t e = k < cnt[i] ? raw[at] : 0u;
                 if (d && k < cnt[i]) {
+                    // 16-bit entries, eight to 16 bytes
+                    const size_t a16 = (((size_t)(i >> 6) * kq + (k >> 3)) * 64 + (i & 63)) * 8 + (k & 7);
+                    e = reinterpret_cast<const uint16_t *>(raw.data())[a16];
                     const uint32_t c = e / ps::kStageChunk;
                     e = c < d->nchunks && c < ps::kStageChunks ? d->src[c] + e % ps::kStageChunk
                                                                : 0xffffffffu;

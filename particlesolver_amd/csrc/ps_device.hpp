@@ -48,6 +48,110 @@ __device__ __forceinline__ const uint4 *nbr_lane(const DevBuffers &b, uint32_t i
     return reinterpret_cast<const uint4 *>(b.nbr) + (size_t)(i >> 6) * b.kq * 64 + (i & 63);
 }
 
+// A staged unit's table holds 16-bit LDS indices: eight entries (two chunks
+// of four) per uint4, in the first half of its particles' share of nbr.
+// Chunk m (entries 4m..4m+3) is the uint2 nbr16_chunk(b, i, m); the two
+// chunks of a pair and consecutive lanes are contiguous.
+__device__ __forceinline__ const uint2 *nbr16_chunk(const DevBuffers &b, uint32_t i, uint32_t m)
+{
+    return reinterpret_cast<const uint2 *>(b.nbr) +
+           (((size_t)(i >> 6) * b.kq + (m >> 1)) * 64 + (i & 63)) * 2 + (m & 1u);
+}
+
+// One lane's share of a staged particle's table, its chunks first, first +
+// STRIDE, ...; the first PRE of them are loaded by load(), which a kernel
+// calls before it stages its unit, so these loads and the staging loads wait
+// together.  (The loads do not depend on the entry count: they are clamped
+// to the particle's share of the table, and chunks past the count hold
+// whatever is there and are never visited.)  The chunks a particle uses are
+// visited whole: the builder pads the last one with the sentinel record,
+// which fails every pair test.  32 entries a particle (PRE chunks of two
+// halves, or of four quarters) cover the mean of about 28.
+// With 32-bit entries fetched as they are visited, at 4,194,304 particles
+// (a table of 470 MB, past the 256 MB of the last-level cache) lambda took
+// 200 us, the solve 221 and finalize 286; with 16-bit entries loaded ahead
+// 159, 200 and 241.  At 1,048,576: 38.0, 43.9 and 56.1 us, now 35.6, 43.5
+// (bound by VALU issue) and 52.1.
+// PIPE: the LDS records of the next chunk go in flight before a chunk is
+// visited; without it a chunk's four records are all that is held (for
+// records of tens of bytes).
+template <uint32_t STRIDE, uint32_t PRE, bool PIPE = true>
+struct StagedTable {
+    static constexpr uint32_t kRows = STRIDE / 2;  // chunk pairs per step
+    const uint2 *base;
+    uint2 q[PRE];
+
+    __device__ __forceinline__ void load(const DevBuffers &b, uint32_t i, uint32_t first)
+    {
+        base = nbr16_chunk(b, i, first);
+        const uint32_t room = b.kq - 1u, r0 = first >> 1;  // pairs of this share: 0 .. room
+#pragma unroll
+        for (uint32_t t = 0; t < PRE; t++)
+            q[t] = *nbr16_chunk(b, i, 2u * min(r0 + kRows * t, room) + (first & 1u));
+    }
+
+    // fn(entry, gather(entry)) for this lane's entries of the first c, in
+    // table order
+    template <typename G, typename Fn>
+    __device__ __forceinline__ void visit(uint32_t first, uint32_t c, G gather, Fn fn) const
+    {
+        const uint32_t nch = (c + 3u) >> 2;  // chunks in use
+        const uint32_t mine = nch > first ? (nch - first + STRIDE - 1u) / STRIDE : 0u;
+        constexpr uint32_t kSent = kStageSentinel | (kStageSentinel << 16);
+        auto take = [&](uint32_t t) {
+            return t < mine ? q[t] : make_uint2(kSent, kSent);
+        };
+        struct Four {
+            decltype(gather(0u)) a, b, c, d;
+        };
+        auto gather4 = [&](const uint2 &e) {
+            return Four{gather(e.x & 0xffffu), gather(e.x >> 16), gather(e.y & 0xffffu), gather(e.y >> 16)};
+        };
+        auto visit4 = [&](const uint2 &e, const Four &r) {
+            fn(e.x & 0xffffu, r.a);
+            fn(e.x >> 16, r.b);
+            fn(e.y & 0xffffu, r.c);
+            fn(e.y >> 16, r.d);
+        };
+        if constexpr (PIPE) {
+            uint2 e = take(0);
+            Four r = gather4(e);
+#pragma unroll
+            for (uint32_t t = 0; t < PRE; t++) {
+                const uint2 en = t + 1 < PRE ? take(t + 1) : e;
+                Four rn = r;
+                if (t + 1 < PRE) rn = gather4(en);
+                if (t < mine) visit4(e, r);
+                e = en;
+                r = rn;
+            }
+        } else {
+#pragma unroll
+            for (uint32_t t = 0; t < PRE; t++)
+                if (t < mine) visit4(q[t], gather4(q[t]));
+        }
+        if (mine > PRE) {
+            uint2 e = base[(size_t)PRE * kRows * 128];
+            for (uint32_t t = PRE; t < mine; t++) {
+                const uint2 en = base[(size_t)min(t + 1u, mine - 1u) * kRows * 128];
+                visit4(e, gather4(e));
+                e = en;
+            }
+        }
+    }
+};
+
+// The entries of half h of a staged particle's first c neighbours in table
+// order, one at a time: for the rarely taken recomputation of one half.
+template <typename Fn>
+__device__ __forceinline__ void for_staged_half_plain(const DevBuffers &b, uint32_t i, uint32_t c, uint32_t h,
+                                                      Fn fn)
+{
+    for (uint32_t q0 = 4u * h; q0 < c; q0 += 8u)
+        for (uint32_t q = q0; q < q0 + 4u && q < c; q++)
+            fn((uint32_t)reinterpret_cast<const uint16_t *>(nbr16_chunk(b, i, q >> 2))[q & 3u]);
+}
+
 // Visit the first c neighbours of particle i in table order, calling
 // fn(j, gather(j)) for each.  Software-pipelined: while chunk m is being
 // processed, the four gathers of chunk m+1 and the index load of chunk m+2
@@ -104,11 +208,9 @@ __device__ __forceinline__ void for_neighbors(const DevBuffers &b, uint32_t i, u
 // 1, 3, 5, ..., each in table order, and then added as half 0 + half 1.  The
 // staged kernels give each half its own lane (two lanes per particle, twice
 // the wavefronts for the same LDS); the others visit both halves in turn.
-// Visits the entries of half h of particle i's first c neighbours, pipelined
-// as for_neighbors.  GUARD = false visits the padding of the last chunk as
-// well: for tables whose padding entries refer to the far-away sentinel
-// record of a staged unit (kStageSentinel), which fails every pair test.
-template <bool GUARD = true, typename G, typename Fn>
+// Visits the entries of half h of particle i's first c neighbours (global
+// slots), pipelined as for_neighbors.
+template <typename G, typename Fn>
 __device__ __forceinline__ void for_neighbors_half(const DevBuffers &b, uint32_t i, uint32_t c, uint32_t h,
                                                    G gather, Fn fn)
 {
@@ -121,9 +223,9 @@ __device__ __forceinline__ void for_neighbors_half(const DevBuffers &b, uint32_t
                      const auto &d3) {
         const uint32_t q = (2u * m + h) << 2;  // table position of jj.x
         fn(jj.x, d0);
-        if (!GUARD || q + 1 < c) fn(jj.y, d1);
-        if (!GUARD || q + 2 < c) fn(jj.z, d2);
-        if (!GUARD || q + 3 < c) fn(jj.w, d3);
+        if (q + 1 < c) fn(jj.y, d1);
+        if (q + 2 < c) fn(jj.z, d2);
+        if (q + 3 < c) fn(jj.w, d3);
     };
     uint4 ja = chunk(0);
     uint4 jb = chunk(1);

@@ -153,7 +153,8 @@ struct DevBuffers {
     uint32_t *cell_count;  // num_cells, zero between builds
     uint32_t *cell_off;    // num_cells + 1
     uint32_t *scan_part;   // per scan tile
-    // neighbours: sliced ELL in chunks of four (see ps_kernels.hip)
+    // neighbours: sliced ELL in chunks of four (see ps_kernels.hip); 16-bit
+    // LDS indices in a staged unit (nbr16_chunk)
     uint32_t *nbr;
     uint32_t *ncnt;
     uint32_t *nbr_glob;    // recording a substep for the reverse pass with staging:

@@ -6,9 +6,11 @@
 // the lambda and delta-p kernels is a single 16-byte gather.  The neighbour
 // table is a sliced ELL in chunks of four: for each group of 64 consecutive
 // particles, entries 4m..4m+3 of every lane form one uint4, and the 64 lanes'
-// uint4s are contiguous.  A wavefront therefore reads four neighbour indices
-// per lane with one coalesced 1-KiB load and issues the four position
-// gathers back to back; the builder writes 16 bytes per lane at a time.
+// uint4s are contiguous, so a wavefront reads four neighbour indices per lane
+// with one coalesced 1-KiB load.  A unit staged in LDS holds 16-bit LDS
+// indices instead, eight to a uint4 (nbr16_chunk): the table is read nine
+// times a substep, and with 32-bit entries it was most of the traffic of the
+// kernels that read it.
 //
 // Arithmetic: built with -ffp-contract=off and IEEE division/sqrt, and every
 // expression is parenthesised as in the CPU oracle, so FP32 results are
@@ -344,7 +346,8 @@ __global__ __launch_bounds__(kMaxBlock) void reorder_k(DevBuffers b, uint32_t n,
 // reads its candidates there instead of one global load per candidate and
 // lane (the loads that bound this kernel).  Any other lane or row reads
 // global memory as without WAVE; the table is the same.
-template <bool GLOB = false, bool WAVE = false, typename Range, typename Emit>
+// S16: the table is a staged unit's, 16-bit entries (nbr16_chunk).
+template <bool GLOB = false, bool WAVE = false, bool S16 = false, typename Range, typename Emit>
 __device__ __forceinline__ uint32_t scan_stencil(const DevBuffers &b, const KConst &k, uint32_t i,
                                                  uint32_t pad, const float4 p, uint32_t kmax,
                                                  Range range, Emit emit, bool valid = true,
@@ -353,17 +356,25 @@ __device__ __forceinline__ uint32_t scan_stencil(const DevBuffers &b, const KCon
     uint4 *out = const_cast<uint4 *>(nbr_lane(b, i));
     uint4 *out2 = GLOB ? reinterpret_cast<uint4 *>(b.nbr_glob) + (size_t)(i >> 6) * b.kq * 64 + (i & 63)
                        : nullptr;
-    uint4 buf = make_uint4(pad, pad, pad, pad);
+    // S16: chunk m is out16[128 (m / 2) + m % 2], its entries in buf.x, buf.y
+    uint2 *out16 = const_cast<uint2 *>(nbr16_chunk(b, i, 0));
+    const uint32_t pad2 = pad | (pad << 16);
+    uint4 buf = S16 ? make_uint4(pad2, pad2, pad, pad) : make_uint4(pad, pad, pad, pad);
     uint4 buf2 = make_uint4(i, i, i, i);
     uint32_t cnt = 0;
     const float r2max = k.search_r2;
     // an accepted candidate: shifted into buf, which after the 4th entry of
     // a chunk holds it in order (x first); chunks past kmax are not stored
     auto accept = [&](uint32_t e, uint32_t j) {
-        buf.x = buf.y;
-        buf.y = buf.z;
-        buf.z = buf.w;
-        buf.w = e;
+        if (S16) {
+            buf.x = (buf.x >> 16) | (buf.y << 16);
+            buf.y = (buf.y >> 16) | (e << 16);
+        } else {
+            buf.x = buf.y;
+            buf.y = buf.z;
+            buf.z = buf.w;
+            buf.w = e;
+        }
         if (GLOB) {
             buf2.x = buf2.y;
             buf2.y = buf2.z;
@@ -371,7 +382,10 @@ __device__ __forceinline__ uint32_t scan_stencil(const DevBuffers &b, const KCon
             buf2.w = j;
         }
         if ((cnt & 3u) == 3u && cnt < kmax) {
-            out[(size_t)(cnt >> 2) * 64] = buf;
+            if (S16)
+                out16[(size_t)(cnt >> 3) * 128 + ((cnt >> 2) & 1u)] = make_uint2(buf.x, buf.y);
+            else
+                out[(size_t)(cnt >> 2) * 64] = buf;
             if (GLOB) out2[(size_t)(cnt >> 2) * 64] = buf2;
         }
         cnt++;
@@ -458,7 +472,16 @@ __device__ __forceinline__ uint32_t scan_stencil(const DevBuffers &b, const KCon
     const uint32_t kept = cnt < kmax ? cnt : kmax;
     // a partial last chunk: its r entries sit at the right end of buf
     const uint32_t r = kept & 3u;
-    if (r == 1u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.w, pad, pad, pad);
+    if (S16) {
+        // shift the r entries down, padding behind them
+        if (r != 0u) {
+            for (uint32_t q = r; q < 4u; q++) {
+                buf.x = (buf.x >> 16) | (buf.y << 16);
+                buf.y = (buf.y >> 16) | (pad << 16);
+            }
+            out16[(size_t)(kept >> 3) * 128 + ((kept >> 2) & 1u)] = make_uint2(buf.x, buf.y);
+        }
+    } else if (r == 1u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.w, pad, pad, pad);
     else if (r == 2u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.z, buf.w, pad, pad);
     else if (r == 3u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.y, buf.z, buf.w, pad);
     if (GLOB) {
@@ -519,33 +542,48 @@ __global__ __launch_bounds__(kMaxBlock) void neighbors_k(DevBuffers b, KConst k,
     neighbor_status(b, cnt, kmax, ldsw);
 }
 
-// Copy a staged unit's chunks of the current data into LDS.  With THREADS
-// threads, thread t handles element t % 16 of chunks c = (THREADS/16) k +
-// t / 16, BATCH chunks' loads in flight at a time; a chunk's elements past
-// its interval read a clamped slot and fill padding that no table entry
-// refers to.  load(j) reads slot j, store(l, v) writes LDS index l.  Every
-// thread of the block calls it.
-template <uint32_t BATCH, uint32_t THREADS = kStageUnit, typename Load, typename Store>
-__device__ __forceinline__ void stage_copy(const StageDesc *d, uint32_t n, Load load, Store store)
-{
+// A staged unit's chunk sources for one thread: with THREADS threads, thread
+// t handles element t % 16 of chunks c = (THREADS/16) k + t / 16.  load() is
+// called before the descriptor's header is known (an unused chunk's source
+// is whatever is there, and is not used), so that the sources, the header
+// and the particle's own records wait together.
+template <uint32_t THREADS>
+struct StageSrc {
     static_assert(THREADS % kStageChunk == 0 && kStageChunks % (THREADS / kStageChunk) == 0,
                   "whole chunks per step");
-    constexpr uint32_t kPerStep = THREADS / kStageChunk;  // chunks per step
-    constexpr uint32_t kSteps = kStageChunks / kPerStep;
-    const uint32_t nch = d->nchunks, sub = threadIdx.x % kStageChunk;
-    const uint32_t c0 = threadIdx.x / kStageChunk;
+    static constexpr uint32_t kPerStep = THREADS / kStageChunk;  // chunks per step
+    static constexpr uint32_t kSteps = kStageChunks / kPerStep;
+    uint32_t src[kSteps];
+
+    __device__ __forceinline__ void load(const StageDesc *d)
+    {
+        const uint32_t c0 = threadIdx.x / kStageChunk;
+#pragma unroll
+        for (uint32_t k = 0; k < kSteps; k++) src[k] = d->src[k * kPerStep + c0];
+    }
+};
+
+// Copy a staged unit's chunks of the current data into LDS, BATCH chunks'
+// loads in flight at a time; a chunk's elements past its interval read a
+// clamped slot and fill padding that no table entry refers to.  load(j)
+// reads slot j, store(l, v) writes LDS index l.  Every thread of the block
+// calls it.
+template <uint32_t BATCH, uint32_t THREADS, typename Load, typename Store>
+__device__ __forceinline__ void stage_copy(const StageSrc<THREADS> &ss, uint32_t nch, uint32_t n, Load load,
+                                           Store store)
+{
+    constexpr uint32_t kPerStep = StageSrc<THREADS>::kPerStep, kSteps = StageSrc<THREADS>::kSteps;
+    static_assert(kSteps % BATCH == 0, "whole batches");
+    const uint32_t sub = threadIdx.x % kStageChunk, c0 = threadIdx.x / kStageChunk;
 #pragma unroll
     for (uint32_t k0 = 0; k0 < kSteps; k0 += BATCH) {
         if (k0 * kPerStep >= nch) break;
-        uint32_t src[BATCH];
+        decltype(load(0u)) v[BATCH];
 #pragma unroll
         for (uint32_t k = 0; k < BATCH; k++) {
             const uint32_t c = (k0 + k) * kPerStep + c0;
-            src[k] = c < nch ? d->src[c] : 0u;
+            v[k] = load(c < nch ? min(ss.src[k0 + k] + sub, n - 1u) : 0u);
         }
-        decltype(load(0u)) v[BATCH];
-#pragma unroll
-        for (uint32_t k = 0; k < BATCH; k++) v[k] = load(min(src[k] + sub, n - 1u));
 #pragma unroll
         for (uint32_t k = 0; k < BATCH; k++) {
             const uint32_t c = (k0 + k) * kPerStep + c0;
@@ -711,9 +749,12 @@ __global__ __launch_bounds__(kStageUnit) void neighbors_staged_k(DevBuffers b, K
         };
         // a staged unit pads with its sentinel record, a global one with i
         const uint32_t lastv = min(63u, n - 1u - wfirst);
-        cnt = scan_stencil<GLOB, true>(b, k, i, staged ? kStageSentinel : i,
-                                       valid ? b.P[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f), kmax,
-                                       range, emit, valid, s_wrow[w], lastv);
+        const float4 p = valid ? b.P[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (staged)
+            cnt = scan_stencil<GLOB, true, true>(b, k, i, kStageSentinel, p, kmax, range, emit, valid, s_wrow[w],
+                                                 lastv);
+        else
+            cnt = scan_stencil<GLOB, true>(b, k, i, i, p, kmax, range, emit, valid, s_wrow[w], lastv);
     }
     neighbor_status(b, cnt, kmax, ldsw);
 }
@@ -747,46 +788,63 @@ __global__ __launch_bounds__(kMaxBlock) void lambda_k(DevBuffers b, KConst k, ui
     const uint32_t hh = STAGED ? (threadIdx.x & 1u) : 0u;
     const uint32_t i = STAGED ? unit * kStageUnit + (threadIdx.x >> 1) : unit * blockDim.x + threadIdx.x;
     bool staged = false;
+    // staged: the particle's own records and the first chunks of its table
+    // go in flight with the staging loads (a thread past the end reads the
+    // last particle's)
+    StagedTable<2, 4> tab;
+    Attr a;
+    float4 p;
+    uint32_t c = 0;
     if (STAGED) {
         const StageDesc *d = b.stage + unit;
+        StageSrc<2 * kStageUnit> ss;
+        const uint32_t ic = min(i, n - 1u);
+        ss.load(d);
+        tab.load(b, ic, hh);
+        a = b.A[ic];
+        p = b.P[ic];
+        c = b.ncnt[ic];
         staged = d->staged != 0u;
+        const uint32_t nch = d->nchunks;
         if (UNIFORM) {
             if (staged && threadIdx.x < 3) lds3[3 * kStageSentinel + threadIdx.x] = __builtin_inff();
             if (staged)
-                stage_copy<6, 2 * kStageUnit>(d, n, [&](uint32_t j) { return b.P[j]; },
-                                              [&](uint32_t l, const float4 &v) {
-                                                  lds3[3 * l] = v.x;
-                                                  lds3[3 * l + 1] = v.y;
-                                                  lds3[3 * l + 2] = v.z;
-                                              });
+                stage_copy<6>(ss, nch, n, [&](uint32_t j) { return b.P[j]; },
+                              [&](uint32_t l, const float4 &v) {
+                                  lds3[3 * l] = v.x;
+                                  lds3[3 * l + 1] = v.y;
+                                  lds3[3 * l + 2] = v.z;
+                              });
         } else {
             const float inf = __builtin_inff();
             if (staged && threadIdx.x == 0) lds4[kStageSentinel] = make_float4(inf, inf, inf, 0.0f);
             if (staged)
-                stage_copy<6, 2 * kStageUnit>(d, n, [&](uint32_t j) { return PM{b.P[j], b.mj[j]}; },
-                                              [&](uint32_t l, const PM &v) {
-                                                  lds4[l] = v.m < 0.0f ? make_float4(inf, inf, inf, 0.0f)
-                                                                       : make_float4(v.p.x, v.p.y, v.p.z, v.m);
-                                              });
+                stage_copy<6>(ss, nch, n, [&](uint32_t j) { return PM{b.P[j], b.mj[j]}; },
+                              [&](uint32_t l, const PM &v) {
+                                  lds4[l] = v.m < 0.0f ? make_float4(inf, inf, inf, 0.0f)
+                                                       : make_float4(v.p.x, v.p.y, v.p.z, v.m);
+                              });
         }
     }
     if (i >= n) return;
     float *Pw = reinterpret_cast<float *>(b.P);
-    const Attr a = b.A[i];
+    if (!STAGED) a = b.A[i];
     if (!UNIFORM && a.phase != PS_PHASE_FLUID) {
         Pw[4 * (size_t)i + 3] = 0.0f;
         if (TAPE) {
-            const float4 pn = b.P[i];
+            const float4 pn = STAGED ? p : b.P[i];
             b.tape_lq[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             b.tape_rho[i] = 0.0f;
             b.tape_pit[i] = make_float4(pn.x, pn.y, pn.z, 0.0f);
         }
         return;
     }
-    const float4 p = b.P[i];
+    if (!STAGED) {
+        p = b.P[i];
+        c = b.ncnt[i];
+    }
     const float r0 = a.rho0;
     const float sk = k.spiky * (1.0f / r0);
-    const uint32_t c = b.ncnt[i];
     // the sums of one half of the table
     struct Sums {
         float rho, gix, giy, giz, den;
@@ -816,8 +874,8 @@ __global__ __launch_bounds__(kMaxBlock) void lambda_k(DevBuffers b, KConst k, ui
         // Both lanes form half 0 + half 1 (addition commutes)
         Sums mine = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         if (UNIFORM && staged)
-            for_neighbors_half<false>(
-                b, i, c, hh,
+            tab.visit(
+                hh, c,
                 [&](uint32_t l) {
                     // byte offset 12 l by the full-rate 24-bit multiply (l <= kStageSentinel)
                     const float *q = reinterpret_cast<const float *>(reinterpret_cast<const char *>(lds3) +
@@ -830,8 +888,8 @@ __global__ __launch_bounds__(kMaxBlock) void lambda_k(DevBuffers b, KConst k, ui
                 b, i, c, hh, [&](uint32_t j) { return b.P[j]; },
                 [&](uint32_t, const float4 &pj) { body(mine, pj, mu); });
         else if (staged)
-            for_neighbors_half<false>(b, i, c, hh, [&](uint32_t l) { return lds4[l]; },
-                                      [&](uint32_t, const float4 &pj) { body(mine, pj, pj.w); });
+            tab.visit(hh, c, [&](uint32_t l) { return lds4[l]; },
+                      [&](uint32_t, const float4 &pj) { body(mine, pj, pj.w); });
         else
             for_neighbors_half(
                 b, i, c, hh, [&](uint32_t j) { return PM{b.P[j], b.mj[j]}; },
@@ -905,30 +963,44 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
     const uint32_t hh = STAGED ? (threadIdx.x & 1u) : 0u;
     const uint32_t i = STAGED ? unit * kStageUnit + (threadIdx.x >> 1) : unit * blockDim.x + threadIdx.x;
     bool staged = false;
+    // staged: the particle's own records and the first chunks of its table
+    // go in flight with the staging loads, as in lambda_k
+    StagedTable<2, 4> tab;
+    Attr a;
+    float4 p;
+    uint32_t c = 0;
     if (STAGED) {
         const StageDesc *d = b.stage + unit;
         // one class of units per launch (the other class's blocks leave)
         if (b.solve_units && ((d->walk != 0u) != (b.solve_units == 2u))) return;
+        StageSrc<2 * kStageUnit> ss;
+        const uint32_t ic = min(i, n - 1u);
+        ss.load(d);
+        tab.load(b, ic, hh);
+        a = b.A[ic];
+        p = b.P[ic];
+        c = b.ncnt[ic];
         staged = d->staged != 0u;
+        const uint32_t nch = d->nchunks;
         const float inf = __builtin_inff();
         if (staged && threadIdx.x == 0) lds[kStageSentinel] = make_float4(inf, inf, inf, 0.0f);
         if ((F & F_CONTACT) && staged && threadIdx.x == 0) lds_ph[kStageSentinel] = 0;
         if ((F & F_CONTACT) && staged)
-            for (uint32_t q = threadIdx.x; q < d->nchunks; q += blockDim.x) s_src[q] = d->src[q];
+            for (uint32_t q = threadIdx.x; q < nch; q += blockDim.x) s_src[q] = d->src[q];
         if (UNIFORM && staged)
-            stage_copy<6, 2 * kStageUnit>(d, n, [&](uint32_t j) { return b.P[j]; },
-                                          [&](uint32_t l, const float4 &v) { lds[l] = v; });
+            stage_copy<6>(ss, nch, n, [&](uint32_t j) { return b.P[j]; },
+                          [&](uint32_t l, const float4 &v) { lds[l] = v; });
         else if ((F & F_CONTACT) && staged && d->walk)
-            stage_copy<6, 2 * kStageUnit>(d, n, [&](uint32_t j) { return PMH{b.P[j], b.mj[j], b.phs[j]}; },
-                                          [&](uint32_t l, const PMH &v) {
-                                              lds[l] = v.m < 0.0f ? make_float4(inf, inf, inf, 0.0f) : v.p;
-                                              lds_ph[l] = v.ph;
-                                          });
+            stage_copy<6>(ss, nch, n, [&](uint32_t j) { return PMH{b.P[j], b.mj[j], b.phs[j]}; },
+                          [&](uint32_t l, const PMH &v) {
+                              lds[l] = v.m < 0.0f ? make_float4(inf, inf, inf, 0.0f) : v.p;
+                              lds_ph[l] = v.ph;
+                          });
         else if (staged)
-            stage_copy<6, 2 * kStageUnit>(d, n, [&](uint32_t j) { return PM{b.P[j], b.mj[j]}; },
-                                          [&](uint32_t l, const PM &v) {
-                                              lds[l] = v.m < 0.0f ? make_float4(inf, inf, inf, 0.0f) : v.p;
-                                          });
+            stage_copy<6>(ss, nch, n, [&](uint32_t j) { return PM{b.P[j], b.mj[j]}; },
+                          [&](uint32_t l, const PM &v) {
+                              lds[l] = v.m < 0.0f ? make_float4(inf, inf, inf, 0.0f) : v.p;
+                          });
     }
     // the storage slot of table entry e (an LDS index in a staged unit; its
     // sentinel padding, never visited, maps to i)
@@ -937,12 +1009,14 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
         return e >= kStageSlots ? i : s_src[e >> 4] + (e & (kStageChunk - 1u));
     };
     if (i >= n) return;
-    const float4 p = b.P[i];
-    const Attr a = b.A[i];
+    if (!STAGED) {
+        p = b.P[i];
+        a = b.A[i];
+        c = b.ncnt[i];
+    }
     const float px = p.x, py = p.y, pz = p.z;
     const int32_t ph = UNIFORM ? PS_PHASE_FLUID : a.phase;
     const float wi = UNIFORM ? wu : a.w;
-    const uint32_t c = b.ncnt[i];
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
     float4 tape = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // (f, contact count) when TAPE
 
@@ -979,8 +1053,8 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
                     // from the staged records: position and phase (a
                     // particle with w = 0 is staged at infinity and marked
                     // by the phase's sign bit: its position from memory)
-                    for_neighbors_half_chunked(
-                        b, i, c, hh, [&](uint32_t e) { return PH{lds[e], lds_ph[e]}; },
+                    tab.visit(
+                        hh, c, [&](uint32_t e) { return PH{lds[e], lds_ph[e]}; },
                         [&](uint32_t e, const PH &d) {
                             const int32_t phj = d.ph & 0x7fffffff;
                             if (ph > PS_PHASE_SOLID && ph == phj) return;
@@ -1097,6 +1171,8 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
                                     correct(ch1, jq[u] & 0x7fffffffu, dq[u]);
                             }
                     }
+                } else if (STAGED && staged) {
+                    for_staged_half_plain(b, i, c, hh, [&](uint32_t e) { correct(ch0, e, pa(e)); });
                 } else if (STAGED) {
                     for_neighbors_half_chunked(b, i, c, hh, pa,
                                                [&](uint32_t e, const PA &d) { correct(ch0, e, d); });
@@ -1190,8 +1266,7 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
                 // a unit that was not staged, in a scene that is not a uniform fluid
                 auto from_glob_m = [&](uint32_t j) { return PM{b.P[j], b.mj[j]}; };
                 if (staged)
-                    for_neighbors_half<false>(b, i, c, hh, from_lds,
-                                              [&](uint32_t, const float4 &pj) { fast(mine, pj); });
+                    tab.visit(hh, c, from_lds, [&](uint32_t, const float4 &pj) { fast(mine, pj); });
                 else if (UNIFORM)
                     for_neighbors_half(b, i, c, hh, from_glob,
                                        [&](uint32_t, const float4 &pj) { fast(mine, pj); });
@@ -1203,7 +1278,7 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
                     mine = {0.0f, 0.0f, 0.0f, false};
                     auto ex = [&](uint32_t, const float4 &pj) { exact(mine, pj); };
                     if (staged)
-                        for_neighbors_half_plain(b, i, c, hh, from_lds, ex);
+                        for_staged_half_plain(b, i, c, hh, [&](uint32_t e) { exact(mine, lds[e]); });
                     else if (UNIFORM)
                         for_neighbors_half_plain(b, i, c, hh, from_glob, ex);
                     else
@@ -1508,24 +1583,32 @@ __global__ __launch_bounds__(STAGED ? kFinalizeStagedBlock : kMaxBlock) void fin
     // particle of one mass (mu >= 0) the mass is mu; with fluid masses that
     // differ (MASS) each slot's mass (x*.w) is staged as well, 12 KB more
     // LDS (one block per CU instead of two).  A unit that was not staged
-    // gathers from global memory through the unit's chunk table (s_src).
+    // gathers from global memory.
     __shared__ float4 lds_pu[STAGED ? kStageSlots + 1 : 1];
     __shared__ float2 lds_u[STAGED ? kStageSlots + 1 : 1];
     __shared__ float lds_m[STAGED && MASS ? kStageSlots + 1 : 1];
-    __shared__ uint32_t s_src[STAGED && !UNIFORM ? kStageChunks : 1];
     const uint32_t unit = xcd_block();
     const uint32_t hh = threadIdx.x & 3u;
     const uint32_t i = STAGED ? unit * kStageUnit + (threadIdx.x >> 2) : (unit * blockDim.x + threadIdx.x) >> 2;
-    bool staged = false, mapped = false;
+    bool staged = false;
+    // staged: the particle's own records and the first chunks of its table
+    // go in flight with the staging loads, as in lambda_k
+    StagedTable<4, 2, false> tab;
+    float4 p, x;
+    Attr a;
+    uint32_t c = 0;
     if (STAGED) {
         const StageDesc *d = b.stage + unit;
+        StageSrc<kFinalizeStagedBlock> ss;
+        const uint32_t ic = min(i, n - 1u);
+        ss.load(d);
+        tab.load(b, ic, hh);
+        p = b.P[ic];
+        x = b.X[ic];
+        a = b.A[ic];
+        c = b.ncnt[ic];
         staged = d->staged != 0u;
-        mapped = !UNIFORM && !MASS && staged && mu < 0.0f;
-        if (mapped) {
-            for (uint32_t q = threadIdx.x; q < d->nchunks; q += blockDim.x) s_src[q] = d->src[q];
-            __syncthreads();
-        }
-        staged = staged && !mapped;
+        const uint32_t nch = d->nchunks;
         const float inf = __builtin_inff();
         if (staged && threadIdx.x == 0) {
             lds_pu[kStageSentinel] = make_float4(inf, inf, inf, 0.0f);
@@ -1533,33 +1616,33 @@ __global__ __launch_bounds__(STAGED ? kFinalizeStagedBlock : kMaxBlock) void fin
             if (MASS) lds_m[kStageSentinel] = 0.0f;
         }
         if (MASS && staged)
-            stage_copy<3, kFinalizeStagedBlock>(d, n, [&](uint32_t j) { return PX{b.P[j], b.X[j]}; },
-                                                [&](uint32_t l, const PX &v) {
-                                                    lds_pu[l] = v.x.w < 0.0f
-                                                                    ? make_float4(inf, inf, inf, 0.0f)
-                                                                    : make_float4(v.p.x, v.p.y, v.p.z, v.p.x - v.x.x);
-                                                    lds_u[l] = make_float2(v.p.y - v.x.y, v.p.z - v.x.z);
-                                                    lds_m[l] = v.x.w;
-                                                });
+            stage_copy<3>(ss, nch, n, [&](uint32_t j) { return PX{b.P[j], b.X[j]}; },
+                          [&](uint32_t l, const PX &v) {
+                              lds_pu[l] = v.x.w < 0.0f ? make_float4(inf, inf, inf, 0.0f)
+                                                       : make_float4(v.p.x, v.p.y, v.p.z, v.p.x - v.x.x);
+                              lds_u[l] = make_float2(v.p.y - v.x.y, v.p.z - v.x.z);
+                              lds_m[l] = v.x.w;
+                          });
         else if (staged)
-            stage_copy<3, kFinalizeStagedBlock>(d, n, [&](uint32_t j) { return PX{b.P[j], b.X[j]}; },
-                                                [&](uint32_t l, const PX &v) {
-                                                    lds_pu[l] = !UNIFORM && v.x.w < 0.0f
-                                                                    ? make_float4(inf, inf, inf, 0.0f)
-                                                                    : make_float4(v.p.x, v.p.y, v.p.z, v.p.x - v.x.x);
-                                                    lds_u[l] = make_float2(v.p.y - v.x.y, v.p.z - v.x.z);
-                                                });
+            stage_copy<3>(ss, nch, n, [&](uint32_t j) { return PX{b.P[j], b.X[j]}; },
+                          [&](uint32_t l, const PX &v) {
+                              lds_pu[l] = !UNIFORM && v.x.w < 0.0f ? make_float4(inf, inf, inf, 0.0f)
+                                                                   : make_float4(v.p.x, v.p.y, v.p.z, v.p.x - v.x.x);
+                              lds_u[l] = make_float2(v.p.y - v.x.y, v.p.z - v.x.z);
+                          });
     }
     // every solve of this substep has completed
     if (i == 0 && hh == 0) b.status->iter += its;
     if (i >= n) return;  // the four lanes of a particle leave together
-    const float4 p = b.P[i];
-    const float4 x = b.X[i];
+    if (!STAGED) {
+        p = b.P[i];
+        x = b.X[i];
+        a = b.A[i];
+        c = b.ncnt[i];
+    }
     const float ux = p.x - x.x, uy = p.y - x.y, uz = p.z - x.z;
     float vx = ux / dt, vy = uy / dt, vz = uz / dt;
-    const Attr a = b.A[i];
     if ((UNIFORM || a.phase == PS_PHASE_FLUID) && k.xsph_c != 0.0f) {
-        const uint32_t c = b.ncnt[i];
         // the XSPH sum of this lane's quarter of the table
         struct Sums {
             float sx, sy, sz;
@@ -1593,23 +1676,13 @@ __global__ __launch_bounds__(STAGED ? kFinalizeStagedBlock : kMaxBlock) void fin
             float m;
         };
         if (STAGED && MASS && staged)
-            for_neighbors_strided_chunked(
-                b, i, c, hh, 4u, [&](uint32_t l) { return PUM{lds_pu[l], lds_u[l], lds_m[l]}; },
+            tab.visit(
+                hh, c, [&](uint32_t l) { return PUM{lds_pu[l], lds_u[l], lds_m[l]}; },
                 [&](uint32_t, const PUM &d) { body(d.pu, d.pu.w, d.u.x, d.u.y, d.m); });
         else if (STAGED && staged)
-            for_neighbors_strided_chunked(
-                b, i, c, hh, 4u, [&](uint32_t l) { return PU{lds_pu[l], lds_u[l]}; },
+            tab.visit(
+                hh, c, [&](uint32_t l) { return PU{lds_pu[l], lds_u[l]}; },
                 [&](uint32_t, const PU &d) { body(d.pu, d.pu.w, d.u.x, d.u.y, mu); });
-        else if (STAGED && mapped)
-            // table entries are LDS indices (the sentinel padding, never
-            // visited, maps to i)
-            for_neighbors_strided_chunked(
-                b, i, c, hh, 4u,
-                [&](uint32_t e) {
-                    const uint32_t j = e >= kStageSlots ? i : s_src[e >> 4] + (e & (kStageChunk - 1u));
-                    return PX{b.P[j], b.X[j]};
-                },
-                [&](uint32_t, const PX &d) { gen(d); });
         else
             for_neighbors_strided_chunked(
                 b, i, c, hh, 4u, [&](uint32_t j) { return PX{b.P[j], b.X[j]}; },
