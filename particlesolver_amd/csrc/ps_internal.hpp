@@ -91,11 +91,12 @@ enum SolveFeature : uint32_t {
 // at most kStageRows grid rows, and the candidates of a particle in row q
 // and stencil row t = (dz+1)*3 + (dy+1) form a slot range inside interval
 // 9q + t: the slots of cells x in [xa_q - 1, xb_q + 1] of the target row.
-// The intervals are laid out in LDS back to back, each padded to a whole
-// number of kStageChunk-slot chunks; a staged unit's table holds LDS
-// indices, and src[c] is the global slot of the first element of chunk c.
+// The intervals' union, as disjoint slot segments in ascending order, is laid
+// out in LDS back to back, each segment padded to a whole number of
+// kStageChunk-slot chunks; a staged unit's table holds LDS indices, and
+// src[c] is the global slot of the first element of chunk c.
 constexpr uint32_t kStageUnit = 256;
-constexpr uint32_t kStageRows = 3;
+constexpr uint32_t kStageRows = 7;
 constexpr uint32_t kStageIv = 9 * kStageRows;
 constexpr uint32_t kStageSlots = 3072;
 // the staged neighbour build: slots of one stencil row a wavefront copies

@@ -322,76 +322,37 @@ __global__ __launch_bounds__(kMaxBlock) void reorder_k(DevBuffers b, uint32_t n,
 // of x-adjacent cells; a row's three cells are one contiguous slot range.
 
 // Scan the nine stencil rows of particle i in order (t = (dz+1)*3 + dy+1)
-// and write its table: every slot j != i of range(t) = [j0, j1) with
-// |p - P[j]|^2 < search_r2, in ascending j, stored as emit(t, j) (the slot
-// itself, or its LDS index in a staged unit); pad fills the last chunk: i's
-// own slot, or a staged unit's sentinel record.  Returns the number found
-// (the table keeps the first kmax).
+// and write its table of global slots: every slot j != i of range(t) =
+// [j0, j1) with |p - P[j]|^2 < search_r2, in ascending j; i's own slot fills
+// the last chunk.  Returns the number found (the table keeps the first kmax).
 // A row is tested in windows of 32 candidates without branches: each test
 // sets one bit of a mask (i's own bit is cleared), and the set bits are then
 // emitted lowest first, so the entries come out in ascending j as from a
 // plain loop over the row, and only accepted candidates pay for the table.
 // p is taken by value: a reference into b.P would be re-read after every
-// table store (the compiler cannot rule out aliasing).  emit(t, j) is
-// j + emit(t, 0) (an offset per stencil row), taken once per row.
-// GLOB: also write the table with global slots (entries j, padding i) to
-// b.nbr_glob in the same layout (the copy a recording for the reverse pass
-// keeps while the staged kernels read LDS indices).
-// WAVE (the staged build; every lane of the wavefront calls it, valid or
-// not): per stencil row the wavefront's lanes, consecutive sorted particles,
-// mostly share one grid row, so their ranges lie in [lo, hi), lo the range
-// start of lane 0 and hi the range end of the last valid lane (lastv).
-// When that span fits kWaveRowSlots the wavefront copies it into its own
-// LDS (wl) with coalesced loads, and a lane whose range lies inside it
-// reads its candidates there instead of one global load per candidate and
-// lane (the loads that bound this kernel).  Any other lane or row reads
-// global memory as without WAVE; the table is the same.
-// S16: the table is a staged unit's, 16-bit entries (nbr16_chunk).
-template <bool GLOB = false, bool WAVE = false, bool S16 = false, typename Range, typename Emit>
-__device__ __forceinline__ uint32_t scan_stencil(const DevBuffers &b, const KConst &k, uint32_t i,
-                                                 uint32_t pad, const float4 p, uint32_t kmax,
-                                                 Range range, Emit emit, bool valid = true,
-                                                 float *wl = nullptr, uint32_t lastv = 63u)
+// table store (the compiler cannot rule out aliasing).
+template <typename Range>
+__device__ __forceinline__ uint32_t scan_stencil(const DevBuffers &b, const KConst &k, uint32_t i, const float4 p,
+                                                 uint32_t kmax, Range range)
 {
     uint4 *out = const_cast<uint4 *>(nbr_lane(b, i));
-    uint4 *out2 = GLOB ? reinterpret_cast<uint4 *>(b.nbr_glob) + (size_t)(i >> 6) * b.kq * 64 + (i & 63)
-                       : nullptr;
-    // S16: chunk m is out16[128 (m / 2) + m % 2], its entries in buf.x, buf.y
-    uint2 *out16 = const_cast<uint2 *>(nbr16_chunk(b, i, 0));
-    const uint32_t pad2 = pad | (pad << 16);
-    uint4 buf = S16 ? make_uint4(pad2, pad2, pad, pad) : make_uint4(pad, pad, pad, pad);
-    uint4 buf2 = make_uint4(i, i, i, i);
+    uint4 buf = make_uint4(i, i, i, i);
     uint32_t cnt = 0;
     const float r2max = k.search_r2;
     // an accepted candidate: shifted into buf, which after the 4th entry of
     // a chunk holds it in order (x first); chunks past kmax are not stored
-    auto accept = [&](uint32_t e, uint32_t j) {
-        if (S16) {
-            buf.x = (buf.x >> 16) | (buf.y << 16);
-            buf.y = (buf.y >> 16) | (e << 16);
-        } else {
-            buf.x = buf.y;
-            buf.y = buf.z;
-            buf.z = buf.w;
-            buf.w = e;
-        }
-        if (GLOB) {
-            buf2.x = buf2.y;
-            buf2.y = buf2.z;
-            buf2.z = buf2.w;
-            buf2.w = j;
-        }
-        if ((cnt & 3u) == 3u && cnt < kmax) {
-            if (S16)
-                out16[(size_t)(cnt >> 3) * 128 + ((cnt >> 2) & 1u)] = make_uint2(buf.x, buf.y);
-            else
-                out[(size_t)(cnt >> 2) * 64] = buf;
-            if (GLOB) out2[(size_t)(cnt >> 2) * 64] = buf2;
-        }
+    auto accept = [&](uint32_t j) {
+        buf.x = buf.y;
+        buf.y = buf.z;
+        buf.z = buf.w;
+        buf.w = j;
+        if ((cnt & 3u) == 3u && cnt < kmax) out[(size_t)(cnt >> 2) * 64] = buf;
         cnt++;
     };
-    // the candidates [j0, j1) of one stencil row; at(j - j0) reads slot j
-    auto scan_row = [&](uint32_t j0, uint32_t j1, uint32_t eoff, auto at) {
+    for (uint32_t t = 0; t < 9; t++) {
+        uint32_t j0 = 0, j1 = 0;
+        if (!range(t, j0, j1)) continue;
+        const float4 *q0 = b.P + j0;
         for (uint32_t w0 = j0; w0 < j1; w0 += 32u) {
             const uint32_t we = min(w0 + 32u, j1);
             uint32_t m = 0;
@@ -402,7 +363,7 @@ __device__ __forceinline__ uint32_t scan_stencil(const DevBuffers &b, const KCon
                 // one address per group, immediate offsets for the four
                 float4 qv[4];
 #pragma unroll
-                for (uint32_t u = 0; u < 4; u++) qv[u] = at(jb - j0 + u);
+                for (uint32_t u = 0; u < 4; u++) qv[u] = q0[jb - j0 + u];
                 uint32_t g = 0;
 #pragma unroll
                 for (uint32_t u = 0; u < 4; u++)
@@ -413,7 +374,7 @@ __device__ __forceinline__ uint32_t scan_stencil(const DevBuffers &b, const KCon
             if (jb < we) {
                 float4 qv[3];
 #pragma unroll
-                for (uint32_t u = 0; u < 3; u++) qv[u] = at(min(jb + u, we - 1u) - j0);
+                for (uint32_t u = 0; u < 3; u++) qv[u] = q0[min(jb + u, we - 1u) - j0];
                 uint32_t g = 0;
 #pragma unroll
                 for (uint32_t u = 0; u < 3; u++)
@@ -426,70 +387,17 @@ __device__ __forceinline__ uint32_t scan_stencil(const DevBuffers &b, const KCon
             while (m != 0u) {
                 const uint32_t u = (uint32_t)__builtin_ctz(m);
                 m &= m - 1u;
-                accept(w0 + u + eoff, w0 + u);
+                accept(w0 + u);
             }
-        }
-    };
-    for (uint32_t t = 0; t < 9; t++) {
-        uint32_t j0 = 0, j1 = 0;
-        const bool ok = valid && range(t, j0, j1);
-        if constexpr (WAVE) {
-            // every lane is here: the span and the copy are the wavefront's
-            const uint32_t lo = __shfl(j0, 0, 64), hi = __shfl(j1, (int)lastv, 64);
-            const bool rowl = lo < hi && hi - lo <= kWaveRowSlots;
-            if (rowl) {
-                // the previous row's LDS reads were issued before these
-                // writes, and a wavefront's LDS operations run in order
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                for (uint32_t s = threadIdx.x & 63u; s < hi - lo; s += 64u) {
-                    const float4 v = b.P[lo + s];
-                    wl[3u * s] = v.x;
-                    wl[3u * s + 1u] = v.y;
-                    wl[3u * s + 2u] = v.z;
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            }
-            if (!ok) continue;
-            const uint32_t eoff = emit(t, 0u);
-            if (rowl && j0 >= lo && j1 <= hi) {
-                const float *w3 = wl + 3u * (j0 - lo);
-                scan_row(j0, j1, eoff, [&](uint32_t d) {
-                    return make_float4(w3[3u * d], w3[3u * d + 1u], w3[3u * d + 2u], 0.0f);
-                });
-            } else {
-                const float4 *q0 = b.P + j0;
-                scan_row(j0, j1, eoff, [&](uint32_t d) { return q0[d]; });
-            }
-        } else {
-            if (!ok) continue;
-            const float4 *q0 = b.P + j0;
-            scan_row(j0, j1, emit(t, 0u), [&](uint32_t d) { return q0[d]; });
         }
     }
     const uint32_t kept = cnt < kmax ? cnt : kmax;
     // a partial last chunk: its r entries sit at the right end of buf
     const uint32_t r = kept & 3u;
-    if (S16) {
-        // shift the r entries down, padding behind them
-        if (r != 0u) {
-            for (uint32_t q = r; q < 4u; q++) {
-                buf.x = (buf.x >> 16) | (buf.y << 16);
-                buf.y = (buf.y >> 16) | (pad << 16);
-            }
-            out16[(size_t)(kept >> 3) * 128 + ((kept >> 2) & 1u)] = make_uint2(buf.x, buf.y);
-        }
-    } else if (r == 1u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.w, pad, pad, pad);
-    else if (r == 2u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.z, buf.w, pad, pad);
-    else if (r == 3u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.y, buf.z, buf.w, pad);
-    if (GLOB) {
-        if (r == 1u) out2[(size_t)(kept >> 2) * 64] = make_uint4(buf2.w, i, i, i);
-        else if (r == 2u) out2[(size_t)(kept >> 2) * 64] = make_uint4(buf2.z, buf2.w, i, i);
-        else if (r == 3u) out2[(size_t)(kept >> 2) * 64] = make_uint4(buf2.y, buf2.z, buf2.w, i);
-    }
-    if (valid) b.ncnt[i] = kept;
+    if (r == 1u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.w, i, i, i);
+    else if (r == 2u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.z, buf.w, i, i);
+    else if (r == 3u) out[(size_t)(kept >> 2) * 64] = make_uint4(buf.y, buf.z, buf.w, i);
+    b.ncnt[i] = kept;
     return cnt;
 }
 
@@ -537,7 +445,7 @@ __global__ __launch_bounds__(kMaxBlock) void neighbors_k(DevBuffers b, KConst k,
             j1 = min(b.cell_off[row + x1 + 1], n);
             return j0 < j1;
         };
-        cnt = scan_stencil(b, k, i, i, b.P[i], kmax, range, [](uint32_t, uint32_t j) { return j; });
+        cnt = scan_stencil(b, k, i, b.P[i], kmax, range);
     }
     neighbor_status(b, cnt, kmax, ldsw);
 }
@@ -593,170 +501,574 @@ __device__ __forceinline__ void stage_copy(const StageSrc<THREADS> &ss, uint32_t
     __syncthreads();
 }
 
-// Staged build (the unit's scene grid): plan the unit's intervals and its
-// chunk table for the kernels that copy them into LDS, then scan the
-// stencil in global memory (full occupancy; this kernel reads each
-// candidate once per particle, so LDS would not save it traffic) and store
-// each neighbour as its LDS index j + base - start of its interval.  A unit
-// spanning more than kStageRows rows or kStageSlots slots keeps global slots
-// (staged = 0).
-template <bool GLOB>
-__global__ __launch_bounds__(kStageUnit) void neighbors_staged_k(DevBuffers b, KConst k, uint32_t n,
-                                                              uint32_t kmax)
+// ---------------------------------------------------------------------------
+// The staged build.  A unit's plan: its intervals (kStageRows), their union as
+// slot segments laid out in LDS, and the chunk table from which the kernels
+// that stage the unit copy it; a unit spanning more rows or slots than they
+// allow, or two scenes of a batch, keeps global slots (staged = 0).  Then the
+// search, in one of two forms.
+
+struct UnitPlan {  // in LDS
+    uint32_t wfirst[4], wlast[4], wheads[4], wwalk[4], total;
+    uint32_t rrow[kStageRows], xa[kStageRows], xb[kStageRows];
+    uint32_t st[kStageIv], en[kStageIv], delta[kStageIv];  // per interval
+    uint32_t src[kStageChunks];
+    uint8_t q[kStageUnit];  // unit row of each particle
+};
+static_assert(kStageIv <= 64, "one lane of a wavefront plans each interval");
+
+// the grid a particle's key refers to: its scene's in a batch
+struct GridOf {
+    uint32_t gx, gy, gz, base;
+};
+__device__ __forceinline__ GridOf grid_of(const DevBuffers &b, const KConst &k, uint32_t sid)
 {
-    __shared__ uint32_t s_start[kStageIv], s_base[kStageIv + 1], s_len[kStageIv];
-    __shared__ uint32_t s_row[kStageRows], s_xa[kStageRows], s_xb[kStageRows];
-    __shared__ uint32_t s_wheads[kStageUnit / 64], s_wlast[kStageUnit / 64], s_wwalk[kStageUnit / 64];
-    __shared__ uint32_t s_staged;
-    __shared__ StageDesc s_desc;
-    __shared__ uint32_t ldsw[kStageUnit / 64];
-    __shared__ float s_wrow[kStageUnit / 64][3 * kWaveRowSlots];  // each wavefront's stencil row (x, y, z)
-    const uint32_t unit = xcd_block();
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-    const uint32_t i = unit * kStageUnit + tid;
-    const bool valid = i < n;  // the valid threads are a prefix of the unit
-    // the particle's grid: in a batch its scene's (cells cbase ..), and a
-    // unit whose particles lie in two scenes keeps global slots
-    uint32_t gx = k.grid[0], gy = k.grid[1], gz = k.grid[2], cbase = 0;
-    bool one_scene = true;
     if (k.nscenes > 1u) {
-        const uint32_t first = unit * kStageUnit, lastv = min(first + kStageUnit, n) - 1u;
-        const uint32_t su = b.sid[first];
-        one_scene = b.sid[lastv] == su;
-        const SceneDev &sc = b.scenes[valid ? b.sid[i] : su];
-        gx = sc.grid[0];
-        gy = sc.grid[1];
-        gz = sc.grid[2];
-        cbase = sc.cell_base;
+        const SceneDev &sc = b.scenes[sid];
+        return GridOf{sc.grid[0], sc.grid[1], sc.grid[2], sc.cell_base};
     }
-    const uint32_t key = valid ? b.key[i] - cbase : 0u;
+    return GridOf{k.grid[0], k.grid[1], k.grid[2], 0u};
+}
+
+// inclusive scan over the wavefront
+template <typename Op>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v, Op op)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t t = __shfl_up(v, d, 64);
+        if (lane >= (uint32_t)d) v = op(v, t);
+    }
+    return v;
+}
+
+__device__ __forceinline__ uint32_t lane_u(uint32_t v, uint32_t l)
+{
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
+}
+
+struct Planned {
+    bool staged;
+    uint32_t nch, walk;
+    GridOf gr;          // of the thread's particle (tid of the unit)
+    uint32_t row, x;    // its cell: row = z gy + y
+};
+
+// kStageUnit threads, thread tid planning particle first + tid (nu of them)
+__device__ __forceinline__ Planned plan_unit(const DevBuffers &b, const KConst &k, uint32_t n, uint32_t first,
+                                             uint32_t nu, UnitPlan &L)
+{
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    const bool pv = tid < nu;
+    const uint32_t ui = first + tid;
+    const bool multi = k.nscenes > 1u;
+    uint32_t sid = 0;
+    bool one_scene = true;
+    if (multi) {
+        const uint32_t su = b.sid[first];
+        one_scene = b.sid[first + nu - 1u] == su;
+        sid = pv ? b.sid[ui] : su;
+    }
+    Planned r;
+    r.gr = grid_of(b, k, sid);
+    const GridOf gr = r.gr;
+    const uint32_t key = pv ? b.key[ui] - gr.base : 0u;
     // whether the particle walks its table for contacts (phase from cloth
     // up, w != 0: the sign bit of phs clear), loaded beside the key
-    const bool walker = valid && b.contacts && b.phs[i] >= PS_PHASE_CLOTH;
-    const uint32_t row = key / gx, x = key % gx;  // row = z gy + y
-    const uint32_t ry = row % gy, rz = row / gy;
-    const uint32_t x0 = x > 0 ? x - 1 : 0, x1 = x + 1 < gx ? x + 1 : gx - 1;
-
-    // rows of the unit: runs of equal row in the (sorted) keys
-    uint32_t prev = __shfl_up(row, 1, 64);
-    if (lane == 63) s_wlast[w] = row;
-    if (tid < kStageRows) {
-        s_xa[tid] = 0xffffffffu;
-        s_xb[tid] = 0u;
-    }
+    const bool walker = pv && b.contacts && b.phs[ui] >= PS_PHASE_CLOTH;
+    const uint32_t row = key / gr.gx, x = key % gr.gx;
+    r.row = row;
+    r.x = x;
+    if (lane == 0u) L.wfirst[w] = row;
+    if (lane == 63u) L.wlast[w] = row;
     __syncthreads();
-    if (lane == 0 && w > 0) prev = s_wlast[w - 1];
-    const bool head = valid && (tid == 0 || row != prev);
+    uint32_t prev = __shfl_up(row, 1, 64), next = __shfl_down(row, 1, 64);
+    if (lane == 0u && w > 0u) prev = L.wlast[w - 1u];
+    if (lane == 63u && w < 3u) next = L.wfirst[w + 1u];
+    const bool head = pv && (tid == 0u || row != prev);
+    const bool tail = pv && (tid + 1u == nu || row != next);
     const uint64_t hm = __ballot(head);
     const uint64_t wm = __ballot(walker);
-    if (lane == 0) {
-        s_wheads[w] = (uint32_t)__popcll(hm);
-        s_wwalk[w] = wm != 0ull ? 1u : 0u;
+    if (lane == 0u) {
+        L.wheads[w] = (uint32_t)__popcll(hm);
+        L.wwalk[w] = wm != 0ull ? 1u : 0u;
     }
     __syncthreads();
     uint32_t before = 0, nrows = 0, walk = 0;
-    for (uint32_t q = 0; q < kStageUnit / 64; q++) {
-        before += q < w ? s_wheads[q] : 0u;
-        nrows += s_wheads[q];
-        walk |= s_wwalk[q];
+#pragma unroll
+    for (uint32_t q = 0; q < 4; q++) {
+        before += q < w ? L.wheads[q] : 0u;
+        nrows += L.wheads[q];
+        walk |= L.wwalk[q];
     }
-    if (!one_scene) nrows = kStageRows + 1u;  // not staged
-    const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-    const uint32_t q = before + (uint32_t)__popcll(hm & upto) - 1u;  // this particle's row
-    if (valid && nrows <= kStageRows) {
-        if (head) s_row[q] = row;
-        atomicMin(&s_xa[q], x);
-        atomicMax(&s_xb[q], x);
-    }
-    __syncthreads();
-
-    // intervals: thread 9q + t plans target row t of unit row q
-    const uint32_t niv = nrows <= kStageRows ? 9u * nrows : 0u;
-    if (tid < niv) {
-        const uint32_t qq = tid / 9u, t = tid % 9u;
-        const uint32_t r = s_row[qq], rry = r % gy, rrz = r / gy;
-        const int z = (int)rrz + (int)(t / 3) - 1, y = (int)rry + (int)(t % 3) - 1;
-        uint32_t st = 0, len = 0;
-        if (z >= 0 && z < (int)gz && y >= 0 && y < (int)gy) {
-            const uint32_t r2 = cbase + ((uint32_t)z * gy + (uint32_t)y) * gx;
-            const uint32_t xa = s_xa[qq], xb = s_xb[qq];
-            st = b.cell_off[r2 + (xa > 0 ? xa - 1 : 0)];
-            const uint32_t en = min(b.cell_off[r2 + (xb + 1 < gx ? xb + 1 : gx - 1) + 1], n);
-            len = en > st ? en - st : 0u;
+    r.walk = walk;
+    const bool planned = one_scene && nrows <= kStageRows;
+    if (planned && pv) {
+        const uint64_t upto = lane == 63u ? ~0ull : ((2ull << lane) - 1ull);
+        const uint32_t q = before + (uint32_t)__popcll(hm & upto) - 1u;  // this particle's row
+        L.q[tid] = (uint8_t)q;
+        if (head) {
+            L.rrow[q] = row;
+            L.xa[q] = x;  // keys ascend: the row's first particle has its lowest x
         }
-        s_start[tid] = st;
-        s_len[tid] = len;
+        if (tail) L.xb[q] = x;
     }
     __syncthreads();
-    if (tid == 0) {
-        // LDS bases: intervals padded to whole chunks
-        uint32_t acc = 0;
-        for (uint32_t iv = 0; iv < niv; iv++) {
-            s_base[iv] = acc;
-            acc += (s_len[iv] + kStageChunk - 1) / kStageChunk * kStageChunk;
-        }
-        s_base[niv] = acc;
-        s_staged = (niv > 0 && acc <= kStageSlots) ? 1u : 0u;
-    }
-    __syncthreads();
-    const bool staged = s_staged != 0u;
-    const uint32_t nch = staged ? s_base[niv] / kStageChunk : 0u;
-    if (tid == 0) {
-        s_desc.staged = staged ? 1u : 0u;
-        s_desc.nchunks = nch;
-    }
-    // chunk table: chunk c lies in the interval whose padded region holds it
-    for (uint32_t c = tid; c < nch; c += kStageUnit) {
-        uint32_t iv = 0;
-        while (iv + 1 < niv && s_base[iv + 1] <= c * kStageChunk) iv++;
-        s_desc.src[c] = s_start[iv] + (c * kStageChunk - s_base[iv]);
-    }
-    __syncthreads();
-    // the descriptor the other staged kernels of this substep read
-    StageDesc *desc = b.stage + unit;
-    if (tid == 0) {
-        desc->staged = s_desc.staged;
-        desc->nchunks = nch;
-        desc->walk = walk;
-    }
-    for (uint32_t c = tid; c < nch; c += kStageUnit) desc->src[c] = s_desc.src[c];
-
-    uint32_t cnt = 0;
-    // the wavefront's first particle and its last valid lane
-    const uint32_t wfirst = unit * kStageUnit + (tid & ~63u);
-    if (wfirst < n) {
-        auto range = [&](uint32_t t, uint32_t &j0, uint32_t &j1) {
-            const int z = (int)rz + (int)(t / 3) - 1, y = (int)ry + (int)(t % 3) - 1;
-            if (z < 0 || z >= (int)gz || y < 0 || y >= (int)gy) return false;
-            const uint32_t r2 = cbase + ((uint32_t)z * gy + (uint32_t)y) * gx;
-            j0 = b.cell_off[r2 + x0];
-            j1 = min(b.cell_off[r2 + x1 + 1], n);
-            if (j0 >= j1) return false;
-            if (staged) {
-                // the row range lies inside its interval (by construction)
-                const uint32_t iv = 9u * q + t;
-                if (j0 < s_start[iv] || j1 - s_start[iv] > s_len[iv]) {
-                    atomicOr(&b.status->flags, PS_STATUS_INTERNAL);
-                    return false;
-                }
+    // The rest is the first wavefront's (the others wait): lane 9q + t takes
+    // the interval of target row t of unit row q.
+    if (w == 0u) {
+        const uint32_t niv = planned ? 9u * nrows : 0u;
+        uint32_t st = 0, en = 0;
+        if (lane < niv) {
+            const uint32_t qq = lane / 9u, t = lane % 9u;
+            const uint32_t rr = L.rrow[qq], ry = rr % gr.gy, rz = rr / gr.gy;
+            const int z = (int)rz + (int)(t / 3u) - 1, y = (int)ry + (int)(t % 3u) - 1;
+            if (z >= 0 && z < (int)gr.gz && y >= 0 && y < (int)gr.gy) {
+                const uint32_t r2 = gr.base + ((uint32_t)z * gr.gy + (uint32_t)y) * gr.gx;
+                const uint32_t xa = L.xa[qq], xb = L.xb[qq];
+                st = b.cell_off[r2 + (xa > 0u ? xa - 1u : 0u)];
+                en = min(b.cell_off[r2 + (xb + 1u < gr.gx ? xb + 1u : gr.gx - 1u) + 1u], n);
             }
-            return true;
-        };
-        // LDS index = slot + (base - start) of the stencil row's interval
-        auto emit = [&](uint32_t t, uint32_t j) {
-            const uint32_t iv = 9u * q + t;
-            return staged ? j + (s_base[iv] - s_start[iv]) : j;
-        };
-        // a staged unit pads with its sentinel record, a global one with i
-        const uint32_t lastv = min(63u, n - 1u - wfirst);
-        const float4 p = valid ? b.P[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (staged)
-            cnt = scan_stencil<GLOB, true, true>(b, k, i, kStageSentinel, p, kmax, range, emit, valid, s_wrow[w],
-                                                 lastv);
+            if (en <= st) st = en = 0xffffffffu;  // empty: behind all others
+            L.st[lane] = st;
+            L.en[lane] = en;
+        } else {
+            st = en = 0xffffffffu;
+        }
+        // in order of their start: lane l of ost, oen is the l-th interval
+        uint32_t rank = 0;
+        for (uint32_t q = 0; q < niv; q++) {
+            const uint32_t a = lane_u(st, q);
+            rank += (a < st || (a == st && q < lane)) ? 1u : 0u;
+        }
+        if (lane >= niv) rank = lane;
+        const uint32_t ost = (uint32_t)__builtin_amdgcn_ds_permute((int)(rank << 2), (int)st);
+        const uint32_t oen = (uint32_t)__builtin_amdgcn_ds_permute((int)(rank << 2), (int)en);
+        const bool have = ost != 0xffffffffu;
+        const uint32_t m = (uint32_t)__popcll(__ballot(have));  // a prefix of the lanes
+        // Their union: an interval that starts past the end of all before it
+        // starts a segment.  A segment's LDS base is the sum of the padded
+        // lengths of those before, each taken by the next one's head.
+        auto mx = [](uint32_t a, uint32_t c) { return a > c ? a : c; };
+        auto add = [](uint32_t a, uint32_t c) { return a + c; };
+        auto pad = [](uint32_t len) { return (len + kStageChunk - 1u) / kStageChunk * kStageChunk; };
+        const uint32_t emax = wave_scan(have ? oen : 0u, mx);
+        const uint32_t ebefore = __shfl_up(emax, 1, 64);  // end of all before
+        const bool shead = have && (lane == 0u || ost > ebefore);
+        const uint32_t shst = wave_scan(shead ? ost : 0u, mx);  // start of the interval's segment
+        const uint32_t sbefore = __shfl_up(shst, 1, 64);
+        const uint32_t plen = shead && lane > 0u ? pad(ebefore - sbefore) : 0u;
+        const uint32_t base = wave_scan(plen, add);
+        const uint32_t mylast = pad(emax - shst);
+        // LDS index = slot + delta, back in interval order
+        const uint32_t dl = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(rank << 2), (int)(base - shst));
+        if (lane < niv) L.delta[lane] = dl;
+        const uint32_t total = m ? lane_u(base + mylast, m - 1u) : 0xffffffffu;
+        if (lane == 0u) L.total = total;
+        if (total <= kStageSlots) {
+            // chunk table: a segment's chunks by the next one's head, the
+            // last's by the last interval
+            for (uint32_t c = 0; c < plen; c += kStageChunk) L.src[(base - plen + c) / kStageChunk] = sbefore + c;
+            if (lane == m - 1u)
+                for (uint32_t c = 0; c < mylast; c += kStageChunk) L.src[(base + c) / kStageChunk] = shst + c;
+        }
+    }
+    __syncthreads();
+    r.staged = planned && L.total <= kStageSlots;
+    r.nch = r.staged ? L.total / kStageChunk : 0u;
+    return r;
+}
+
+// the descriptor the other staged kernels of this substep read
+__device__ __forceinline__ void put_desc(StageDesc *desc, const Planned &pl, const UnitPlan &L)
+{
+    const uint32_t tid = threadIdx.x;
+    if (tid == 0u) {
+        desc->staged = pl.staged ? 1u : 0u;
+        desc->nchunks = pl.nch;
+        desc->walk = pl.walk;
+    }
+    if (tid < pl.nch) desc->src[tid] = L.src[tid];
+}
+
+// (m << 1) | (a < b): the compare's carry shifted in, false for a NaN
+__device__ __forceinline__ uint32_t push_less(uint32_t m, float a, float b)
+{
+    asm("v_cmp_lt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(a), "v"(b) : "vcc");
+    return m;
+}
+
+// The search of a chip full of units: one particle a lane, a unit a block.
+// Per stencil row the wavefront's lanes, consecutive sorted particles, mostly
+// share one grid row, so their ranges lie in [lo, hi), lo the range start of
+// lane 0 and hi the range end of the last valid lane (lastv), about 80 slots.
+// When that span fits kWaveRowSlots the wavefront copies it into its own LDS
+// (wl) with coalesced loads, and a lane whose range lies inside it reads its
+// candidates there; any other lane or row reads global memory.  A candidate
+// costs 8 VALU: the squared distance (6), its comparison and the carry that
+// shifts the result into the row's mask; the set bits are then emitted from
+// the top, in ascending slot.
+template <bool GLOB, bool S16>
+__device__ __forceinline__ uint32_t scan_unit_rows(const DevBuffers &b, const KConst &k, uint32_t n, uint32_t kmax,
+                                                   uint32_t i, bool valid, uint32_t lastv, const Planned &pl,
+                                                   const UnitPlan &L, float *wl)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const GridOf gr = pl.gr;
+    const float4 p = valid ? b.P[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float r2max = k.search_r2;
+    const uint32_t q9 = S16 ? 9u * L.q[threadIdx.x] : 0u;
+    const uint32_t ry = pl.row % gr.gy, rz = pl.row / gr.gy;
+    const uint32_t x0 = pl.x > 0u ? pl.x - 1u : 0u, x1 = pl.x + 1u < gr.gx ? pl.x + 1u : gr.gx - 1u;
+    uint4 *out = const_cast<uint4 *>(nbr_lane(b, i));
+    uint2 *out16 = const_cast<uint2 *>(nbr16_chunk(b, i, 0));
+    uint4 *out2 = GLOB ? reinterpret_cast<uint4 *>(b.nbr_glob) + (size_t)(i >> 6) * b.kq * 64 + (i & 63) : nullptr;
+    uint4 buf = make_uint4(i, i, i, i), buf2 = make_uint4(i, i, i, i);
+    uint32_t cnt = 0;
+    // an accepted candidate: shifted into buf, which after the 4th entry of
+    // a chunk holds it in order (x first); chunks past kmax are not stored
+    auto accept = [&](uint32_t e, uint32_t j) {
+        if (S16) {
+            buf.x = __builtin_amdgcn_alignbit(buf.y, buf.x, 16);
+            buf.y = __builtin_amdgcn_alignbit(e, buf.y, 16);
+        } else {
+            buf.x = buf.y;
+            buf.y = buf.z;
+            buf.z = buf.w;
+            buf.w = e;
+        }
+        if (GLOB) {
+            buf2.x = buf2.y;
+            buf2.y = buf2.z;
+            buf2.z = buf2.w;
+            buf2.w = j;
+        }
+        if ((cnt & 3u) == 3u && cnt < kmax) {
+            if (S16)
+                out16[(size_t)(cnt >> 3) * 128 + ((cnt >> 2) & 1u)] = make_uint2(buf.x, buf.y);
+            else
+                out[(size_t)(cnt >> 2) * 64] = buf;
+            if (GLOB) out2[(size_t)(cnt >> 2) * 64] = buf2;
+        }
+        cnt++;
+    };
+    // the candidates [j0, j1) of one stencil row; at(j - j0) reads slot j
+    auto scan_row = [&](uint32_t j0, uint32_t j1, uint32_t eoff, auto at) {
+        for (uint32_t w0 = j0; w0 < j1; w0 += 32u) {
+            const uint32_t we = min(w0 + 32u, j1);
+            uint32_t m = 0;
+            uint32_t jb = w0;
+            // whole groups of four: no bound test, one address, immediate
+            // offsets; the loads go ahead of the tests
+            for (; jb + 4u <= we; jb += 4u) {
+                float4 qv[4];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; u++) qv[u] = at(jb - j0 + u);
+#pragma unroll
+                for (uint32_t u = 0; u < 4; u++)
+                    m = push_less(m, dist2(p.x - qv[u].x, p.y - qv[u].y, p.z - qv[u].z), r2max);
+            }
+            // the last one to three
+            if (jb < we) {
+                float4 qv[3];
+#pragma unroll
+                for (uint32_t u = 0; u < 3; u++) qv[u] = at(min(jb + u, we - 1u) - j0);
+#pragma unroll
+                for (uint32_t u = 0; u < 3; u++)
+                    m = push_less(m, dist2(p.x - qv[u].x, p.y - qv[u].y, p.z - qv[u].z), r2max);
+                m >>= 3u - (we - jb);
+            }
+            m <<= 32u - (we - w0);  // candidate w0 + u at bit 31 - u
+            // i itself (in its own row only)
+            if (i - w0 < 32u) m &= ~(0x80000000u >> (i - w0));
+            while (m != 0u) {
+                const uint32_t u = (uint32_t)__builtin_clz(m);
+                m ^= 0x80000000u >> u;
+                accept(w0 + u + eoff, w0 + u);
+            }
+        }
+    };
+    for (uint32_t t = 0; t < 9u; t++) {
+        uint32_t j0 = 0, j1 = 0, eoff = 0;
+        const int z = (int)rz + (int)(t / 3u) - 1, y = (int)ry + (int)(t % 3u) - 1;
+        if (valid && z >= 0 && z < (int)gr.gz && y >= 0 && y < (int)gr.gy) {
+            const uint32_t r2 = gr.base + ((uint32_t)z * gr.gy + (uint32_t)y) * gr.gx;
+            j0 = b.cell_off[r2 + x0];
+            j1 = min(b.cell_off[r2 + x1 + 1u], n);
+        }
+        // every lane is here: the span and the copy are the wavefront's
+        const uint32_t lo = __shfl(j0, 0, 64), hi = __shfl(j1, (int)lastv, 64);
+        const bool rowl = lo < hi && hi - lo <= kWaveRowSlots;
+        if (rowl) {
+            // the previous row's LDS reads were issued before these writes,
+            // and a wavefront's LDS operations run in order
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            for (uint32_t s = lane; s < hi - lo; s += 64u) {
+                const float4 v = b.P[lo + s];
+                wl[3u * s] = v.x;
+                wl[3u * s + 1u] = v.y;
+                wl[3u * s + 2u] = v.z;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        if (j0 >= j1) continue;
+        if (S16) {
+            // the row range lies inside its interval (by construction)
+            const uint32_t iv = q9 + t;
+            eoff = L.delta[iv];
+            if (j0 < L.st[iv] || j1 > L.en[iv]) {
+                atomicOr(&b.status->flags, PS_STATUS_INTERNAL);
+                continue;
+            }
+        }
+        if (rowl && j0 >= lo && j1 <= hi) {
+            const float *w3 = wl + 3u * (j0 - lo);
+            scan_row(j0, j1, eoff, [&](uint32_t d) {
+                return make_float4(w3[3u * d], w3[3u * d + 1u], w3[3u * d + 2u], 0.0f);
+            });
+        } else {
+            const float4 *q0 = b.P + j0;
+            scan_row(j0, j1, eoff, [&](uint32_t d) { return q0[d]; });
+        }
+    }
+    const uint32_t kept = cnt < kmax ? cnt : kmax;
+    // a partial last chunk: its c entries sit at the right end of buf; a
+    // staged unit pads with its sentinel record, a global one with i
+    const uint32_t c = kept & 3u;
+    if (c != 0u) {
+        if (S16) {
+            for (uint32_t u = c; u < 4u; u++) {
+                buf.x = __builtin_amdgcn_alignbit(buf.y, buf.x, 16);
+                buf.y = __builtin_amdgcn_alignbit(kStageSentinel, buf.y, 16);
+            }
+            out16[(size_t)(kept >> 3) * 128 + ((kept >> 2) & 1u)] = make_uint2(buf.x, buf.y);
+        } else {
+            out[(size_t)(kept >> 2) * 64] = c == 1u   ? make_uint4(buf.w, i, i, i)
+                                            : c == 2u ? make_uint4(buf.z, buf.w, i, i)
+                                                      : make_uint4(buf.y, buf.z, buf.w, i);
+        }
+        if (GLOB)
+            out2[(size_t)(kept >> 2) * 64] = c == 1u   ? make_uint4(buf2.w, i, i, i)
+                                             : c == 2u ? make_uint4(buf2.z, buf2.w, i, i)
+                                                       : make_uint4(buf2.y, buf2.z, buf2.w, i);
+    }
+    if (valid) b.ncnt[i] = kept;
+    return cnt;
+}
+
+template <bool GLOB>
+__global__ __launch_bounds__(kStageUnit) void neighbors_staged_k(DevBuffers b, KConst k, uint32_t n, uint32_t kmax)
+{
+    __shared__ UnitPlan L;
+    __shared__ uint32_t ldsw[kStageUnit / 64];
+    __shared__ float s_wrow[kStageUnit / 64][3 * kWaveRowSlots];  // each wavefront's stencil row (x, y, z)
+    const uint32_t unit = xcd_block(), first = unit * kStageUnit, nu = min(kStageUnit, n - first);
+    const uint32_t tid = threadIdx.x, w = tid >> 6;
+    const Planned pl = plan_unit(b, k, n, first, nu, L);
+    put_desc(b.stage + unit, pl, L);
+    uint32_t cnt = 0;
+    if ((tid & ~63u) < nu) {
+        const uint32_t lastv = min(63u, nu - 1u - (tid & ~63u));
+        if (pl.staged)
+            cnt = scan_unit_rows<GLOB, true>(b, k, n, kmax, first + tid, tid < nu, lastv, pl, L, s_wrow[w]);
         else
-            cnt = scan_stencil<GLOB, true>(b, k, i, i, p, kmax, range, emit, valid, s_wrow[w], lastv);
+            cnt = scan_unit_rows<GLOB, false>(b, k, n, kmax, first + tid, tid < nu, lastv, pl, L, s_wrow[w]);
     }
     neighbor_status(b, cnt, kmax, ldsw);
+}
+
+// The search of a few units, bound by its chain of dependent loads: each
+// unit's particles go to four blocks (each plans the unit for itself), four
+// lanes a particle, lane g over the stencil rows from kRowOf(g) to
+// kRowOf(g + 1).  A lane reads its rows' ranges and the first eight
+// candidates before the plan, which only the entries need, and from then on
+// the next eight while it tests eight.  A lane's accepted entries go to its
+// list in LDS; the lists of a particle, in lane order, are its table, written
+// as whole uint4s.  A particle with a list past kLaneOut has its rows
+// searched again, with the positions known, into memory.
+// With one lane a particle the nine rows follow one another, each waiting
+// for its range and its slots.
+
+constexpr uint32_t kNbrParts = 4;                  // blocks per unit
+constexpr uint32_t kNbrOwn = kStageUnit / kNbrParts;
+constexpr uint32_t kLaneOut = 28;                  // entries of a lane's list
+constexpr uint32_t kLaneStride = kLaneOut + 1;     // odd: lanes on distinct banks
+constexpr uint32_t kNbrSplitUnits = 32;           // up to here a unit's search is split over four blocks
+
+__device__ __forceinline__ uint32_t row_of(uint32_t g) { return g == 0u ? 0u : 2u * g + 1u; }  // 0, 3, 5, 7, 9
+
+template <bool GLOB>
+__global__ __launch_bounds__(kStageUnit) void neighbors_split_k(DevBuffers b, KConst k, uint32_t n, uint32_t kmax)
+{
+    __shared__ UnitPlan L;
+    __shared__ uint32_t ldsw[kStageUnit / 64];
+    __shared__ uint32_t s_list[kStageUnit * kLaneStride];
+    const uint32_t bid = xcd_block(), unit = bid / kNbrParts, part = bid % kNbrParts;
+    const uint32_t first = unit * kStageUnit, nu = min(kStageUnit, n - first);
+    const uint32_t g = threadIdx.x & 3u, li = part * kNbrOwn + (threadIdx.x >> 2);
+    const bool valid = li < nu;
+    const uint32_t i = first + li, ic = valid ? i : first;
+    const float r2max = k.search_r2;
+    const GridOf gr = grid_of(b, k, k.nscenes > 1u ? b.sid[ic] : 0u);
+    const uint32_t key = b.key[ic] - gr.base;
+    const float4 p = b.P[ic];
+    const uint32_t x = key % gr.gx, row = key / gr.gx, ry = row % gr.gy, rz = row / gr.gy;
+    const uint32_t x0 = x > 0u ? x - 1u : 0u, x1 = x + 1u < gr.gx ? x + 1u : gr.gx - 1u;
+    // the ranges of the lane's rows (three for lane 0, two for the others)
+    const uint32_t t0 = row_of(g), nt = row_of(g + 1u) - t0;
+    uint32_t ja[3], je[3];
+#pragma unroll
+    for (uint32_t u = 0; u < 3; u++) {
+        const uint32_t t = t0 + u;
+        const int z = (int)rz + (int)(t / 3u) - 1, y = (int)ry + (int)(t % 3u) - 1;
+        ja[u] = je[u] = 0u;
+        if (valid && u < nt && z >= 0 && z < (int)gr.gz && y >= 0 && y < (int)gr.gy) {
+            const uint32_t r2 = gr.base + ((uint32_t)z * gr.gy + (uint32_t)y) * gr.gx;
+            ja[u] = b.cell_off[r2 + x0];
+            je[u] = min(b.cell_off[r2 + x1 + 1u], n);
+            if (je[u] < ja[u]) je[u] = ja[u];
+        }
+    }
+    // eight candidates from j of row u (u = 3: none left)
+    struct At {
+        uint32_t u, j, e;
+    };
+    auto from = [&](uint32_t u) {  // the first non-empty row from u on
+        At a = {3u, 0u, 0u};
+        if (u <= 2u && ja[2] < je[2]) a = At{2u, ja[2], je[2]};
+        if (u <= 1u && ja[1] < je[1]) a = At{1u, ja[1], je[1]};
+        if (u == 0u && ja[0] < je[0]) a = At{0u, ja[0], je[0]};
+        return a;
+    };
+    auto after = [&](const At &a) { return a.j + 8u < a.e ? At{a.u, a.j + 8u, a.e} : from(a.u + 1u); };
+    struct Eight {
+        float4 c[8];
+    };
+    auto fetch = [&](const At &a) {
+        Eight v;
+        if (a.u < 3u) {
+#pragma unroll
+            for (uint32_t q = 0; q < 8; q++) v.c[q] = b.P[min(a.j + q, a.e - 1u)];
+        }
+        return v;
+    };
+    At at = from(0u);
+    Eight v = fetch(at);
+    const Planned pl = plan_unit(b, k, n, first, nu, L);
+    const bool staged = pl.staged;
+    if (part == 0u) put_desc(b.stage + unit, pl, L);
+    // LDS index = slot + dl of the row
+    uint32_t dl[3] = {0u, 0u, 0u};
+    if (staged && valid) {
+#pragma unroll
+        for (uint32_t u = 0; u < 3; u++)
+            if (ja[u] < je[u]) {
+                // the range lies inside its interval (by construction)
+                const uint32_t iv = 9u * L.q[li] + t0 + u;
+                dl[u] = L.delta[iv];
+                if (ja[u] < L.st[iv] || je[u] > L.en[iv]) {
+                    atomicOr(&b.status->flags, PS_STATUS_INTERNAL);
+                    at.u = 3u;
+                }
+            }
+    }
+    // every accepted candidate of the lane in order: put(m, j, dl), m of them
+    // before; returns how many
+    auto search = [&](At a, Eight w, auto put) {
+        uint32_t m = 0;
+        while (a.u < 3u) {
+            const At na = after(a);
+            const Eight nw = fetch(na);
+            uint32_t bits = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < 8; q++)
+                bits = push_less(bits, dist2(p.x - w.c[q].x, p.y - w.c[q].y, p.z - w.c[q].z), r2max);
+            bits <<= 24;  // candidate j + q at bit 31 - q
+            if (a.e - a.j < 8u) bits &= 0xffffffffu << (32u - (a.e - a.j));
+            if (i - a.j < 8u) bits &= ~(0x80000000u >> (i - a.j));
+            const uint32_t d = a.u == 0u ? dl[0] : a.u == 1u ? dl[1] : dl[2];
+            while (bits) {
+                const uint32_t q = (uint32_t)__builtin_clz(bits);
+                bits ^= 0x80000000u >> q;
+                put(m++, a.j + q, d);
+            }
+            a = na;
+            w = nw;
+        }
+        return m;
+    };
+    uint32_t *list = s_list + threadIdx.x * kLaneStride;
+    const uint32_t own = search(at, v, [&](uint32_t m, uint32_t j, uint32_t d) {
+        if (m < kLaneOut) list[m] = j + d;
+    });
+    // the particle's lanes: entries before this one's, and in all
+    const uint32_t c1 = __shfl_xor(own, 1, 64), p2 = own + c1, p2o = __shfl_xor(p2, 2, 64);
+    const uint32_t pre = ((g & 1u) ? c1 : 0u) + (g >= 2u ? p2o : 0u);
+    const uint32_t cnt = p2 + p2o, kept = min(cnt, kmax);
+    uint32_t over = own > kLaneOut ? 1u : 0u;
+    over |= __shfl_xor(over, 1, 64);
+    over |= __shfl_xor(over, 2, 64);
+    uint16_t *g16 = reinterpret_cast<uint16_t *>(const_cast<uint2 *>(nbr16_chunk(b, ic, 0)));
+    uint32_t *g32 = reinterpret_cast<uint32_t *>(const_cast<uint4 *>(nbr_lane(b, ic)));
+    uint32_t *gl = GLOB ? b.nbr_glob + ((size_t)(ic >> 6) * b.kq * 64 + (ic & 63u)) * 4 : nullptr;
+    if (valid && over) {
+        search(from(0u), fetch(from(0u)), [&](uint32_t m, uint32_t j, uint32_t d) {
+            const uint32_t pos = pre + m;
+            if (pos >= kmax) return;
+            if (staged)
+                g16[(size_t)(pos >> 3) * 512 + (pos & 7u)] = (uint16_t)(j + d);
+            else
+                g32[(size_t)(pos >> 2) * 256 + (pos & 3u)] = j;
+            if (GLOB) gl[(size_t)(pos >> 2) * 256 + (pos & 3u)] = j;
+        });
+        // padding of the last chunk: the sentinel record, in a global table i
+        const uint32_t pos = kept + g;
+        if (pos < ((kept + 3u) & ~3u)) {
+            if (staged)
+                g16[(size_t)(pos >> 3) * 512 + (pos & 7u)] = (uint16_t)kStageSentinel;
+            else
+                g32[(size_t)(pos >> 2) * 256 + (pos & 3u)] = i;
+            if (GLOB) gl[(size_t)(pos >> 2) * 256 + (pos & 3u)] = i;
+        }
+    }
+    if (valid && g == 0u) b.ncnt[i] = kept;
+    // the lists meet in a wavefront's LDS (its operations run in order)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // where the lists of lanes 1, 2 and 3 begin
+    const uint32_t lane0 = (threadIdx.x & 63u) & ~3u;
+    const uint32_t b1 = __shfl(pre, (int)lane0 + 1, 64), b2 = __shfl(pre, (int)lane0 + 2, 64),
+                   b3 = __shfl(pre, (int)lane0 + 3, 64);
+    if (valid && !over) {
+        const uint32_t *l0 = s_list + (threadIdx.x & ~3u) * kLaneStride;
+        const uint32_t fill = staged ? kStageSentinel : i;
+        auto entry = [&](uint32_t pos) {
+            const uint32_t o = pos < b1   ? pos
+                               : pos < b2 ? kLaneStride + pos - b1
+                               : pos < b3 ? 2u * kLaneStride + pos - b2
+                                          : 3u * kLaneStride + pos - b3;
+            return pos < kept ? l0[o] : fill;
+        };
+        auto slot = [&](uint32_t e) {
+            return !staged ? e : e >= kStageSlots ? i : L.src[e / kStageChunk] + e % kStageChunk;
+        };
+        // four entries (a chunk) at a time, the lanes in turn
+        for (uint32_t c = g; c * 4u < kept; c += 4u) {
+            const uint4 e = make_uint4(entry(4u * c), entry(4u * c + 1u), entry(4u * c + 2u), entry(4u * c + 3u));
+            if (staged)
+                *const_cast<uint2 *>(nbr16_chunk(b, i, c)) = make_uint2(e.x | (e.y << 16), e.z | (e.w << 16));
+            else
+                const_cast<uint4 *>(nbr_lane(b, i))[(size_t)c * 64] = e;
+            if (GLOB)
+                reinterpret_cast<uint4 *>(gl)[(size_t)c * 64] = make_uint4(slot(e.x), slot(e.y), slot(e.z), slot(e.w));
+        }
+    }
+    neighbor_status(b, valid ? cnt : 0u, kmax, ldsw);
 }
 
 // ---------------------------------------------------------------------------
@@ -1776,12 +2088,19 @@ hipError_t launch_neighbors(hipStream_t st, const DevBuffers &b, const KConst &k
                             uint32_t kmax, uint32_t bs)
 {
     if (n == 0) return hipSuccess;
-    if (b.staging && b.nbr_glob)  // recording: the global-slot copy as well
-        PS_LAUNCH(neighbors_staged_k<true>, dim3(blocks_for(n, kStageUnit)), dim3(kStageUnit), 0,
-                           st, b, k, n, kmax);
-    else if (b.staging)
-        PS_LAUNCH(neighbors_staged_k<false>, dim3(blocks_for(n, kStageUnit)), dim3(kStageUnit), 0,
-                           st, b, k, n, kmax);
+    if (b.staging) {
+        // few units: their search split over four blocks each
+        const uint32_t units = blocks_for(n, kStageUnit);
+        const dim3 t(kStageUnit);
+        if (units <= kNbrSplitUnits && b.nbr_glob)  // recording: the global-slot copy as well
+            PS_LAUNCH(neighbors_split_k<true>, dim3(kNbrParts * units), t, 0, st, b, k, n, kmax);
+        else if (units <= kNbrSplitUnits)
+            PS_LAUNCH(neighbors_split_k<false>, dim3(kNbrParts * units), t, 0, st, b, k, n, kmax);
+        else if (b.nbr_glob)
+            PS_LAUNCH(neighbors_staged_k<true>, dim3(units), t, 0, st, b, k, n, kmax);
+        else
+            PS_LAUNCH(neighbors_staged_k<false>, dim3(units), t, 0, st, b, k, n, kmax);
+    }
     else
         PS_LAUNCH(neighbors_k, dim3(blocks_for(n, bs)), dim3(bs), 0, st, b, k, n, kmax);
     return hipGetLastError();
