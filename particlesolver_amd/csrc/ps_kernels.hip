@@ -507,6 +507,13 @@ __device__ __forceinline__ void stage_copy(const StageSrc<THREADS> &ss, uint32_t
 // that stage the unit copy it; a unit spanning more rows or slots than they
 // allow, or two scenes of a batch, keeps global slots (staged = 0).  Then the
 // search, in one of two forms.
+// The union is what a unit of several rows needs: the stencils of adjacent
+// rows share two of three target rows.  With three rows a unit and every
+// interval laid out apart, 79 % of the units of a 128-scene ensemble (2.55 M
+// particles) staged, with seven merged rows 95 %: lambda 147 -> 118 us, the
+// solve 202 -> 187, finalize 185 -> 140 a launch.  The plan is the first
+// wavefront's work (on all four it cost the build 10 us at 1,048,576
+// particles).
 
 struct UnitPlan {  // in LDS
     uint32_t wfirst[4], wlast[4], wheads[4], wwalk[4], total;
@@ -707,8 +714,12 @@ __device__ __forceinline__ uint32_t push_less(uint32_t m, float a, float b)
 // (wl) with coalesced loads, and a lane whose range lies inside it reads its
 // candidates there; any other lane or row reads global memory.  A candidate
 // costs 8 VALU: the squared distance (6), its comparison and the carry that
-// shifts the result into the row's mask; the set bits are then emitted from
-// the top, in ascending slot.
+// shifts the result into the row's mask (10 with the result as a number ored
+// in); the set bits are then emitted from the top, in ascending slot.  Bound
+// by VALU issue at 1,048,576 particles: 111.6 -> 108.6 us.  Reading the rows'
+// ranges and first slots ahead took it from 60 to 76 VGPRs (64 with spills)
+// and was slower: 117 (131) us, and at 131,072 particles, two wavefronts a
+// SIMD, 49 against 44 us.
 template <bool GLOB, bool S16>
 __device__ __forceinline__ uint32_t scan_unit_rows(const DevBuffers &b, const KConst &k, uint32_t n, uint32_t kmax,
                                                    uint32_t i, bool valid, uint32_t lastv, const Planned &pl,
@@ -891,13 +902,16 @@ __global__ __launch_bounds__(kStageUnit) void neighbors_staged_k(DevBuffers b, K
 // as whole uint4s.  A particle with a list past kLaneOut has its rows
 // searched again, with the positions known, into memory.
 // With one lane a particle the nine rows follow one another, each waiting
-// for its range and its slots.
+// for its range and its slots: 20.8 us at 2,048 particles (8 units), now 14.1;
+// 26.3 -> 17.7 at 7,096 of a mixed scene (28 units).  Every lane's loads are
+// its own, so the line lies where the chip begins to fill: at 17,391
+// particles (68 units) 31.5 us against 33.7, at 131,072 (512) 111 against 44.
 
 constexpr uint32_t kNbrParts = 4;                  // blocks per unit
 constexpr uint32_t kNbrOwn = kStageUnit / kNbrParts;
 constexpr uint32_t kLaneOut = 28;                  // entries of a lane's list
 constexpr uint32_t kLaneStride = kLaneOut + 1;     // odd: lanes on distinct banks
-constexpr uint32_t kNbrSplitUnits = 32;           // up to here a unit's search is split over four blocks
+constexpr uint32_t kNbrSplitUnits = 32;            // up to here a unit's search is split over four blocks
 
 __device__ __forceinline__ uint32_t row_of(uint32_t g) { return g == 0u ? 0u : 2u * g + 1u; }  // 0, 3, 5, 7, 9
 
