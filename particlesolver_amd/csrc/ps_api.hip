@@ -69,8 +69,19 @@ struct ps_system {
     uint32_t last_scene = 0;
     // captured substep graph (ps_step_graph)
     hipGraphExec_t gexec = nullptr;
+    DevBuffers g_before;
     float g_dt = 0.0f;
     uint32_t g_sub = 0;
+    // graphs of ps_step (step_replayed): one for each buffer arrangement the
+    // handle rotates through, all of sg_sub substeps of sg_dt; sg_calls
+    // counts such calls in a row
+    struct StepGraph {
+        hipGraphExec_t exec;
+        DevBuffers before, after;
+    };
+    std::vector<StepGraph> sgraphs;
+    float sg_dt = 0.0f;
+    uint32_t sg_sub = 0, sg_calls = 0;
     // substep state
     uint32_t it_sub = 0;    // iterations done in the open substep
     int stage = 0;          // 1 between predict and end
@@ -410,6 +421,9 @@ void drop_graph(ps_system *s)
 {
     if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
     s->gexec = nullptr;
+    for (ps_system::StepGraph &g : s->sgraphs) (void)hipGraphExecDestroy(g.exec);
+    s->sgraphs.clear();
+    s->sg_calls = 0;
 }
 
 // ---- timing -------------------------------------------------------------
@@ -1727,15 +1741,10 @@ int ps_substep_end(ps_system *s)
     return any_end(s);
 }
 
-int ps_step(ps_system *s, float dt, uint32_t substeps)
+namespace {
+
+int substeps_of(ps_system *s, float dt, uint32_t substeps)
 {
-    if (int rc = check_sys(s)) return rc;
-    if (s->stage) return fail(s, PS_ERR_STATE, "ps_step inside an open substep");
-    if (!(dt > 0.0f) || !is_finite(dt)) return fail(s, PS_ERR_INVALID_ARGUMENT, "dt must be > 0");
-    if (s->n == 0) return PS_OK;
-    // emitters overflowing within the call fail it before the first substep
-    if (!s->emitters.empty() || !s->femitters.empty())
-        if (int rc = emission_check(s, dt, substeps)) return rc;
     for (uint32_t k = 0; k < substeps; k++) {
         int rc;
         if ((rc = ps_substep_begin(s, dt))) return rc;
@@ -1746,6 +1755,118 @@ int ps_step(ps_system *s, float dt, uint32_t substeps)
     return PS_OK;
 }
 
+// Capture `substeps` substeps into *exec without running them; *after gets
+// the buffers as they leave them, and the handle's state is as before.
+int capture_substeps(ps_system *s, float dt, uint32_t substeps, hipGraphExec_t *exec, DevBuffers *after)
+{
+    *exec = nullptr;
+    const DevBuffers start = s->b;
+    const uint64_t sub0 = s->substeps, it0 = s->iters;
+    const bool hashed = s->hashed, valid = s->nbr_valid, bnd = s->cr_bnd_done;
+    const float dt0 = s->dt;
+    const uint32_t timing = s->timing;
+    s->timing = 0;  // no event records inside the graph
+    HIP_TRY(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
+    const int rc = substeps_of(s, dt, substeps);
+    hipGraph_t g = nullptr;
+    hipError_t e = hipStreamEndCapture(s->stream, &g);
+    s->timing = timing;
+    s->substeps = sub0;
+    s->iters = it0;
+    s->stage = 0;
+    s->it_sub = 0;
+    s->cr_swapped = false;
+    s->hashed = hashed;
+    s->nbr_valid = valid;
+    s->cr_bnd_done = bnd;
+    s->dt = dt0;
+    *after = s->b;
+    s->b = start;
+    if (rc == PS_OK && e == hipSuccess) e = hipGraphInstantiate(exec, g, nullptr, nullptr, 0);
+    if (g) (void)hipGraphDestroy(g);
+    if (rc != PS_OK) return rc;
+    if (e != hipSuccess) {
+        *exec = nullptr;
+        return fail(s, PS_ERR_DEVICE, std::string("graph capture: ") + hipGetErrorString(e));
+    }
+    return PS_OK;
+}
+
+// the same buffers in the same places; the staging mode is whatever the
+// last neighbour build chose
+bool same_buffers(DevBuffers a, DevBuffers c)
+{
+    a.staging = c.staging = 0;
+    return memcmp(&a, &c, sizeof(DevBuffers)) == 0;
+}
+
+// A small scene's substeps replayed from graphs.  The launches of a substep
+// of 2,048 particles (15, at 2.3 us each) take the host longer than the GPU
+// needs for them once several handles step at a time: with three handles in
+// turn a substep and two exports took 64 us, replayed 34 (7,096 particles of
+// a mixed scene 81 -> 56, 17,391 of fluid 107 -> 72 for two substeps).  A
+// handle that makes the same call kGraphAfter times in
+// a row captures the next ones, one graph for each arrangement its buffers
+// rotate through (a graph bakes in the pointers it was captured with), which
+// a capture repeats at most kGraphMost times; a call of another dt or
+// length, or any change to the scene (drop_graph), starts over.  Scenes past
+// kGraphParticles keep the GPU busy longer than their launches take (131,072
+// particles: 90 us a substep for 35 us of launches).
+constexpr uint32_t kGraphParticles = 65536, kGraphSubsteps = 8, kGraphAfter = 16, kGraphMost = 12;
+
+// 1: the call's substeps were enqueued; 0: not replayed; < 0: an error
+int step_replayed(ps_system *s, float dt, uint32_t substeps)
+{
+    if (s->n > kGraphParticles || substeps == 0 || substeps > kGraphSubsteps || s->timing ||
+        !s->emitters.empty() || !s->femitters.empty())
+        return 0;
+    if (s->sg_dt != dt || s->sg_sub != substeps) {
+        for (ps_system::StepGraph &g : s->sgraphs) (void)hipGraphExecDestroy(g.exec);
+        s->sgraphs.clear();
+        s->sg_dt = dt;
+        s->sg_sub = substeps;
+        s->sg_calls = 0;
+    }
+    if (s->sg_calls < kGraphAfter) {
+        s->sg_calls++;
+        return 0;
+    }
+    ps_system::StepGraph *use = nullptr;
+    for (ps_system::StepGraph &g : s->sgraphs)
+        if (same_buffers(g.before, s->b)) use = &g;
+    if (!use) {
+        if (s->sgraphs.size() >= kGraphMost) return 0;
+        ps_system::StepGraph g{};
+        g.before = s->b;
+        if (int rc = capture_substeps(s, dt, substeps, &g.exec, &g.after)) return rc;
+        s->sgraphs.push_back(g);
+        use = &s->sgraphs.back();
+    }
+    HIP_TRY(s, hipGraphLaunch(use->exec, s->stream));
+    s->b = use->after;
+    s->dt = dt;
+    s->substeps += substeps;
+    s->iters += (uint64_t)substeps * s->prm.iterations;
+    s->hashed = false;
+    s->nbr_valid = !s->cpuref;
+    return 1;
+}
+
+}  // namespace
+
+int ps_step(ps_system *s, float dt, uint32_t substeps)
+{
+    if (int rc = check_sys(s)) return rc;
+    if (s->stage) return fail(s, PS_ERR_STATE, "ps_step inside an open substep");
+    if (!(dt > 0.0f) || !is_finite(dt)) return fail(s, PS_ERR_INVALID_ARGUMENT, "dt must be > 0");
+    if (s->n == 0) return PS_OK;
+    // emitters overflowing within the call fail it before the first substep
+    if (!s->emitters.empty() || !s->femitters.empty())
+        if (int rc = emission_check(s, dt, substeps)) return rc;
+    const int rc = step_replayed(s, dt, substeps);
+    return rc ? (rc < 0 ? rc : (int)PS_OK) : substeps_of(s, dt, substeps);
+}
+
 int ps_step_graph(ps_system *s, float dt, uint32_t substeps)
 {
     if (int rc = check_sys(s)) return rc;
@@ -1754,50 +1875,19 @@ int ps_step_graph(ps_system *s, float dt, uint32_t substeps)
     if (s->n == 0 || substeps == 0) return PS_OK;
     if (!s->emitters.empty() || !s->femitters.empty())
         return fail(s, PS_ERR_UNSUPPORTED, "ps_step_graph with emitters (the particle count grows)");
-    if (!s->gexec || s->g_dt != dt || s->g_sub != substeps) {
+    if (!s->gexec || s->g_dt != dt || s->g_sub != substeps || !same_buffers(s->g_before, s->b)) {
         drop_graph(s);
-        const DevBuffers start = s->b;
-        const uint64_t sub0 = s->substeps, it0 = s->iters;
-        const uint32_t timing = s->timing;
-        s->timing = 0;  // no event records inside the graph
-        HIP_TRY(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-        int rc = PS_OK;
-        for (uint32_t k = 0; k < substeps && rc == PS_OK; k++) {
-            rc = ps_substep_begin(s, dt);
-            for (uint32_t it = 0; it < s->prm.iterations && rc == PS_OK; it++) rc = any_iterate(s);
-            if (rc == PS_OK) rc = any_end(s);
-        }
-        hipGraph_t g = nullptr;
-        hipError_t e = hipStreamEndCapture(s->stream, &g);
-        s->timing = timing;
-        s->substeps = sub0;
-        s->iters = it0;
-        s->stage = 0;
-        s->it_sub = 0;
-        s->cr_swapped = false;
-        // the buffer pointers must come back to where the capture began; the
-        // staging mode is whatever the captured neighbour builds chose
-        DevBuffers end = s->b, begin = start;
-        end.staging = begin.staging = 0;
-        const bool rotated_back = memcmp(&begin, &end, sizeof(DevBuffers)) == 0;
-        const uint32_t staging = s->b.staging;
-        s->b = start;
-        s->b.staging = staging;
-        if (rc != PS_OK || e != hipSuccess || !rotated_back) {
-            if (g) (void)hipGraphDestroy(g);
-            if (rc != PS_OK) return rc;
-            if (e != hipSuccess)
-                return fail(s, PS_ERR_DEVICE, std::string("graph capture: ") + hipGetErrorString(e));
+        DevBuffers after;
+        s->g_before = s->b;
+        if (int rc = capture_substeps(s, dt, substeps, &s->gexec, &after)) return rc;
+        // the buffer pointers must come back to where the capture began
+        if (!same_buffers(s->g_before, after)) {
+            drop_graph(s);
             return fail(s, PS_ERR_INVALID_ARGUMENT,
                         "substeps must be a multiple of the buffer rotation period "
                         "(4 for an even iteration count, 6 for odd)");
         }
-        e = hipGraphInstantiate(&s->gexec, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (e != hipSuccess) {
-            s->gexec = nullptr;
-            return fail(s, PS_ERR_DEVICE, std::string("graph instantiate: ") + hipGetErrorString(e));
-        }
+        s->b.staging = after.staging;
         s->g_dt = dt;
         s->g_sub = substeps;
     }
