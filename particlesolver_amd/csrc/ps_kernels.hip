@@ -510,7 +510,7 @@ __device__ __forceinline__ void stage_copy(const StageSrc<THREADS> &ss, uint32_t
 // The union is what a unit of several rows needs: the stencils of adjacent
 // rows share two of three target rows.  With three rows a unit and every
 // interval laid out apart, 79 % of the units of a 128-scene ensemble (2.55 M
-// particles) staged, with seven merged rows 95 %: lambda 147 -> 118 us, the
+// particles) staged, with seven merged rows 94 %: lambda 147 -> 118 us, the
 // solve 202 -> 187, finalize 185 -> 140 a launch.  The plan is the first
 // wavefront's work (on all four it cost the build 10 us at 1,048,576
 // particles).
