@@ -52,7 +52,11 @@ struct ps_system {
     bool any_fluid = false;
     float wf = 1.0f;
     bool any_contact_phase = false;
-    uint64_t n_walk = 0;  // particles that walk their table for contacts (phase >= cloth, w != 0)
+    std::vector<float> inv_mass;  // per insertion index
+    std::vector<uint8_t> mark;    // host copy of DevBuffers::omark
+    // the particles that links move (w != 0), ranked as they got their first
+    // link, and per insertion index the rank
+    std::vector<uint32_t> linked, link_rank;
     bool any_solid_phase = false;  // SOLID or RIGID particles present
     // host copies of the constraint sets (insertion indices)
     std::vector<uint32_t> dist_pairs;
@@ -413,6 +417,9 @@ void free_all(ps_system *s)
     dev_free(b.force); dev_free(b.tmass); dev_free(b.ttimer); dev_free(b.cnum); dev_free(b.clist);
     dev_free(b.sflag);
     dev_free(b.stage);
+    dev_free(b.omark); dev_free(b.smark); dev_free(b.walk_rank); dev_free(b.link_rank);
+    dev_free(b.walk_slot); dev_free(b.link_slot);
+    dev_free(b.link_off); dev_free(b.links); dev_free(b.link_own); dev_free(b.con_c); dev_free(b.con_d);
     for (ps_system::Emitter &e : s->emitters) dev_free(e.mark);
     adj_free(s);
 }
@@ -569,8 +576,6 @@ int stage_iterate(ps_system *s)
     const bool uni = uniform_fluid(s);
     LAUNCH(s, PS_K_LAMBDA,
            ps::launch_lambda(s->stream, s->b, s->kc, s->n, uni, s->wu, s->block[PS_K_LAMBDA]));
-    const uint32_t nbody = (uint32_t)s->body_off.size() - 1;
-    if (nbody) LAUNCH(s, PS_K_SHAPE, ps::launch_shape(s->stream, s->b, nbody));
     LAUNCH(s, PS_K_SOLVE,
            ps::launch_solve(s->stream, s->b, s->kc, s->n, features(s), uni, s->wu, s->it_sub,
                             s->block[PS_K_SOLVE]));
@@ -793,8 +798,51 @@ int check_sys(ps_system *s)
     return PS_OK;
 }
 
-// Upload the whole constraint incidence structure (insertion indices).
-int upload_constraints(ps_system *s)
+// Room for the constraint blocks' lists and results, made when the first
+// particle that needs them is added.
+int con_reserve(ps_system *s)
+{
+    DevBuffers &b = s->b;
+    int rc;
+    for (uint32_t **p : {&b.walk_rank, &b.link_rank, &b.walk_slot, &b.link_slot})
+        if (!*p && (rc = dev_alloc(s, p, s->cap))) return rc;
+    if (!b.link_off && (rc = dev_alloc(s, &b.link_off, (size_t)s->cap + 1))) return rc;
+    if (!b.link_own && (rc = dev_alloc(s, &b.link_own, s->cap))) return rc;
+    if (!b.con_c && (rc = dev_alloc(s, &b.con_c, s->cap))) return rc;
+    if (!b.con_d && (rc = dev_alloc(s, &b.con_d, s->cap))) return rc;
+    return PS_OK;
+}
+
+// A range of insertion indices, and the upload of a per-particle array there.
+struct Touched {
+    uint32_t lo = ~0u, hi = 0;
+    void add(uint32_t o)
+    {
+        lo = std::min(lo, o);
+        hi = std::max(hi, o + 1);
+    }
+    template <typename T>
+    hipError_t upload(T *dst, const std::vector<T> &src) const
+    {
+        if (lo >= hi) return hipSuccess;
+        return hipMemcpy(dst + lo, src.data() + lo, sizeof(T) * (hi - lo), hipMemcpyHostToDevice);
+    }
+};
+
+// each linked particle's inverse mass and number of constraints
+int upload_link_own(ps_system *s)
+{
+    std::vector<float2> own;
+    own.reserve(s->linked.size());
+    for (uint32_t o : s->linked) own.push_back(make_float2(s->inv_mass[o], (float)s->occ[o]));
+    if (!own.empty())
+        HIP_TRY(s, hipMemcpy(s->b.link_own, own.data(), sizeof(float2) * own.size(), hipMemcpyHostToDevice));
+    return PS_OK;
+}
+
+// Upload the constraint incidence structure (insertion indices); constraints
+// from c0 on are new.
+int upload_constraints(ps_system *s, size_t c0)
 {
     DevBuffers &b = s->b;
     const size_t m = s->dist_rest.size();
@@ -803,11 +851,13 @@ int upload_constraints(ps_system *s)
         dev_free(b.dist_adj);
         dev_free(b.dist_pairs);
         dev_free(b.dist_rs);
-        s->dist_cap = 0;
+        dev_free(b.links);
+        s->dist_cap = b.nlink = 0;
         int rc;
         if ((rc = dev_alloc(s, &b.dist_adj, 2 * nc))) return rc;
         if ((rc = dev_alloc(s, &b.dist_pairs, nc))) return rc;
         if ((rc = dev_alloc(s, &b.dist_rs, nc))) return rc;
+        if ((rc = dev_alloc(s, &b.links, 2 * nc))) return rc;
         s->dist_cap = nc;
     }
     std::vector<uint32_t> off(s->cap + 1, 0), adj(2 * m), fill(s->cap, 0);
@@ -826,18 +876,50 @@ int upload_constraints(ps_system *s)
         rs[2 * c] = s->dist_rest[c];
         rs[2 * c + 1] = s->dist_stiff[c];
     }
+    // the constraint blocks' copy: each linked particle's links in constraint order
+    Touched touched;
+    for (size_t e = 2 * c0; e < 2 * m; e++) {
+        const uint32_t o = s->dist_pairs[e];
+        touched.add(o);
+        if (s->inv_mass[o] == 0.0f || (s->mark[o] & ps::kMarkDist)) continue;
+        s->mark[o] |= ps::kMarkDist;
+        s->link_rank[o] = (uint32_t)s->linked.size();
+        s->linked.push_back(o);
+    }
+    std::vector<uint32_t> link_off(1, 0);
+    std::vector<float4> links;
+    links.reserve(2 * m);
+    for (uint32_t o : s->linked) {
+        for (uint32_t q = off[o]; q < off[o + 1]; q++) {
+            const uint32_t c = adj[q], first = s->dist_pairs[2 * c];
+            const uint32_t other = first == o ? s->dist_pairs[2 * c + 1] : first;
+            float bits;
+            memcpy(&bits, &other, sizeof(bits));
+            links.push_back(make_float4(bits, s->dist_rest[c], s->dist_stiff[c], s->inv_mass[other]));
+        }
+        link_off.push_back((uint32_t)links.size());
+    }
     HIP_TRY(s, hipMemcpy(b.dist_off, off.data(), sizeof(uint32_t) * off.size(), hipMemcpyHostToDevice));
+    HIP_TRY(s, touched.upload(b.occ, s->occ));
+    HIP_TRY(s, touched.upload(b.omark, s->mark));
+    HIP_TRY(s, touched.upload(b.link_rank, s->link_rank));
+    if (int rc = upload_link_own(s)) return rc;
+    if (!s->linked.empty()) {
+        HIP_TRY(s, hipMemcpy(b.link_off, link_off.data(), sizeof(uint32_t) * link_off.size(), hipMemcpyHostToDevice));
+        HIP_TRY(s, hipMemcpy(b.links, links.data(), sizeof(float4) * links.size(), hipMemcpyHostToDevice));
+    }
+    b.nlink = (uint32_t)s->linked.size();
     if (m) {
         HIP_TRY(s, hipMemcpy(b.dist_adj, adj.data(), sizeof(uint32_t) * adj.size(), hipMemcpyHostToDevice));
         HIP_TRY(s, hipMemcpy(b.dist_pairs, s->dist_pairs.data(), sizeof(uint32_t) * 2 * m,
                              hipMemcpyHostToDevice));
         HIP_TRY(s, hipMemcpy(b.dist_rs, rs.data(), sizeof(float) * 2 * m, hipMemcpyHostToDevice));
     }
-    HIP_TRY(s, hipMemcpy(b.occ, s->occ.data(), sizeof(uint32_t) * s->cap, hipMemcpyHostToDevice));
     return PS_OK;
 }
 
-int upload_pins(ps_system *s)
+// t: the particles pinned or set free since the last upload
+int upload_pins(ps_system *s, const Touched &t)
 {
     DevBuffers &b = s->b;
     const size_t np = s->pin_xyz.size() / 3;
@@ -857,9 +939,10 @@ int upload_pins(ps_system *s)
     }
     if (np)
         HIP_TRY(s, hipMemcpy(b.pin_xyz, p4.data(), sizeof(float) * 4 * np, hipMemcpyHostToDevice));
-    HIP_TRY(s, hipMemcpy(b.pin_of, s->pin_of.data(), sizeof(uint32_t) * s->cap, hipMemcpyHostToDevice));
-    HIP_TRY(s, hipMemcpy(b.occ, s->occ.data(), sizeof(uint32_t) * s->cap, hipMemcpyHostToDevice));
-    return PS_OK;
+    HIP_TRY(s, t.upload(b.pin_of, s->pin_of));
+    HIP_TRY(s, t.upload(b.occ, s->occ));
+    HIP_TRY(s, t.upload(b.omark, s->mark));
+    return upload_link_own(s);
 }
 
 // Start keeping slot_of (insertion index -> storage slot) current: rebuilt
@@ -1031,6 +1114,9 @@ static int create_impl(const ps_params *params, uint32_t nscenes, const ps_scene
     s->tiles = ps::scan_tiles(s->ncell);
     s->occ.assign(s->cap, 0);
     s->pin_of.assign(s->cap, 0);
+    s->inv_mass.assign(s->cap, 0.0f);
+    s->mark.assign(s->cap, 0);
+    s->link_rank.assign(s->cap, 0);
     s->body_of.assign(s->cap, 0);
     s->member_of.assign(s->cap, 0);
     const size_t c = s->cap;
@@ -1055,6 +1141,7 @@ static int create_impl(const ps_params *params, uint32_t nscenes, const ps_scene
     ALLOC(b.dist_off, c + 1); ALLOC(b.occ, c); ALLOC(b.pin_of, c);
     ALLOC(b.body_of, c); ALLOC(b.member_of, c); ALLOC(b.status, 1);
     ALLOC(b.stage, (c + ps::kStageUnit - 1) / ps::kStageUnit);
+    ALLOC(b.omark, c); ALLOC(b.smark, c);
     ALLOC(b.scenes, nscenes);
     if (nscenes > 1) {
         ALLOC(b.sid, c);
@@ -1078,6 +1165,7 @@ static int create_impl(const ps_params *params, uint32_t nscenes, const ps_scene
     if (e == hipSuccess) e = hipMemset(b.dist_off, 0, sizeof(uint32_t) * (c + 1));
     if (e == hipSuccess) e = hipMemset(b.occ, 0, sizeof(uint32_t) * c);
     if (e == hipSuccess) e = hipMemset(b.pin_of, 0, sizeof(uint32_t) * c);
+    if (e == hipSuccess) e = hipMemset(b.omark, 0, c);
     if (e == hipSuccess) e = hipMemset(b.body_of, 0, sizeof(uint32_t) * c);
     if (e == hipSuccess) e = hipMemset(b.member_of, 0, sizeof(uint32_t) * c);
     if (e == hipSuccess) e = hipMemset(b.status, 0, sizeof(ps::DevStatus));
@@ -1364,7 +1452,8 @@ static int add_particles_impl(ps_system *s, uint32_t scene, uint32_t n, const fl
     bool uni = s->uniform;
     float wu = s->n ? s->wu : inv_mass[0];
     bool contact = s->any_contact_phase, solid = s->any_solid_phase;
-    uint64_t nwalk = s->n_walk;
+    std::vector<uint32_t> walk(n, 0);  // rank among the contact walkers
+    uint32_t nwalk = s->b.nwalk;
     bool fmu = s->fluid_mass_uniform, anyf = s->any_fluid;
     float wf = s->wf;
     for (uint32_t k = 0; k < n; k++) {
@@ -1395,12 +1484,17 @@ static int add_particles_impl(ps_system *s, uint32_t scene, uint32_t n, const fl
             anyf = true;
         }
         if (phase[k] >= PS_PHASE_CLOTH) contact = true;
-        if (phase[k] >= PS_PHASE_CLOTH && inv_mass[k] != 0.0f) nwalk++;
+        const bool walker = phase[k] >= PS_PHASE_CLOTH && inv_mass[k] != 0.0f;
+        if (walker) walk[k] = nwalk++;
         if (phase[k] >= PS_PHASE_SOLID) solid = true;
     }
     const size_t o = s->n;
     DevBuffers &b = s->b;
+    if (s->cpuref) nwalk = 0;
+    if (nwalk)
+        if (int rc = con_reserve(s)) return rc;
     HIP_TRY(s, hipStreamSynchronize(s->stream));
+    if (nwalk) HIP_TRY(s, hipMemcpy(b.walk_rank + o, walk.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
     HIP_TRY(s, hipMemcpy(b.X + o, X.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
     // the iterate starts equal to the positions (lambda 0)
     HIP_TRY(s, hipMemcpy(b.P + o, X.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
@@ -1432,17 +1526,8 @@ static int add_particles_impl(ps_system *s, uint32_t scene, uint32_t n, const fl
     s->any_fluid = anyf;
     s->wf = wf;
     s->any_contact_phase = contact;
-    s->b.contacts = contact ? 1u : 0u;
-    // the solve runs units without contact-walking particles through the
-    // variant without contacts when such particles are rare (at most 1 in
-    // 32: ropes in fluid); with more of them (cloth, rigid bodies) most
-    // units hold one and a second launch over the others would not pay.
-    // Only the launch plan depends on this count: the neighbour build
-    // classifies the units each substep from the particles' phases and
-    // masses as they are then, so a count made stale by a later change of
-    // w or phase costs time, never a different result.
-    s->n_walk = nwalk;
-    s->b.split_solve = (contact && nwalk * 32u <= (uint64_t)s->n) ? 1u : 0u;
+    std::copy(inv_mass, inv_mass + n, s->inv_mass.begin() + o);
+    b.nwalk = nwalk;
     s->any_solid_phase = solid;
     s->nbr_valid = false;
     return PS_OK;
@@ -1467,6 +1552,7 @@ int ps_add_distance_constraints(ps_system *s, uint32_t m, const uint32_t *pairs,
     HIP_TRY(s, hipStreamSynchronize(s->stream));
     drop_graph(s);
     if (int rc = enable_slot_tracking(s)) return rc;
+    if (int rc = con_reserve(s)) return rc;
     const size_t m0 = s->dist_rest.size();
     for (uint32_t k = 0; k < m; k++) {
         s->dist_pairs.push_back(pairs[2 * k]);
@@ -1476,7 +1562,8 @@ int ps_add_distance_constraints(ps_system *s, uint32_t m, const uint32_t *pairs,
         s->occ[pairs[2 * k]]++;
         s->occ[pairs[2 * k + 1]]++;
     }
-    const int rc = upload_constraints(s);
+    const size_t linked0 = s->linked.size();
+    const int rc = upload_constraints(s, m0);
     if (rc) {
         // keep the host sets equal to what the device last received: undo
         // this call's constraints and re-upload the earlier ones (best effort;
@@ -1488,8 +1575,14 @@ int ps_add_distance_constraints(ps_system *s, uint32_t m, const uint32_t *pairs,
         s->dist_pairs.resize(2 * m0);
         s->dist_rest.resize(m0);
         s->dist_stiff.resize(m0);
+        for (size_t q = linked0; q < s->linked.size(); q++) s->mark[s->linked[q]] &= ~ps::kMarkDist;
+        s->linked.resize(linked0);
         const std::string why = s->err;
-        (void)upload_constraints(s);
+        Touched back;
+        for (uint32_t k = 0; k < 2 * m; k++) back.add(pairs[k]);
+        (void)back.upload(s->b.occ, s->occ);
+        (void)back.upload(s->b.omark, s->mark);
+        (void)upload_constraints(s, m0);
         s->err = why;
     }
     return rc;
@@ -1515,6 +1608,7 @@ int ps_add_point_constraints(ps_system *s, uint32_t m, const uint32_t *idx, cons
     HIP_TRY(s, hipStreamSynchronize(s->stream));
     drop_graph(s);
     const size_t np0 = s->pin_xyz.size();
+    Touched touched;
     std::vector<std::pair<uint32_t, uint32_t>> prev;  // (particle, its pin before this call)
     for (uint32_t k = 0; k < m; k++) {
         const uint32_t pid = (uint32_t)(s->pin_xyz.size() / 3);
@@ -1523,19 +1617,22 @@ int ps_add_point_constraints(ps_system *s, uint32_t m, const uint32_t *idx, cons
         s->pin_xyz.push_back(xyz[3 * k + 2]);
         prev.emplace_back(idx[k], s->pin_of[idx[k]]);
         s->pin_of[idx[k]] = pid + 1;
+        s->mark[idx[k]] |= ps::kMarkPin;
         s->occ[idx[k]]++;
+        touched.add(idx[k]);
     }
-    const int rc = upload_pins(s);
+    const int rc = upload_pins(s, touched);
     if (rc) {
         // undo this call's pins (in reverse, so a particle pinned twice gets
         // its first value back) and re-upload the earlier ones (best effort)
         for (size_t k = prev.size(); k-- > 0;) {
             s->pin_of[prev[k].first] = prev[k].second;
+            if (!prev[k].second) s->mark[prev[k].first] &= ~ps::kMarkPin;
             s->occ[prev[k].first]--;
         }
         s->pin_xyz.resize(np0);
         const std::string why = s->err;
-        (void)upload_pins(s);
+        (void)upload_pins(s, touched);
         s->err = why;
     }
     return rc;
@@ -1640,6 +1737,9 @@ int ps_add_rigid_bodies(ps_system *s, uint32_t nbody, const uint32_t *offsets,
     HIP_TRY(s, hipMemcpy(b.body_mass, s->body_mass.data(), sizeof(float) * nb, hipMemcpyHostToDevice));
     HIP_TRY(s, hipMemcpy(b.body_of, s->body_of.data(), sizeof(uint32_t) * s->cap, hipMemcpyHostToDevice));
     HIP_TRY(s, hipMemcpy(b.member_of, s->member_of.data(), sizeof(uint32_t) * s->cap, hipMemcpyHostToDevice));
+    for (uint32_t k = 0; k < total; k++) s->mark[idx[k]] |= ps::kMarkBody;
+    HIP_TRY(s, hipMemcpy(b.omark, s->mark.data(), s->n, hipMemcpyHostToDevice));
+    b.nbody = (uint32_t)nb;
     if (first_body_out) *first_body_out = bfirst;
     drop_graph(s);
     return PS_OK;

@@ -8,9 +8,8 @@
 
 namespace ps {
 
-__device__ __forceinline__ uint32_t xcd_block()
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b = blockIdx.x, uint32_t nb = gridDim.x)
 {
-    const uint32_t nb = gridDim.x, b = blockIdx.x;
     const uint32_t x = b & 7u, q = nb >> 3, r = nb & 7u;
     return x * q + (x < r ? x : r) + (b >> 3);
 }
@@ -253,32 +252,6 @@ __device__ __forceinline__ void for_neighbors_half(const DevBuffers &b, uint32_t
     }
 }
 
-// Half h of particle i's first c neighbours, one chunk at a time as
-// for_neighbors_chunked (four records in flight): for a kernel whose
-// records or arithmetic are large that gives each half its own lane.
-template <typename G, typename Fn>
-__device__ __forceinline__ void for_neighbors_half_chunked(const DevBuffers &b, uint32_t i, uint32_t c,
-                                                           uint32_t h, G gather, Fn fn)
-{
-    const uint32_t nch = (c + 3u) >> 2;  // chunks in use; half h has 2m + h
-    if (h >= nch) return;
-    const uint4 *nb = nbr_lane(b, i);
-    uint4 jj = nb[(size_t)h * 64];
-    for (uint32_t m = h; m < nch; m += 2u) {
-        const uint4 jn = nb[(size_t)(m + 2u < nch ? m + 2u : m) * 64];
-        auto d0 = gather(jj.x);
-        auto d1 = gather(jj.y);
-        auto d2 = gather(jj.z);
-        auto d3 = gather(jj.w);
-        const uint32_t q = m << 2;
-        fn(jj.x, d0);
-        if (q + 1 < c) fn(jj.y, d1);
-        if (q + 2 < c) fn(jj.z, d2);
-        if (q + 3 < c) fn(jj.w, d3);
-        jj = jn;
-    }
-}
-
 // The chunks first, first + stride, first + 2 stride, ... of particle i's
 // first c neighbours, one chunk at a time (four records in flight), each in
 // table order: quarter q of the table is first = q, stride = 4.
@@ -397,57 +370,6 @@ __device__ __forceinline__ void for_neighbors_split(const DevBuffers &b, uint32_
     }
 }
 
-// As for_neighbors, one chunk at a time: the four gathers of chunk m are
-// issued together (and the index load of chunk m+1), then processed.  Half
-// the records in flight, for kernels whose records or arithmetic are large.
-template <typename G, typename Fn>
-__device__ __forceinline__ void for_neighbors_chunked(const DevBuffers &b, uint32_t i, uint32_t c, G gather,
-                                                      Fn fn)
-{
-    if (c == 0) return;
-    const uint4 *nb = nbr_lane(b, i);
-    const uint32_t last = (c - 1) >> 2;
-    uint4 jj = nb[0];
-    for (uint32_t m = 0; m <= last; m++) {
-        const uint4 jn = nb[(size_t)min(m + 1, last) * 64];
-        auto d0 = gather(jj.x);
-        auto d1 = gather(jj.y);
-        auto d2 = gather(jj.z);
-        auto d3 = gather(jj.w);
-        const uint32_t q = m << 2;
-        fn(jj.x, d0);
-        if (q + 1 < c) fn(jj.y, d1);
-        if (q + 2 < c) fn(jj.z, d2);
-        if (q + 3 < c) fn(jj.w, d3);
-        jj = jn;
-    }
-}
-
-// As for_neighbors_chunked, and fn(h, j, record) is told the half h of the
-// table the entry lies in (its chunk's parity).
-template <typename G, typename Fn>
-__device__ __forceinline__ void for_neighbors_chunked_h(const DevBuffers &b, uint32_t i, uint32_t c, G gather,
-                                                        Fn fn)
-{
-    if (c == 0) return;
-    const uint4 *nb = nbr_lane(b, i);
-    const uint32_t last = (c - 1) >> 2;
-    uint4 jj = nb[0];
-    for (uint32_t m = 0; m <= last; m++) {
-        const uint4 jn = nb[(size_t)min(m + 1, last) * 64];
-        auto d0 = gather(jj.x);
-        auto d1 = gather(jj.y);
-        auto d2 = gather(jj.z);
-        auto d3 = gather(jj.w);
-        const uint32_t q = m << 2, h = m & 1u;
-        fn(h, jj.x, d0);
-        if (q + 1 < c) fn(h, jj.y, d1);
-        if (q + 2 < c) fn(h, jj.z, d2);
-        if (q + 3 < c) fn(h, jj.w, d3);
-        jj = jn;
-    }
-}
-
 struct PA {
     float4 p;
     Attr a;
@@ -461,19 +383,6 @@ struct PX {
 struct PM {
     float4 p;
     float m;
-};
-
-// the same and the phase (a staged unit's contact records)
-struct PMH {
-    float4 p;
-    float m;
-    int32_t ph;
-};
-
-// a staged position and phase
-struct PH {
-    float4 p;
-    int32_t ph;
 };
 
 // entry q of particle i (single-entry access for the less travelled loops)

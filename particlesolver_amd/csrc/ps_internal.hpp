@@ -75,9 +75,8 @@ struct CrConst {
     uint64_t seed;
 };
 
-// Scene-composition switches chosen on the host per launch; each selects a
-// separately compiled variant of the solve kernel, so a pure-fluid scene runs
-// without the contact/distance/shape code paths.
+// Scene-composition switches; a scene of F_FLUID alone runs the solve without
+// the code of the others.
 enum SolveFeature : uint32_t {
     F_FLUID = 1u,
     F_CONTACT = 2u,
@@ -110,18 +109,22 @@ constexpr uint32_t kStageChunks = kStageSlots / kStageChunk;
 // the staged kernels visit whole chunks without bound checks.
 constexpr uint32_t kStageSentinel = kStageSlots;
 
-// Contacts a particle of the global-slot solve lists in LDS during its
-// counting walk; the corrections visit the listed ones, or walk the whole
-// table again when there are more.
+// Contacts that the constraint blocks list in LDS per lane of their counting
+// walk in the global-slot variants (the staged ones have room for 24); the
+// four lanes of a half share theirs, and walk the half again when it holds
+// more.
 constexpr uint32_t kContactList = 16;
-// the same per lane in the staged solve (two lanes per particle, each over
-// one half of the table)
-constexpr uint32_t kHalfContactList = 8;
+
+// What a particle has beside the fluid (DevBuffers::omark, smark).
+enum Mark : uint8_t {
+    kMarkDist = 1,  // distance constraints, and w != 0
+    kMarkBody = 2,  // a rigid body
+    kMarkPin = 4,   // a pin
+};
 
 struct StageDesc {
     uint32_t staged;              // 1: the unit's table entries are LDS indices
     uint32_t nchunks;             // chunks in use
-    uint32_t walk;                // 1: a particle of the unit walks its table for contacts
     uint32_t src[kStageChunks];   // global slot of each chunk's first element
 };
 
@@ -144,11 +147,19 @@ struct DevBuffers {
                            // neighbour, 1/w (times s_solid if not fluid), or -1
                            // for w = 0 (left out of the fluid sums)
     int32_t *phs;          // per slot, written with mj: the phase, its sign bit
-                           // set for w = 0 (the staged solve's contact records)
-    uint32_t contacts;     // the scene has contact phases (then phs is written)
-    uint32_t solve_units;  // staged solve launches: 0 every unit, 1 the units without a
-                           // contact-walking particle, 2 the units with one
-    uint32_t split_solve;  // such particles are rare: launch the two classes apart
+                           // set for w = 0 (the contact walk's records)
+    uint8_t *omark, *smark;  // Mark bits per insertion index, and (the sort, with mj) per slot
+    // constraint blocks of the lambda launch: the slots of the particles that
+    // walk their table for contacts and of those with distance constraints
+    // (written by the sort at the particle's rank among them), the latter's
+    // links (partner index, rest, stiffness, the partner's w) and their own w
+    // and incidence count; and per slot of one of them its corrections of the
+    // iteration
+    uint32_t *walk_rank, *link_rank, *walk_slot, *link_slot, *link_off;
+    float4 *links;
+    float2 *link_own;
+    float4 *con_c, *con_d;
+    uint32_t nwalk, nlink, nbody, con_blocks;
     SceneDev *scenes;
     // grid
     uint32_t *cell_count;  // num_cells, zero between builds
@@ -256,9 +267,8 @@ struct AdjBuffers {
 // here before calling a launcher, and the launcher's kernel, started with
 // PS_LAUNCH, takes it (hipExtLaunchKernelGGL records the pair at the
 // kernel's own start and end, so no stream interval outside the kernel lies
-// between them) and clears it.  Launchers of two kernels leave it (the scan)
-// or split it (the solve of a scene with contacts: the first launch records
-// the start, the second the end).
+// between them) and clears it.  A launcher of two kernels (the scan) leaves
+// it alone.
 struct LaunchEvents {
     hipEvent_t start = nullptr, stop = nullptr;
 };
@@ -291,7 +301,6 @@ hipError_t launch_neighbors(hipStream_t st, const DevBuffers &b, const KConst &k
                             uint32_t kmax, uint32_t bs);
 hipError_t launch_lambda(hipStream_t st, const DevBuffers &b, const KConst &k, uint32_t n,
                          bool uniform, float wu, uint32_t bs);
-hipError_t launch_shape(hipStream_t st, const DevBuffers &b, uint32_t nbody);
 // it: iteration index inside the current substep (the RNG key is the device
 // iteration counter + it); finalize advances the counter by `its`.
 hipError_t launch_solve(hipStream_t st, const DevBuffers &b, const KConst &k, uint32_t n,

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(kBlock) void scatter_k(DevBuffers b, uint32_t n)
 // of (hash, index) in sortParticles (integration.cu:270-275) is meant to
 // give.  Every per-particle array moves with the particle.
 // mj_solid >= 0: also write mj (the neighbour density mass) with s_solid =
-// mj_solid.
+// mj_solid, and the particle's marks.
 __global__ __launch_bounds__(kMaxBlock) void reorder_k(DevBuffers b, uint32_t n, float mj_solid)
 {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -301,8 +301,13 @@ __global__ __launch_bounds__(kMaxBlock) void reorder_k(DevBuffers b, uint32_t n,
             if (a.phase != PS_PHASE_FLUID) m = m * mj_solid;
         }
         b.mj[d] = m;
-        // the phase as the staged contact walk reads it
+        // the phase as the contact walk reads it
         b.phs[d] = a.w != 0.0f ? a.phase : (int32_t)((uint32_t)a.phase | 0x80000000u);
+        // where the constraint blocks find it
+        const uint8_t mark = b.omark[a.orig];
+        b.smark[d] = mark;
+        if (a.phase >= PS_PHASE_CLOTH && a.w != 0.0f) b.walk_slot[b.walk_rank[a.orig]] = d;
+        if (mark & kMarkDist) b.link_slot[b.link_rank[a.orig]] = d;
     }
     if (b.sid) b.sid2[d] = b.sid[s];
     // a scatter by insertion index: skipped when no kernel reads it
@@ -516,7 +521,7 @@ __device__ __forceinline__ void stage_copy(const StageSrc<THREADS> &ss, uint32_t
 // particles).
 
 struct UnitPlan {  // in LDS
-    uint32_t wfirst[4], wlast[4], wheads[4], wwalk[4], total;
+    uint32_t wfirst[4], wlast[4], wheads[4], total;
     uint32_t rrow[kStageRows], xa[kStageRows], xb[kStageRows];
     uint32_t st[kStageIv], en[kStageIv], delta[kStageIv];  // per interval
     uint32_t src[kStageChunks];
@@ -557,7 +562,7 @@ __device__ __forceinline__ uint32_t lane_u(uint32_t v, uint32_t l)
 
 struct Planned {
     bool staged;
-    uint32_t nch, walk;
+    uint32_t nch;
     GridOf gr;          // of the thread's particle (tid of the unit)
     uint32_t row, x;    // its cell: row = z gy + y
 };
@@ -581,9 +586,6 @@ __device__ __forceinline__ Planned plan_unit(const DevBuffers &b, const KConst &
     r.gr = grid_of(b, k, sid);
     const GridOf gr = r.gr;
     const uint32_t key = pv ? b.key[ui] - gr.base : 0u;
-    // whether the particle walks its table for contacts (phase from cloth
-    // up, w != 0: the sign bit of phs clear), loaded beside the key
-    const bool walker = pv && b.contacts && b.phs[ui] >= PS_PHASE_CLOTH;
     const uint32_t row = key / gr.gx, x = key % gr.gx;
     r.row = row;
     r.x = x;
@@ -596,20 +598,14 @@ __device__ __forceinline__ Planned plan_unit(const DevBuffers &b, const KConst &
     const bool head = pv && (tid == 0u || row != prev);
     const bool tail = pv && (tid + 1u == nu || row != next);
     const uint64_t hm = __ballot(head);
-    const uint64_t wm = __ballot(walker);
-    if (lane == 0u) {
-        L.wheads[w] = (uint32_t)__popcll(hm);
-        L.wwalk[w] = wm != 0ull ? 1u : 0u;
-    }
+    if (lane == 0u) L.wheads[w] = (uint32_t)__popcll(hm);
     __syncthreads();
-    uint32_t before = 0, nrows = 0, walk = 0;
+    uint32_t before = 0, nrows = 0;
 #pragma unroll
     for (uint32_t q = 0; q < 4; q++) {
         before += q < w ? L.wheads[q] : 0u;
         nrows += L.wheads[q];
-        walk |= L.wwalk[q];
     }
-    r.walk = walk;
     const bool planned = one_scene && nrows <= kStageRows;
     if (planned && pv) {
         const uint64_t upto = lane == 63u ? ~0ull : ((2ull << lane) - 1ull);
@@ -694,7 +690,6 @@ __device__ __forceinline__ void put_desc(StageDesc *desc, const Planned &pl, con
     if (tid == 0u) {
         desc->staged = pl.staged ? 1u : 0u;
         desc->nchunks = pl.nch;
-        desc->walk = pl.walk;
     }
     if (tid < pl.nch) desc->src[tid] = L.src[tid];
 }
@@ -1086,6 +1081,381 @@ __global__ __launch_bounds__(kStageUnit) void neighbors_split_k(DevBuffers b, KC
 }
 
 // ---------------------------------------------------------------------------
+// a12: shape matching per body (one wavefront per body): centre of mass, A_pq,
+// rotation by the fixed-point quaternion iteration (Mueller, Bender,
+// Chentanez, Macklin, MIG 2016) with a first-order quaternion step, goals.
+
+__device__ __forceinline__ void quat_to_mat(float w, float x, float y, float z, float *m)
+{
+    m[0] = 1.0f - (2.0f * ((y * y) + (z * z)));
+    m[1] = 2.0f * ((x * y) - (w * z));
+    m[2] = 2.0f * ((x * z) + (w * y));
+    m[3] = 2.0f * ((x * y) + (w * z));
+    m[4] = 1.0f - (2.0f * ((x * x) + (z * z)));
+    m[5] = 2.0f * ((y * z) - (w * x));
+    m[6] = 2.0f * ((x * z) - (w * y));
+    m[7] = 2.0f * ((y * z) + (w * x));
+    m[8] = 1.0f - (2.0f * ((x * x) + (y * y)));
+}
+
+// The sum of v over the 64 lanes in pairwise order, v[l] + v[l + s] for
+// s = 32, 16, ..., 1 (the oracle's lane_tree_sum), returned to every lane.
+__device__ __forceinline__ float wave_tree_sum(float v)
+{
+#pragma unroll
+    for (uint32_t s = 32; s > 0; s >>= 1) v = v + __shfl_down(v, s, 64);
+    return __shfl(v, 0, 64);
+}
+
+// One wavefront per body: member q (of a0..a1) belongs to lane (q - a0) %
+// 64, each lane sums its members in order and the lanes are added pairwise;
+// every lane then runs the same rotation iteration on the same sums, and
+// the members' goals are written lane-parallel.
+__device__ __forceinline__ void shape_body(const DevBuffers &b, uint32_t bd)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t a0 = b.body_off[bd], a1 = b.body_off[bd + 1];
+    const float M = b.body_mass[bd];
+    float cx = 0.0f, cy = 0.0f, cz = 0.0f;
+    for (uint32_t q = a0 + lane; q < a1; q += 64u) {
+        const uint32_t t = b.slot_of[b.body_idx[q]];
+        const float m = 1.0f / b.A[t].w;
+        const float4 p = b.P[t];
+        cx = cx + (m * p.x);
+        cy = cy + (m * p.y);
+        cz = cz + (m * p.z);
+    }
+    cx = wave_tree_sum(cx) / M;
+    cy = wave_tree_sum(cy) / M;
+    cz = wave_tree_sum(cz) / M;
+    float A[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (uint32_t q = a0 + lane; q < a1; q += 64u) {
+        const uint32_t t = b.slot_of[b.body_idx[q]];
+        const float m = 1.0f / b.A[t].w;
+        const float4 p = b.P[t];
+        const float ux = m * (p.x - cx), uy = m * (p.y - cy), uz = m * (p.z - cz);
+        const float4 r = b.body_rest[q];
+        A[0] = A[0] + (ux * r.x); A[1] = A[1] + (ux * r.y); A[2] = A[2] + (ux * r.z);
+        A[3] = A[3] + (uy * r.x); A[4] = A[4] + (uy * r.y); A[5] = A[5] + (uy * r.z);
+        A[6] = A[6] + (uz * r.x); A[7] = A[7] + (uz * r.y); A[8] = A[8] + (uz * r.z);
+    }
+#pragma unroll
+    for (int e = 0; e < 9; e++) A[e] = wave_tree_sum(A[e]);
+    float4 qt = b.body_q[bd];
+    float qw = qt.x, qx = qt.y, qy = qt.z, qz = qt.w;
+    for (int it = 0; it < 10; it++) {
+        float m[9];
+        quat_to_mat(qw, qx, qy, qz, m);
+        float ox = 0.0f, oy = 0.0f, oz = 0.0f, dot = 0.0f;
+        for (int col = 0; col < 3; col++) {
+            float rx = m[col], ry = m[3 + col], rz = m[6 + col];
+            float ax_ = A[col], ay_ = A[3 + col], az_ = A[6 + col];
+            ox = ox + ((ry * az_) - (rz * ay_));
+            oy = oy + ((rz * ax_) - (rx * az_));
+            oz = oz + ((rx * ay_) - (ry * ax_));
+            dot = dot + (((rx * ax_) + (ry * ay_)) + (rz * az_));
+        }
+        float den = (dot < 0.0f ? -dot : dot) + 1e-9f;
+        ox = ox / den;
+        oy = oy / den;
+        oz = oz / den;
+        float wl2 = ((ox * ox) + (oy * oy)) + (oz * oz);
+        if (wl2 < 1e-18f) break;  // the same on every lane
+        float dw = 1.0f, dx = ox * 0.5f, dy = oy * 0.5f, dz = oz * 0.5f;
+        float nw = (((dw * qw) - (dx * qx)) - (dy * qy)) - (dz * qz);
+        float nx = (((dw * qx) + (dx * qw)) + (dy * qz)) - (dz * qy);
+        float ny = (((dw * qy) - (dx * qz)) + (dy * qw)) + (dz * qx);
+        float nz = (((dw * qz) + (dx * qy)) - (dy * qx)) + (dz * qw);
+        float nl = sqrtf((((nw * nw) + (nx * nx)) + (ny * ny)) + (nz * nz));
+        qw = nw / nl;
+        qx = nx / nl;
+        qy = ny / nl;
+        qz = nz / nl;
+    }
+    if (lane == 0) b.body_q[bd] = make_float4(qw, qx, qy, qz);
+    float m[9];
+    quat_to_mat(qw, qx, qy, qz, m);
+    for (uint32_t q = a0 + lane; q < a1; q += 64u) {
+        const float4 r = b.body_rest[q];
+        b.body_goal[q] = make_float4((((m[0] * r.x) + (m[1] * r.y)) + (m[2] * r.z)) + cx,
+                                     (((m[3] * r.x) + (m[4] * r.y)) + (m[5] * r.z)) + cy,
+                                     (((m[6] * r.x) + (m[7] * r.y)) + (m[8] * r.z)) + cz, 0.0f);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// a7 and a9 of one iteration, for the particles that have them: contact
+// corrections of those that walk their table for contacts (walk_slot: phase
+// from cloth up, w != 0) to con_c (xyz, and the contact count in w), distance
+// corrections of those with distance constraints (link_slot) to con_d.  Neither
+// reads lambda, so they and shape matching are the first blocks of the lambda
+// launch (constraint_block), beside the fluid's, and the solve adds their
+// results in its order.
+//
+// Inside the solve, a walker's chain of waits (its table, the partners'
+// records, its constraints' indices, pairs, slots and records) held up the 31
+// others of its wavefront, and the contact lists and staged phases took its
+// block from 49 to 78 KB of LDS, two blocks a CU instead of three.  Lambda,
+// shape matching and solve, before and with these blocks, in us a launch:
+// 766k particles (cloth 65k, 3,125 bodies) 42 + 20 + 143, 119 + 49; an
+// ensemble of 2.6M with 128 ropes 118 + 187 (solve), 121 + 142; 7k mixed
+// 5.2 + 9.1 + 12.5, 11.3 + 6.9; cloth over a pool, 82k, 10 + 24, 12 + 11.
+
+// the value of lane S of each four
+template <int S>
+__device__ __forceinline__ uint32_t quad_value(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, S * 0x55, 0xf, 0xf, false);
+}
+template <int S>
+__device__ __forceinline__ float quad_value(float v)
+{
+    return __uint_as_float(quad_value<S>(__float_as_uint(v)));
+}
+
+// a7: particle contacts + friction (collideD, integration_kernel.cuh:358-462).
+// The corrections are summed in the two halves of the table, each in table
+// order, then added half 0 + half 1 (the oracle's order).  Eight lanes a
+// particle, four a half: in the counting walk lane s of the four takes every
+// fourth chunk of its half (with up to 32 neighbours one chunk each, so the
+// chain of table, slots and records is waited for once), and the contacts are
+// listed in the half's LDS in table order; then each of the four forms the
+// terms of every fourth contact (about 300 VALU between solids) and all add
+// them in order.  With one lane a half the lambda launch was 23.6 us at the
+// 82k cloth scene and 15.0 at its 5k one (12.3 and 7.6 with four: a chain of
+// up to eight chunks, one after the other, is what it waited for), and 115 at
+// the 766k scene (119), which has walkers enough to hide it.
+__device__ __forceinline__ void constrain_contacts(const DevBuffers &b, const KConst &k, uint32_t q, uint32_t lane8,
+                                                   uint32_t *list, uint32_t cap)
+{
+    const uint32_t hh = lane8 >> 2, s = lane8 & 3u;
+    const uint32_t i = b.walk_slot[q];
+    const Attr a = b.A[i];
+    const float4 p = b.P[i], xi = b.X[i];
+    const uint32_t c = b.ncnt[i];
+    const StageDesc *d = b.stage + i / kStageUnit;
+    const bool staged = b.staging && d->staged;
+    const float px = p.x, py = p.y, pz = p.z;
+    const int32_t ph = a.phase;
+    const float wi = a.w;
+    const uint32_t nch = (c + 3u) >> 2, half = nch > hh ? (nch - hh + 1u) >> 1 : 0u;  // chunks hh + 2t
+    auto chunk = [&](uint32_t t) {
+        if (!staged) return nbr_lane(b, i)[(size_t)(hh + 2u * t) * 64];
+        const uint2 e = *nbr16_chunk(b, i, hh + 2u * t);
+        return make_uint4(e.x & 0xffffu, e.x >> 16, e.y & 0xffffu, e.y >> 16);
+    };
+    // the slot of an entry (a staged unit's sentinel padding maps to i)
+    auto slot = [&](uint32_t e) {
+        return !staged ? e : e >= kStageSlots ? i : d->src[e / kStageChunk] + e % kStageChunk;
+    };
+    auto is_contact = [&](const float4 &qj, int32_t pj) {
+        if (ph > PS_PHASE_SOLID && ph == pj) return false;
+        const float dx = px - qj.x, dy = py - qj.y, dz = pz - qj.z;
+        const float r2 = ((dx * dx) + (dy * dy)) + (dz * dz);
+        return r2 < k.collide_r2;
+    };
+    uint32_t found = 0;  // contacts of the half (listed up to cap), the same in its four lanes
+    for (uint32_t t0 = 0; t0 < half; t0 += 4u) {
+        const uint32_t t = t0 + s;
+        uint32_t mine = 0, j[4] = {i, i, i, i};  // a bit per contact of the chunk
+        if (t < half) {
+            const uint4 e = chunk(t);
+            j[0] = slot(e.x);
+            j[1] = slot(e.y);
+            j[2] = slot(e.z);
+            j[3] = slot(e.w);
+            float4 r[4];
+            int32_t pj[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) {
+                r[u] = b.P[j[u]];
+                pj[u] = b.phs[j[u]] & 0x7fffffff;
+            }
+            const uint32_t at = (hh + 2u * t) << 2;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++)
+                if (at + u < c && is_contact(r[u], pj[u])) mine |= 1u << u;
+        }
+        const uint32_t n = (uint32_t)__popc(mine);
+        const uint32_t n0 = quad_value<0>(n), n1 = quad_value<1>(n), n2 = quad_value<2>(n), n3 = quad_value<3>(n);
+        uint32_t m = found + (s > 0u ? n0 : 0u) + (s > 1u ? n1 : 0u) + (s > 2u ? n2 : 0u);
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++)
+            if (mine & (1u << u)) {
+                if (m < cap) list[m] = j[u];
+                m++;
+            }
+        found += n0 + n1 + n2 + n3;
+    }
+    const uint32_t nc = found + __shfl_xor(found, 4, 64);
+    float cx = 0.0f, cy = 0.0f, cz = 0.0f;  // the half's sum
+    if (nc > 0) {
+        const float fnc = (float)nc;
+        const float ewi = wi * ps_exp(py);
+        // a contact's terms: e is added, then f subtracted (0 if left out:
+        // the sums start at +0 and never are -0)
+        struct Terms {
+            float ex, ey, ez, fx, fy, fz;
+        };
+        auto terms = [&](uint32_t j) {
+            Terms r = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+            const float4 qj = b.P[j];
+            const Attr aj = b.A[j];
+            const int32_t pj = aj.phase;
+            float dx = px - qj.x, dy = py - qj.y, dz = pz - qj.z;
+            float r2 = ((dx * dx) + (dy * dy)) + (dz * dz);
+            float dist = sqrtf(r2);
+            if (dist < 1e-6f) return r;
+            const float wj = aj.w;
+            float cw = wi, cw2 = wj;
+            const bool solid = ph >= PS_PHASE_SOLID && pj >= PS_PHASE_SOLID;
+            if (solid) {
+                cw = ewi;
+                cw2 = wj * ps_exp(qj.y);
+            }
+            float wsum = cw + cw2;
+            if (wsum == 0.0f) return r;
+            float mag = dist - k.collide_dist;
+            float sc = (((mag / wsum) / dist) * cw) / fnc;
+            r.ex = -(sc * dx);
+            r.ey = -(sc * dy);
+            r.ez = -(sc * dz);
+            if (!solid) return r;
+            const float4 xj = b.X[j];
+            float sc2 = (((mag / wsum) / dist) * cw2) / fnc;
+            float gx = sc2 * dx, gy = sc2 * dy, gz = sc2 * dz;
+            float rx = ((px + r.ex) - xi.x) - ((qj.x + gx) - xj.x);
+            float ry = ((py + r.ey) - xi.y) - ((qj.y + gy) - xj.y);
+            float rz = ((pz + r.ez) - xi.z) - ((qj.z + gz) - xj.z);
+            float nx = dx / dist, ny = dy / dist, nz = dz / dist;
+            float dn = ((rx * nx) + (ry * ny)) + (rz * nz);
+            float tx = rx - (dn * nx), ty = ry - (dn * ny), tz = rz - (dn * nz);
+            float lt = sqrtf(((tx * tx) + (ty * ty)) + (tz * tz));
+            if (lt < 0.001f) return r;
+            float share = cw / wsum;
+            if (lt < (k.mu_s * dist)) {
+                r.fx = tx * share;
+                r.fy = ty * share;
+                r.fz = tz * share;
+            } else {
+                float f = (k.mu_k * dist) / lt;
+                if (f > 1.0f) f = 1.0f;
+                r.fx = (tx * f) * share;
+                r.fy = (ty * f) * share;
+                r.fz = (tz * f) * share;
+            }
+            return r;
+        };
+        if (found <= cap) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the list is the wavefront's
+            for (uint32_t m = 0; m < found; m += 4u) {
+                Terms r = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                if (m + s < found) r = terms(list[m + s]);
+                cx = (cx + quad_value<0>(r.ex)) - quad_value<0>(r.fx);
+                cy = (cy + quad_value<0>(r.ey)) - quad_value<0>(r.fy);
+                cz = (cz + quad_value<0>(r.ez)) - quad_value<0>(r.fz);
+                cx = (cx + quad_value<1>(r.ex)) - quad_value<1>(r.fx);
+                cy = (cy + quad_value<1>(r.ey)) - quad_value<1>(r.fy);
+                cz = (cz + quad_value<1>(r.ez)) - quad_value<1>(r.fz);
+                cx = (cx + quad_value<2>(r.ex)) - quad_value<2>(r.fx);
+                cy = (cy + quad_value<2>(r.ey)) - quad_value<2>(r.fy);
+                cz = (cz + quad_value<2>(r.ez)) - quad_value<2>(r.fz);
+                cx = (cx + quad_value<3>(r.ex)) - quad_value<3>(r.fx);
+                cy = (cy + quad_value<3>(r.ey)) - quad_value<3>(r.fy);
+                cz = (cz + quad_value<3>(r.ez)) - quad_value<3>(r.fz);
+            }
+        } else {
+            // more contacts than the list holds (rare): each of the four
+            // lanes walks the half again
+            for (uint32_t t = 0; t < half; t++) {
+                const uint4 e = chunk(t);
+                const uint32_t at = (hh + 2u * t) << 2;
+                for (uint32_t u = 0; u < 4u && at + u < c; u++) {
+                    const uint32_t j = slot(u == 0u ? e.x : u == 1u ? e.y : u == 2u ? e.z : e.w);
+                    if (!is_contact(b.P[j], b.phs[j] & 0x7fffffff)) continue;
+                    const Terms r = terms(j);
+                    cx = (cx + r.ex) - r.fx;
+                    cy = (cy + r.ey) - r.fy;
+                    cz = (cz + r.ez) - r.fz;
+                }
+            }
+        }
+    }
+    const float hx = __shfl_xor(cx, 4, 64), hy = __shfl_xor(cy, 4, 64), hz = __shfl_xor(cz, 4, 64);
+    if (!lane8) b.con_c[i] = make_float4(cx + hx, cy + hy, cz + hz, __uint_as_float(nc));
+}
+
+// a9: distance constraints, gathered over a particle's incident list in order
+// (links: the partner's insertion index, rest length, stiffness and the
+// partner's inverse mass).  The partner's position is two loads away; four
+// lanes take a particle's links in turn, three of each at once, so a cloth
+// particle's twelve wait together, and every lane subtracts all terms in
+// order.
+__device__ __forceinline__ void constrain_links(const DevBuffers &b, uint32_t q, uint32_t g)
+{
+    const uint32_t i = b.link_slot[q];
+    const uint32_t a0 = b.link_off[q], a1 = b.link_off[q + 1];
+    const float2 own = b.link_own[q];  // its inverse mass and incidence count
+    const float wi = own.x;
+    const float4 p = b.P[i];
+    float cx = 0.0f, cy = 0.0f, cz = 0.0f;
+    constexpr uint32_t kR = 3;
+    for (uint32_t q0 = a0; q0 < a1; q0 += 4u * kR) {  // the same trip count in the four lanes
+        float4 ln[kR], pj[kR];
+#pragma unroll
+        for (uint32_t r = 0; r < kR; r++) ln[r] = b.links[min(q0 + 4u * r + g, a1 - 1u)];
+#pragma unroll
+        for (uint32_t r = 0; r < kR; r++) pj[r] = b.P[b.slot_of[__float_as_uint(ln[r].x)]];
+#pragma unroll
+        for (uint32_t r = 0; r < kR; r++) {
+            float tx = 0.0f, ty = 0.0f, tz = 0.0f;  // a term that is left out subtracts 0
+            const float dx = p.x - pj[r].x, dy = p.y - pj[r].y, dz = p.z - pj[r].z;
+            const float dist = sqrtf(((dx * dx) + (dy * dy)) + (dz * dz));
+            const float wsum = wi + ln[r].w;
+            if (q0 + 4u * r + g < a1 && !(dist < 1e-6f || wsum == 0.0f)) {
+                const float sc = ((((dist - ln[r].y) / wsum) / dist) * wi) * ln[r].z;
+                tx = sc * dx;
+                ty = sc * dy;
+                tz = sc * dz;
+            }
+            cx = (((cx - quad_value<0>(tx)) - quad_value<1>(tx)) - quad_value<2>(tx)) - quad_value<3>(tx);
+            cy = (((cy - quad_value<0>(ty)) - quad_value<1>(ty)) - quad_value<2>(ty)) - quad_value<3>(ty);
+            cz = (((cz - quad_value<0>(tz)) - quad_value<1>(tz)) - quad_value<2>(tz)) - quad_value<3>(tz);
+        }
+    }
+    if (!g) b.con_d[i] = make_float4(cx / own.y, cy / own.y, cz / own.y, 0.0f);
+}
+
+// Block bid of the constraint blocks: contacts (eight lanes a particle;
+// lds holds their lists, cap entries a lane), links (four lanes), bodies (a
+// wavefront), the longest chains first.
+__host__ __device__ __forceinline__ uint32_t con_parts(const DevBuffers &b, uint32_t threads, uint32_t &walks, uint32_t &links)
+{
+    walks = (8u * b.nwalk + threads - 1u) / threads;
+    links = (4u * b.nlink + threads - 1u) / threads;
+    return walks + links + (64u * b.nbody + threads - 1u) / threads;
+}
+
+__device__ __forceinline__ void constraint_block(const DevBuffers &b, const KConst &k, uint32_t bid, uint32_t *lds,
+                                                 uint32_t cap)
+{
+    uint32_t walks, links;
+    con_parts(b, blockDim.x, walks, links);
+    if (bid < walks) {
+        // a half's list is its four lanes' share
+        const uint32_t q = (bid * blockDim.x + threadIdx.x) >> 3;
+        if (q < b.nwalk)
+            constrain_contacts(b, k, q, threadIdx.x & 7u, lds + (threadIdx.x & ~3u) * cap, 4u * cap);
+    } else if (bid < walks + links) {
+        const uint32_t q = ((bid - walks) * blockDim.x + threadIdx.x) >> 2;
+        if (q < b.nlink) constrain_links(b, q, threadIdx.x & 3u);
+    } else {
+        const uint32_t bd = ((bid - walks - links) * blockDim.x + threadIdx.x) >> 6;
+        if (bd < b.nbody) shape_body(b, bd);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // a5: PBF multiplier (findLambdasD, integration_kernel.cuh:521-593)
 //   rho_i = W(0)/w_i + sum_j s_j W(r)/w_j,  grad_j = a d,
 //   a = (spiky/rho0_i) (h-r)^2 / r,
@@ -1099,8 +1469,11 @@ __global__ __launch_bounds__(kStageUnit) void neighbors_split_k(DevBuffers b, KC
 // UNIFORM: every particle is fluid with inverse mass wu (no Attr gathers).
 
 // TAPE (reverse-pass recording): also store S, D and rho per particle.
+// A scene that is not a uniform fluid: the first con_blocks blocks (a multiple
+// of the XCDs) are its constraints' (constraint_block).  Six wavefronts a
+// SIMD (80 VGPRs) are what three staged blocks a CU take.
 template <bool UNIFORM, bool STAGED, bool TAPE = false>
-__global__ __launch_bounds__(kMaxBlock) void lambda_k(DevBuffers b, KConst k, uint32_t n, float mu)
+__global__ __launch_bounds__(kMaxBlock, UNIFORM ? 1 : 6) void lambda_k(DevBuffers b, KConst k, uint32_t n, float mu)
 {
     // staged: a uniform fluid stages neighbour positions only, 12 bytes
     // per slot (36 KB, so four blocks fit in a CU's LDS where 16-byte slots
@@ -1110,7 +1483,21 @@ __global__ __launch_bounds__(kMaxBlock) void lambda_k(DevBuffers b, KConst k, ui
     // particle (2 kStageUnit threads), lane hh summing half hh
     __shared__ float lds3[STAGED && UNIFORM ? 3 * (kStageSlots + 1) : 1];
     __shared__ float4 lds4[STAGED && !UNIFORM ? kStageSlots + 1 : 1];
-    const uint32_t unit = xcd_block();
+    extern __shared__ uint32_t contact_lds[];
+    uint32_t unit;
+    if constexpr (UNIFORM) {
+        unit = xcd_block();
+    } else {
+        if (blockIdx.x < b.con_blocks) {
+            if (STAGED)
+                constraint_block(b, k, blockIdx.x, reinterpret_cast<uint32_t *>(lds4),
+                                 4u * kStageSlots / (2u * kStageUnit));
+            else
+                constraint_block(b, k, blockIdx.x, contact_lds, kContactList);
+            return;
+        }
+        unit = xcd_block(blockIdx.x - b.con_blocks, gridDim.x - b.con_blocks);
+    }
     const uint32_t hh = STAGED ? (threadIdx.x & 1u) : 0u;
     const uint32_t i = STAGED ? unit * kStageUnit + (threadIdx.x >> 1) : unit * blockDim.x + threadIdx.x;
     bool staged = false;
@@ -1260,31 +1647,23 @@ __global__ __launch_bounds__(kMaxBlock) void lambda_k(DevBuffers b, KConst k, ui
 // ---------------------------------------------------------------------------
 // One Jacobi iteration for every particle: contacts (a7), fluid delta-p
 // (a6), distance (a9), shape goal (a12) summed in that order from the same
-// snapshot P, then walls (a8) and pins (a10); result to Q.
+// snapshot P, then walls (a8) and pins (a10); result to Q.  The contact and
+// distance corrections come from the constraint blocks (con_c, con_d).
 
-// TAPE (reverse-pass recording): also store the fluid sum f (before the
-// division by rho0) and the contact count per particle.
-template <uint32_t F, bool UNIFORM, uint32_t NC, bool STAGED, bool TAPE = false>
+// GEN: the scene has contact phases, constraints, bodies or pins; smark says
+// per slot which of them a particle has.  TAPE (reverse-pass recording): also
+// store the fluid sum f (before the division by rho0) and the contact count
+// per particle.
+template <bool GEN, bool UNIFORM, uint32_t NC, bool STAGED, bool TAPE = false>
 __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uint32_t n, float wu,
                                                   uint32_t it)
 {
     // staged: two lanes per particle (2 kStageUnit threads), lane hh summing
     // half hh of the fluid sum; lane 0 finishes the particle.  The LDS holds
-    // the unit's slots and the sentinel record
-    // In a scene that is not a uniform fluid a particle with w = 0 is
-    // staged as a position at infinity (the fluid sum leaves it out, as the
-    // global path does).  With contacts, in a unit where some particle
-    // walks its table for them (the neighbour build's StageDesc::walk), each
-    // slot's phase is staged as well (lds_ph, from the sort's contiguous phs:
-    // the sign bit set for a particle with w = 0), so the counting walk runs
-    // from LDS, reading the true position of such a particle from global
-    // memory; the corrections gather through the unit's chunk table (s_src).
+    // the unit's slots and the sentinel record.  In a scene that is not a
+    // uniform fluid a particle with w = 0 is staged as a position at infinity
+    // (the fluid sum leaves it out, as the global path does).
     __shared__ float4 lds[STAGED ? kStageSlots + 1 : 1];
-    __shared__ int32_t lds_ph[STAGED && (F & F_CONTACT) ? kStageSlots + 1 : 1];
-    __shared__ uint32_t s_src[STAGED && (F & F_CONTACT) ? kStageChunks : 1];
-    // the contact lists of the block (global-slot variants with contacts):
-    // kContactList entries per thread, entry q of thread t at q blockDim + t
-    extern __shared__ uint32_t contact_lds[];
     const uint32_t unit = xcd_block();
     const uint32_t hh = STAGED ? (threadIdx.x & 1u) : 0u;
     const uint32_t i = STAGED ? unit * kStageUnit + (threadIdx.x >> 1) : unit * blockDim.x + threadIdx.x;
@@ -1297,8 +1676,6 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
     uint32_t c = 0;
     if (STAGED) {
         const StageDesc *d = b.stage + unit;
-        // one class of units per launch (the other class's blocks leave)
-        if (b.solve_units && ((d->walk != 0u) != (b.solve_units == 2u))) return;
         StageSrc<2 * kStageUnit> ss;
         const uint32_t ic = min(i, n - 1u);
         ss.load(d);
@@ -1310,30 +1687,15 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
         const uint32_t nch = d->nchunks;
         const float inf = __builtin_inff();
         if (staged && threadIdx.x == 0) lds[kStageSentinel] = make_float4(inf, inf, inf, 0.0f);
-        if ((F & F_CONTACT) && staged && threadIdx.x == 0) lds_ph[kStageSentinel] = 0;
-        if ((F & F_CONTACT) && staged)
-            for (uint32_t q = threadIdx.x; q < nch; q += blockDim.x) s_src[q] = d->src[q];
         if (UNIFORM && staged)
             stage_copy<6>(ss, nch, n, [&](uint32_t j) { return b.P[j]; },
                           [&](uint32_t l, const float4 &v) { lds[l] = v; });
-        else if ((F & F_CONTACT) && staged && d->walk)
-            stage_copy<6>(ss, nch, n, [&](uint32_t j) { return PMH{b.P[j], b.mj[j], b.phs[j]}; },
-                          [&](uint32_t l, const PMH &v) {
-                              lds[l] = v.m < 0.0f ? make_float4(inf, inf, inf, 0.0f) : v.p;
-                              lds_ph[l] = v.ph;
-                          });
         else if (staged)
             stage_copy<6>(ss, nch, n, [&](uint32_t j) { return PM{b.P[j], b.mj[j]}; },
                           [&](uint32_t l, const PM &v) {
                               lds[l] = v.m < 0.0f ? make_float4(inf, inf, inf, 0.0f) : v.p;
                           });
     }
-    // the storage slot of table entry e (an LDS index in a staged unit; its
-    // sentinel padding, never visited, maps to i)
-    auto slot = [&](uint32_t e) -> uint32_t {
-        if (!(STAGED && (F & F_CONTACT)) || !staged) return e;
-        return e >= kStageSlots ? i : s_src[e >> 4] + (e & (kStageChunk - 1u));
-    };
     if (i >= n) return;
     if (!STAGED) {
         p = b.P[i];
@@ -1346,185 +1708,14 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
     float4 tape = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // (f, contact count) when TAPE
 
-    // a7: particle contacts + friction (collideD, integration_kernel.cuh:358-462)
-    if (F & F_CONTACT) {
-        if (ph >= PS_PHASE_CLOTH && wi != 0.0f) {
-            // The corrections are summed in the two halves of the table, each
-            // in table order, then added half 0 + half 1 (the oracle's
-            // order).  The counting walk lists the contacts in the block's
-            // LDS (entry m of thread t at contact_lds[m blockDim + t]) and
-            // the corrections visit only those, or walk the table again when
-            // the list overflowed.  Global-slot variants: one lane walks both
-            // halves (pipelined two chunks at a time), listing slot | half
-            // << 31.  Staged: each of the pair's two lanes counts and
-            // corrects its own half, listing LDS indices (global slots in a
-            // unit that was not staged), and the halves meet by a shuffle.
-            auto pa = [&](uint32_t e) {
-                const uint32_t j = slot(e);
-                return PA{b.P[j], b.A[j]};
-            };
-            auto is_contact = [&](const PA &d) {
-                if (ph > PS_PHASE_SOLID && ph == d.a.phase) return false;
-                const float4 qj = d.p;
-                float dx = px - qj.x, dy = py - qj.y, dz = pz - qj.z;
-                float r2 = ((dx * dx) + (dy * dy)) + (dz * dz);
-                return r2 < k.collide_r2;
-            };
-            uint32_t *clist = contact_lds + threadIdx.x;
-            const uint32_t cstride = blockDim.x;
-            constexpr uint32_t kList = STAGED ? kHalfContactList : kContactList;
-            uint32_t nc = 0;
-            if constexpr (STAGED) {
-                if (staged) {
-                    // from the staged records: position and phase (a
-                    // particle with w = 0 is staged at infinity and marked
-                    // by the phase's sign bit: its position from memory)
-                    tab.visit(
-                        hh, c, [&](uint32_t e) { return PH{lds[e], lds_ph[e]}; },
-                        [&](uint32_t e, const PH &d) {
-                            const int32_t phj = d.ph & 0x7fffffff;
-                            if (ph > PS_PHASE_SOLID && ph == phj) return;
-                            float qx = d.p.x, qy = d.p.y, qz = d.p.z;
-                            if (d.ph < 0) {
-                                // a rare path; read through a volatile
-                                // pointer, which the compiler cannot merge
-                                // with the staged record's (merged, the
-                                // records went through scratch memory)
-                                const volatile float *g = &b.P[slot(e)].x;
-                                qx = g[0];
-                                qy = g[1];
-                                qz = g[2];
-                            }
-                            float dx = px - qx, dy = py - qy, dz = pz - qz;
-                            float r2 = ((dx * dx) + (dy * dy)) + (dz * dz);
-                            if (r2 < k.collide_r2) {
-                                if (nc < kList) clist[nc * cstride] = e;
-                                nc++;
-                            }
-                        });
-                } else {
-                    for_neighbors_half_chunked(b, i, c, hh, pa, [&](uint32_t e, const PA &d) {
-                        if (is_contact(d)) {
-                            if (nc < kList) clist[nc * cstride] = e;
-                            nc++;
-                        }
-                    });
-                }
-            } else {
-                for_neighbors_chunked_h(b, i, c, pa, [&](uint32_t h, uint32_t j, const PA &d) {
-                    if (is_contact(d)) {
-                        if (nc < kList) clist[nc * cstride] = j | (h << 31);
-                        nc++;
-                    }
-                });
-            }
-            const uint32_t nmine = nc;  // contacts this lane found (and listed up to kList)
-            if (STAGED) nc = nc + __shfl_xor(nc, 1, 64);
-            if (TAPE) tape.w = __uint_as_float(nc);
-            if (nc > 0) {
-                const float fnc = (float)nc;
-                const float ewi = wi * ps_exp(py);
-                const float4 xi = b.X[i];
-                struct C3 {
-                    float x, y, z;
-                };
-                auto correct = [&](C3 &cs, uint32_t e, const PA &d) {
-                    const Attr aj = d.a;
-                    const int32_t pj = aj.phase;
-                    if (ph > PS_PHASE_SOLID && ph == pj) return;
-                    const float4 qj = d.p;
-                    float dx = px - qj.x, dy = py - qj.y, dz = pz - qj.z;
-                    float r2 = ((dx * dx) + (dy * dy)) + (dz * dz);
-                    if (!(r2 < k.collide_r2)) return;
-                    float dist = sqrtf(r2);
-                    if (dist < 1e-6f) return;
-                    const float wj = aj.w;
-                    float cw = wi, cw2 = wj;
-                    const bool solid = ph >= PS_PHASE_SOLID && pj >= PS_PHASE_SOLID;
-                    if (solid) {
-                        cw = ewi;
-                        cw2 = wj * ps_exp(qj.y);
-                    }
-                    float wsum = cw + cw2;
-                    if (wsum == 0.0f) return;
-                    float mag = dist - k.collide_dist;
-                    float sc = (((mag / wsum) / dist) * cw) / fnc;
-                    float ex = -(sc * dx), ey = -(sc * dy), ez = -(sc * dz);
-                    cs.x = cs.x + ex;
-                    cs.y = cs.y + ey;
-                    cs.z = cs.z + ez;
-                    if (!solid) return;
-                    float sc2 = (((mag / wsum) / dist) * cw2) / fnc;
-                    float fx = sc2 * dx, fy = sc2 * dy, fz = sc2 * dz;
-                    const float4 xj = b.X[slot(e)];
-                    float rx = ((px + ex) - xi.x) - ((qj.x + fx) - xj.x);
-                    float ry = ((py + ey) - xi.y) - ((qj.y + fy) - xj.y);
-                    float rz = ((pz + ez) - xi.z) - ((qj.z + fz) - xj.z);
-                    float nx = dx / dist, ny = dy / dist, nz = dz / dist;
-                    float dn = ((rx * nx) + (ry * ny)) + (rz * nz);
-                    float tx = rx - (dn * nx), ty = ry - (dn * ny), tz = rz - (dn * nz);
-                    float lt = sqrtf(((tx * tx) + (ty * ty)) + (tz * tz));
-                    if (lt < 0.001f) return;
-                    float share = cw / wsum;
-                    if (lt < (k.mu_s * dist)) {
-                        cs.x = cs.x - (tx * share);
-                        cs.y = cs.y - (ty * share);
-                        cs.z = cs.z - (tz * share);
-                    } else {
-                        float f = (k.mu_k * dist) / lt;
-                        if (f > 1.0f) f = 1.0f;
-                        cs.x = cs.x - ((tx * f) * share);
-                        cs.y = cs.y - ((ty * f) * share);
-                        cs.z = cs.z - ((tz * f) * share);
-                    }
-                };
-                C3 ch0 = {0.0f, 0.0f, 0.0f}, ch1 = {0.0f, 0.0f, 0.0f};  // the halves
-                if (nmine <= kList) {
-                    // the listed contacts in order, four records in flight
-                    for (uint32_t q0 = 0; q0 < nmine; q0 += 4u) {
-                        uint32_t jq[4];
-                        PA dq[4];
-#pragma unroll
-                        for (uint32_t u = 0; u < 4; u++) jq[u] = clist[min(q0 + u, nmine - 1u) * cstride];
-#pragma unroll
-                        for (uint32_t u = 0; u < 4; u++) dq[u] = pa(STAGED ? jq[u] : (jq[u] & 0x7fffffffu));
-#pragma unroll
-                        for (uint32_t u = 0; u < 4; u++)
-                            if (q0 + u < nmine) {
-                                if (STAGED || !(jq[u] >> 31))
-                                    correct(ch0, jq[u] & (STAGED ? ~0u : 0x7fffffffu), dq[u]);
-                                else
-                                    correct(ch1, jq[u] & 0x7fffffffu, dq[u]);
-                            }
-                    }
-                } else if (STAGED && staged) {
-                    for_staged_half_plain(b, i, c, hh, [&](uint32_t e) { correct(ch0, e, pa(e)); });
-                } else if (STAGED) {
-                    for_neighbors_half_chunked(b, i, c, hh, pa,
-                                               [&](uint32_t e, const PA &d) { correct(ch0, e, d); });
-                } else {
-                    for_neighbors_chunked_h(b, i, c, pa, [&](uint32_t h, uint32_t j, const PA &d) {
-                        if (h)
-                            correct(ch1, j, d);
-                        else
-                            correct(ch0, j, d);
-                    });
-                }
-                if (STAGED) {
-                    // this lane's half is in ch0; the partner lane holds the other
-                    const C3 other = {__shfl_xor(ch0.x, 1, 64), __shfl_xor(ch0.y, 1, 64), __shfl_xor(ch0.z, 1, 64)};
-                    if (hh) {
-                        ch1 = ch0;
-                        ch0 = other;
-                    } else {
-                        ch1 = other;
-                    }
-                }
-                ax = ax + (ch0.x + ch1.x);
-                ay = ay + (ch0.y + ch1.y);
-                az = az + (ch0.z + ch1.z);
-            }
-        }
+    const uint32_t mark = GEN ? b.smark[i] : 0u;
+    // a7: particle contacts + friction
+    if (GEN && ph >= PS_PHASE_CLOTH && wi != 0.0f && (!STAGED || !hh)) {
+        const float4 cc = b.con_c[i];
+        ax = ax + cc.x;
+        ay = ay + cc.y;
+        az = az + cc.z;
+        if (TAPE) tape.w = cc.w;
     }
 
     // a6: PBF delta-p with tensile correction s_corr = -k h^2 (W/W(dq h))^n
@@ -1534,7 +1725,7 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
     // = fma(-w_scale, r^2, w_scale_h2), coef = fma(-k, (W/W(dq h))^n,
     // l_i + l_j), and the term -coef q^2 (1/r) d; spiky multiplies the
     // finished sum
-    if (F & F_FLUID) {
+    {
         if (ph == PS_PHASE_FLUID) {
             const float li = p.w, ir0 = 1.0f / a.rho0;
             // r^2 < 1e-8: gradient (0, -0.001 spiky h^2, 0) (integration_kernel.cuh:625-626)
@@ -1664,93 +1855,25 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
         }
     }
 
-    // a9: distance constraints, gathered over this particle's incident list
-    // in order.  Each is a chain of dependent loads (index, pair, slot,
-    // position, attributes); staged, the particle's two lanes take two at a
-    // time, kR such rounds at once, each level of the chains going out for
-    // all of them together, and lane 0 subtracts the terms in constraint
-    // order
-    if (F & F_DIST) {
-        const uint32_t o = a.orig;
-        const uint32_t a0 = b.dist_off[o], a1 = b.dist_off[o + 1];
-        if (a1 > a0 && wi != 0.0f) {
-            float cx = 0.0f, cy = 0.0f, cz = 0.0f;
-            constexpr uint32_t kStep = STAGED ? 2u : 1u, kR = 3;
-            for (uint32_t q0 = a0; q0 < a1; q0 += kStep * kR) {  // the same trip count in both lanes
-                uint32_t cid[kR], j[kR];
-                bool ok[kR];
-#pragma unroll
-                for (uint32_t r = 0; r < kR; r++) {
-                    const uint32_t q = q0 + kStep * r + (STAGED ? hh : 0u);
-                    ok[r] = q < a1;
-                    cid[r] = b.dist_adj[ok[r] ? q : a0];
-                }
-                uint2 pr[kR];
-#pragma unroll
-                for (uint32_t r = 0; r < kR; r++) pr[r] = b.dist_pairs[cid[r]];
-#pragma unroll
-                for (uint32_t r = 0; r < kR; r++) j[r] = b.slot_of[pr[r].x == o ? pr[r].y : pr[r].x];
-                float4 pj[kR];
-                float wj[kR];
-                float2 rs[kR];
-#pragma unroll
-                for (uint32_t r = 0; r < kR; r++) {
-                    pj[r] = b.P[j[r]];
-                    wj[r] = b.A[j[r]].w;
-                    rs[r] = b.dist_rs[cid[r]];
-                }
-#pragma unroll
-                for (uint32_t r = 0; r < kR; r++) {
-                    float tx = 0.0f, ty = 0.0f, tz = 0.0f;
-                    bool use = false;
-                    float dx = px - pj[r].x, dy = py - pj[r].y, dz = pz - pj[r].z;
-                    float dist = sqrtf(((dx * dx) + (dy * dy)) + (dz * dz));
-                    float wsum = wi + wj[r];
-                    if (ok[r] && !(dist < 1e-6f || wsum == 0.0f)) {
-                        float sc = ((((dist - rs[r].x) / wsum) / dist) * wi) * rs[r].y;
-                        tx = sc * dx;
-                        ty = sc * dy;
-                        tz = sc * dz;
-                        use = true;
-                    }
-                    if (use) {
-                        cx = cx - tx;
-                        cy = cy - ty;
-                        cz = cz - tz;
-                    }
-                    if (STAGED) {
-                        // lane 0: then its partner's constraint of the round
-                        const float ox = __shfl_xor(tx, 1, 64), oy = __shfl_xor(ty, 1, 64),
-                                    oz = __shfl_xor(tz, 1, 64);
-                        if (__shfl_xor(use ? 1 : 0, 1, 64)) {
-                            cx = cx - ox;
-                            cy = cy - oy;
-                            cz = cz - oz;
-                        }
-                    }
-                }
-            }
-            const float occ = (float)b.occ[o];
-            ax = ax + (cx / occ);
-            ay = ay + (cy / occ);
-            az = az + (cz / occ);
-        }
-    }
-
     // staged: the pair's lane 0 finishes the particle
     if (STAGED && hh) return;
 
+    // a9: distance constraints
+    if (GEN && (mark & kMarkDist)) {
+        const float4 cd = b.con_d[i];
+        ax = ax + cd.x;
+        ay = ay + cd.y;
+        az = az + cd.z;
+    }
+
     // a12: shape-matching goal pull
-    if (F & F_SHAPE) {
+    if (GEN && (mark & kMarkBody)) {
         const uint32_t o = a.orig;
-        const uint32_t bo = b.body_of[o];
-        if (bo) {
-            const float4 g = b.body_goal[b.member_of[o]];
-            const float st = b.body_stiff[bo - 1];
-            ax = ax + ((g.x - px) * st);
-            ay = ay + ((g.y - py) * st);
-            az = az + ((g.z - pz) * st);
-        }
+        const float4 g = b.body_goal[b.member_of[o]];
+        const float st = b.body_stiff[b.body_of[o] - 1];
+        ax = ax + ((g.x - px) * st);
+        ay = ay + ((g.y - py) * st);
+        az = az + ((g.z - pz) * st);
     }
 
     float nxp = px + ax, nyp = py + ay, nzp = pz + az;
@@ -1759,15 +1882,12 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
     const uint64_t iter = b.status->iter + it;
     float4 wrec;
     uint32_t set = walls(k, wall_box(k, b, i, a.orig), ph, xs, nxp, nyp, nzp, iter, wrec);
-    if (F & F_PIN) {
-        const uint32_t pin = b.pin_of[a.orig];
-        if (pin) {
-            const float4 t = b.pin_xyz[pin - 1];
-            nxp = t.x;
-            nyp = t.y;
-            nzp = t.z;
-            set |= 7u | kPinned;
-        }
+    if (GEN && (mark & kMarkPin)) {
+        const float4 t = b.pin_xyz[b.pin_of[a.orig] - 1];
+        nxp = t.x;
+        nyp = t.y;
+        nzp = t.z;
+        set |= 7u | kPinned;
     }
     if (TAPE) {
         b.clamp_rec[i] = (uint8_t)set;
@@ -1776,111 +1896,6 @@ __global__ __launch_bounds__(kMaxBlock) void solve_k(DevBuffers b, KConst k, uin
     }
     b.Q[i] = make_float4(nxp, nyp, nzp, 0.0f);
     if (TAPE && b.tape_q) b.tape_q[i] = make_float4(nxp, nyp, nzp, 0.0f);
-}
-
-// ---------------------------------------------------------------------------
-// a12: shape matching per body (one wavefront per body): centre of mass, A_pq,
-// rotation by the fixed-point quaternion iteration (Mueller, Bender,
-// Chentanez, Macklin, MIG 2016) with a first-order quaternion step, goals.
-
-__device__ __forceinline__ void quat_to_mat(float w, float x, float y, float z, float *m)
-{
-    m[0] = 1.0f - (2.0f * ((y * y) + (z * z)));
-    m[1] = 2.0f * ((x * y) - (w * z));
-    m[2] = 2.0f * ((x * z) + (w * y));
-    m[3] = 2.0f * ((x * y) + (w * z));
-    m[4] = 1.0f - (2.0f * ((x * x) + (z * z)));
-    m[5] = 2.0f * ((y * z) - (w * x));
-    m[6] = 2.0f * ((x * z) - (w * y));
-    m[7] = 2.0f * ((y * z) + (w * x));
-    m[8] = 1.0f - (2.0f * ((x * x) + (y * y)));
-}
-
-// The sum of v over the 64 lanes in pairwise order, v[l] + v[l + s] for
-// s = 32, 16, ..., 1 (the oracle's lane_tree_sum), returned to every lane.
-__device__ __forceinline__ float wave_tree_sum(float v)
-{
-#pragma unroll
-    for (uint32_t s = 32; s > 0; s >>= 1) v = v + __shfl_down(v, s, 64);
-    return __shfl(v, 0, 64);
-}
-
-// One wavefront per body: member q (of a0..a1) belongs to lane (q - a0) %
-// 64, each lane sums its members in order and the lanes are added pairwise;
-// every lane then runs the same rotation iteration on the same sums, and
-// the members' goals are written lane-parallel.
-__global__ __launch_bounds__(kBlock) void shape_k(DevBuffers b, uint32_t nbody)
-{
-    const uint32_t bd = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    const uint32_t lane = threadIdx.x & 63u;
-    if (bd >= nbody) return;  // the whole wavefront leaves together
-    const uint32_t a0 = b.body_off[bd], a1 = b.body_off[bd + 1];
-    const float M = b.body_mass[bd];
-    float cx = 0.0f, cy = 0.0f, cz = 0.0f;
-    for (uint32_t q = a0 + lane; q < a1; q += 64u) {
-        const uint32_t t = b.slot_of[b.body_idx[q]];
-        const float m = 1.0f / b.A[t].w;
-        const float4 p = b.P[t];
-        cx = cx + (m * p.x);
-        cy = cy + (m * p.y);
-        cz = cz + (m * p.z);
-    }
-    cx = wave_tree_sum(cx) / M;
-    cy = wave_tree_sum(cy) / M;
-    cz = wave_tree_sum(cz) / M;
-    float A[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (uint32_t q = a0 + lane; q < a1; q += 64u) {
-        const uint32_t t = b.slot_of[b.body_idx[q]];
-        const float m = 1.0f / b.A[t].w;
-        const float4 p = b.P[t];
-        const float ux = m * (p.x - cx), uy = m * (p.y - cy), uz = m * (p.z - cz);
-        const float4 r = b.body_rest[q];
-        A[0] = A[0] + (ux * r.x); A[1] = A[1] + (ux * r.y); A[2] = A[2] + (ux * r.z);
-        A[3] = A[3] + (uy * r.x); A[4] = A[4] + (uy * r.y); A[5] = A[5] + (uy * r.z);
-        A[6] = A[6] + (uz * r.x); A[7] = A[7] + (uz * r.y); A[8] = A[8] + (uz * r.z);
-    }
-#pragma unroll
-    for (int e = 0; e < 9; e++) A[e] = wave_tree_sum(A[e]);
-    float4 qt = b.body_q[bd];
-    float qw = qt.x, qx = qt.y, qy = qt.z, qz = qt.w;
-    for (int it = 0; it < 10; it++) {
-        float m[9];
-        quat_to_mat(qw, qx, qy, qz, m);
-        float ox = 0.0f, oy = 0.0f, oz = 0.0f, dot = 0.0f;
-        for (int col = 0; col < 3; col++) {
-            float rx = m[col], ry = m[3 + col], rz = m[6 + col];
-            float ax_ = A[col], ay_ = A[3 + col], az_ = A[6 + col];
-            ox = ox + ((ry * az_) - (rz * ay_));
-            oy = oy + ((rz * ax_) - (rx * az_));
-            oz = oz + ((rx * ay_) - (ry * ax_));
-            dot = dot + (((rx * ax_) + (ry * ay_)) + (rz * az_));
-        }
-        float den = (dot < 0.0f ? -dot : dot) + 1e-9f;
-        ox = ox / den;
-        oy = oy / den;
-        oz = oz / den;
-        float wl2 = ((ox * ox) + (oy * oy)) + (oz * oz);
-        if (wl2 < 1e-18f) break;  // the same on every lane
-        float dw = 1.0f, dx = ox * 0.5f, dy = oy * 0.5f, dz = oz * 0.5f;
-        float nw = (((dw * qw) - (dx * qx)) - (dy * qy)) - (dz * qz);
-        float nx = (((dw * qx) + (dx * qw)) + (dy * qz)) - (dz * qy);
-        float ny = (((dw * qy) - (dx * qz)) + (dy * qw)) + (dz * qx);
-        float nz = (((dw * qz) + (dx * qy)) - (dy * qx)) + (dz * qw);
-        float nl = sqrtf((((nw * nw) + (nx * nx)) + (ny * ny)) + (nz * nz));
-        qw = nw / nl;
-        qx = nx / nl;
-        qy = ny / nl;
-        qz = nz / nl;
-    }
-    if (lane == 0) b.body_q[bd] = make_float4(qw, qx, qy, qz);
-    float m[9];
-    quat_to_mat(qw, qx, qy, qz, m);
-    for (uint32_t q = a0 + lane; q < a1; q += 64u) {
-        const float4 r = b.body_rest[q];
-        b.body_goal[q] = make_float4((((m[0] * r.x) + (m[1] * r.y)) + (m[2] * r.z)) + cx,
-                                     (((m[3] * r.x) + (m[4] * r.y)) + (m[5] * r.z)) + cy,
-                                     (((m[6] * r.x) + (m[7] * r.y)) + (m[8] * r.z)) + cz, 0.0f);
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2120,131 +2135,84 @@ hipError_t launch_neighbors(hipStream_t st, const DevBuffers &b, const KConst &k
     return hipGetLastError();
 }
 
-hipError_t launch_lambda(hipStream_t st, const DevBuffers &b, const KConst &k, uint32_t n,
+hipError_t launch_lambda(hipStream_t st, const DevBuffers &b0, const KConst &k, uint32_t n,
                          bool uniform, float wu, uint32_t bs)
 {
     if (n == 0) return hipSuccess;
-    const dim3 g(blocks_for(n, bs)), t(bs);
     const float mu = 1.0f / wu;
-    const dim3 gs(blocks_for(n, kStageUnit)), ts(2 * kStageUnit);  // staged: two lanes per particle
-    if (b.tape_lq && b.staging && uniform)  // recording for the reverse pass
-        PS_LAUNCH((lambda_k<true, true, true>), gs, ts, 0, st, b, k, n, mu);
-    else if (b.tape_lq && b.staging)
-        PS_LAUNCH((lambda_k<false, true, true>), gs, ts, 0, st, b, k, n, mu);
-    else if (b.tape_lq && uniform)
-        PS_LAUNCH((lambda_k<true, false, true>), g, t, 0, st, b, k, n, mu);
+    // staged: two lanes per particle
+    const uint32_t threads = b0.staging ? 2u * kStageUnit : bs;
+    const uint32_t blocks = blocks_for(n, b0.staging ? kStageUnit : bs);
+    const dim3 t(threads);
+    if (uniform) {
+        const dim3 g(blocks);
+        if (b0.tape_lq && b0.staging)  // recording for the reverse pass
+            PS_LAUNCH((lambda_k<true, true, true>), g, t, 0, st, b0, k, n, mu);
+        else if (b0.tape_lq)
+            PS_LAUNCH((lambda_k<true, false, true>), g, t, 0, st, b0, k, n, mu);
+        else if (b0.staging)
+            PS_LAUNCH((lambda_k<true, true>), g, t, 0, st, b0, k, n, mu);
+        else
+            PS_LAUNCH((lambda_k<true, false>), g, t, 0, st, b0, k, n, mu);
+        return hipGetLastError();
+    }
+    // the constraint blocks first, in whole turns of the XCDs
+    DevBuffers b = b0;
+    uint32_t walks, links;
+    b.con_blocks = (con_parts(b, threads, walks, links) + 7u) & ~7u;
+    const dim3 g(b.con_blocks + blocks);
+    // contact lists of the global-slot variants (the staged ones' share the
+    // staged cells' LDS)
+    const size_t cl = b.nwalk ? sizeof(uint32_t) * kContactList * bs : 0;
+    if (b.tape_lq && b.staging)
+        PS_LAUNCH((lambda_k<false, true, true>), g, t, 0, st, b, k, n, mu);
     else if (b.tape_lq)
-        PS_LAUNCH((lambda_k<false, false, true>), g, t, 0, st, b, k, n, mu);
-    else if (uniform && b.staging)
-        PS_LAUNCH((lambda_k<true, true>), dim3(blocks_for(n, kStageUnit)), dim3(2 * kStageUnit),
-                           0, st, b, k, n, mu);
+        PS_LAUNCH((lambda_k<false, false, true>), g, t, cl, st, b, k, n, mu);
     else if (b.staging)
-        PS_LAUNCH((lambda_k<false, true>), dim3(blocks_for(n, kStageUnit)), dim3(2 * kStageUnit),
-                           0, st, b, k, n, mu);
-    else if (uniform)
-        PS_LAUNCH((lambda_k<true, false>), g, t, 0, st, b, k, n, mu);
+        PS_LAUNCH((lambda_k<false, true>), g, t, 0, st, b, k, n, mu);
     else
-        PS_LAUNCH((lambda_k<false, false>), g, t, 0, st, b, k, n, mu);
-    return hipGetLastError();
-}
-
-hipError_t launch_shape(hipStream_t st, const DevBuffers &b, uint32_t nbody)
-{
-    if (nbody == 0) return hipSuccess;
-    // one wavefront per body
-    PS_LAUNCH(shape_k, dim3(blocks_for(nbody, kBlock / 64)), dim3(kBlock), 0, st, b, nbody);
+        PS_LAUNCH((lambda_k<false, false>), g, t, cl, st, b, k, n, mu);
     return hipGetLastError();
 }
 
 // NC: tensile exponent known at compile time (4, as in the reference's
 // E_P, integration_kernel.cuh:34) or 0 = read from the parameters
-template <uint32_t F>
-static void solve_variant(hipStream_t st, const DevBuffers &b, const KConst &k, uint32_t n,
-                          bool uniform, float wu, uint32_t iter, uint32_t bs)
+template <bool GEN, bool UNIFORM, uint32_t NC>
+static void solve_variant(hipStream_t st, const DevBuffers &b, const KConst &k, uint32_t n, float wu, uint32_t iter,
+                          uint32_t bs)
 {
     const dim3 g(blocks_for(n, bs)), t(bs);
     const dim3 gs(blocks_for(n, kStageUnit)), ts(2 * kStageUnit);  // two lanes per particle
-    const bool n4 = k.n_corr == 4u;
-    // the contact lists of a block
-    const size_t cl = (F & F_CONTACT) ? sizeof(uint32_t) * kContactList * bs : 0;
-    const size_t cls = (F & F_CONTACT) ? sizeof(uint32_t) * kHalfContactList * 2 * kStageUnit : 0;  // per lane
-    // staged variants for every composition (uniform fluid or not)
-    constexpr bool CAN_STAGE = true;
-    if (b.tape_f && b.staging) {  // recording for the reverse pass
-        if (uniform && n4)
-            PS_LAUNCH((solve_k<F, true, 4, true, true>), gs, ts, cls, st, b, k, n, wu, iter);
-        else if (uniform)
-            PS_LAUNCH((solve_k<F, true, 0, true, true>), gs, ts, cls, st, b, k, n, wu, iter);
-        else if (n4)
-            PS_LAUNCH((solve_k<F, false, 4, true, true>), gs, ts, cls, st, b, k, n, wu, iter);
-        else
-            PS_LAUNCH((solve_k<F, false, 0, true, true>), gs, ts, cls, st, b, k, n, wu, iter);
-        return;
-    }
-    if (b.tape_f) {  // recording for the reverse pass
-        if (uniform && n4)
-            PS_LAUNCH((solve_k<F, true, 4, false, true>), g, t, cl, st, b, k, n, wu, iter);
-        else if (uniform)
-            PS_LAUNCH((solve_k<F, true, 0, false, true>), g, t, cl, st, b, k, n, wu, iter);
-        else if (n4)
-            PS_LAUNCH((solve_k<F, false, 4, false, true>), g, t, cl, st, b, k, n, wu, iter);
-        else
-            PS_LAUNCH((solve_k<F, false, 0, false, true>), g, t, cl, st, b, k, n, wu, iter);
-        return;
-    }
-    if (CAN_STAGE && uniform && b.staging && n4)
-        PS_LAUNCH((solve_k<F, true, 4, CAN_STAGE>), gs, ts, 0, st, b, k, n, wu, iter);
-    else if (CAN_STAGE && uniform && b.staging)
-        PS_LAUNCH((solve_k<F, true, 0, CAN_STAGE>), gs, ts, 0, st, b, k, n, wu, iter);
-    else if (CAN_STAGE && b.staging && n4)
-        PS_LAUNCH((solve_k<F, false, 4, CAN_STAGE>), gs, ts, cls, st, b, k, n, wu, iter);
-    else if (CAN_STAGE && b.staging)
-        PS_LAUNCH((solve_k<F, false, 0, CAN_STAGE>), gs, ts, cls, st, b, k, n, wu, iter);
-    else if (uniform && n4)
-        PS_LAUNCH((solve_k<F, true, 4, false>), g, t, cl, st, b, k, n, wu, iter);
-    else if (uniform)
-        PS_LAUNCH((solve_k<F, true, 0, false>), g, t, cl, st, b, k, n, wu, iter);
-    else if (n4)
-        PS_LAUNCH((solve_k<F, false, 4, false>), g, t, cl, st, b, k, n, wu, iter);
+    if (b.tape_f && b.staging)  // recording for the reverse pass
+        PS_LAUNCH((solve_k<GEN, UNIFORM, NC, true, true>), gs, ts, 0, st, b, k, n, wu, iter);
+    else if (b.tape_f)
+        PS_LAUNCH((solve_k<GEN, UNIFORM, NC, false, true>), g, t, 0, st, b, k, n, wu, iter);
+    else if (b.staging)
+        PS_LAUNCH((solve_k<GEN, UNIFORM, NC, true>), gs, ts, 0, st, b, k, n, wu, iter);
     else
-        PS_LAUNCH((solve_k<F, false, 0, false>), g, t, cl, st, b, k, n, wu, iter);
+        PS_LAUNCH((solve_k<GEN, UNIFORM, NC, false>), g, t, 0, st, b, k, n, wu, iter);
+}
+
+template <uint32_t NC>
+static void solve_composition(hipStream_t st, const DevBuffers &b, const KConst &k, uint32_t n, uint32_t features,
+                              bool uniform, float wu, uint32_t iter, uint32_t bs)
+{
+    if (features != F_FLUID)
+        solve_variant<true, false, NC>(st, b, k, n, wu, iter, bs);
+    else if (uniform)
+        solve_variant<false, true, NC>(st, b, k, n, wu, iter, bs);
+    else
+        solve_variant<false, false, NC>(st, b, k, n, wu, iter, bs);
 }
 
 hipError_t launch_solve(hipStream_t st, const DevBuffers &b, const KConst &k, uint32_t n,
                         uint32_t features, bool uniform, float wu, uint32_t iter, uint32_t bs)
 {
     if (n == 0) return hipSuccess;
-    // uniform-fluid scenes have no contacts, constraints or bodies
-    switch (features) {
-    case F_FLUID: solve_variant<F_FLUID>(st, b, k, n, uniform, wu, iter, bs); break;
-    case F_FLUID | F_PIN: solve_variant<F_FLUID | F_PIN>(st, b, k, n, false, wu, iter, bs); break;
-    default:
-        if (b.staging && !b.tape_f && b.split_solve) {
-            // Scenes where contact-walking particles are rare (ropes in a
-            // fluid): units without one run the variant without contacts
-            // (their particles take no contact branch, so the results are
-            // the same), which has no contact lists or staged phases in LDS,
-            // 49 KB against 78 KB, three blocks per CU instead of two.  The
-            // units with one run the full variant.  Each launch covers every
-            // unit and the other class's blocks leave at once, so where most
-            // units hold such a particle (cloth, rigid bodies) the split
-            // does not pay and is not made.  Timed as one: the event pair
-            // brackets both launches.
-            const LaunchEvents ev = g_launch_events;
-            g_launch_events = LaunchEvents{};
-            DevBuffers b1 = b, b2 = b;
-            b1.solve_units = 1u;
-            b2.solve_units = 2u;
-            g_launch_events = LaunchEvents{ev.start, nullptr};
-            solve_variant<F_FLUID | F_DIST | F_SHAPE | F_PIN>(st, b1, k, n, false, wu, iter, bs);
-            g_launch_events = LaunchEvents{nullptr, ev.stop};
-            solve_variant<F_FLUID | F_CONTACT | F_DIST | F_SHAPE | F_PIN>(st, b2, k, n, false, wu, iter, bs);
-            g_launch_events = LaunchEvents{};
-        } else {
-            solve_variant<F_FLUID | F_CONTACT | F_DIST | F_SHAPE | F_PIN>(st, b, k, n, false, wu, iter, bs);
-        }
-        break;
-    }
+    if (k.n_corr == 4u)
+        solve_composition<4>(st, b, k, n, features, uniform, wu, iter, bs);
+    else
+        solve_composition<0>(st, b, k, n, features, uniform, wu, iter, bs);
     return hipGetLastError();
 }
 
