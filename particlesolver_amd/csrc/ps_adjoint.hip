@@ -7,8 +7,8 @@
 // vector-Jacobian product is written out by hand below.  Every transposed
 // sum is a gather over the particle's own neighbour table, which holds the
 // same pairs as its neighbours' tables (r^2 < R^2 is symmetric and no table
-// overflowed), so there are no scatters and no atomics: one thread per
-// particle (or per distance constraint), sums in table order.  The
+// overflowed), so there are no scatters and no atomics: four or sixteen lanes
+// per particle, sums in table order.  The
 // arithmetic is the CPU oracle's, operation by operation (built with
 // -ffp-contract=off), so FP32 gradients match it bit for bit.
 //
@@ -115,10 +115,10 @@ __device__ __forceinline__ void yd_of(const KConst &k, const float4 &Y, float *y
 // owner that does not take part (op, oj false) enters with zeros.  cc and
 // c6 are the tensile term's and W's gradient factors (dW/dd = c6 d).  A
 // degenerate pair (G the constant (0, g0y, 0) for both owners) adds
-// (cc g0y (mu_p.y + mu_j.y) + cms c6) d.  Adds the terms to acc.
+// (cc g0y (mu_p.y + mu_j.y) + cms c6) d.  The sum goes to out.
 __device__ __forceinline__ void adj_pair_sum(const KConst &k, const float *dv, float r2, float lsum, bool op,
                                              bool oj, const float4 &mcp, const float4 &mcj, const float4 &kvp,
-                                             const float4 &kvj, float massp, float massj, float *acc)
+                                             const float4 &kvj, float massp, float massj, float *out)
 {
     const float t = k.h2 - r2;
     const float tt = t * t;
@@ -136,7 +136,7 @@ __device__ __forceinline__ void adj_pair_sum(const KConst &k, const float *dv, f
     if (r2 < kDegenerateR2) {
         const float g0y = -((k.spiky * (k.h * k.h)) * 0.001f);
         const float be = (cc * (g0y * (mup[1] + muj[1]))) + (cms * c6);
-        for (int a = 0; a < 3; a++) acc[a] = acc[a] + (be * dv[a]);
+        for (int a = 0; a < 3; a++) out[a] = be * dv[a];
         return;
     }
     const float ri = rsq(r2);
@@ -158,7 +158,7 @@ __device__ __forceinline__ void adj_pair_sum(const KConst &k, const float *dv, f
     const float vD = dot3(dv, dV);
     const float al = (C * us) - ((2.0f * Bq) * vD);
     const float be = (al - (K * mD)) + (cms * c6);
-    for (int a = 0; a < 3; a++) acc[a] = acc[a] + ((be * dv[a]) + ((A2 * dV[a]) - (cb * dmu[a])));
+    for (int a = 0; a < 3; a++) out[a] = (be * dv[a]) + ((A2 * dV[a]) - (cb * dmu[a]));
 }
 
 // density multiplier of a neighbour in rho_i
@@ -196,6 +196,62 @@ struct GXYA {
     float4 p, x, y;
     Attr a;
 };
+
+// ---------------------------------------------------------------------------
+// The gathers take 4 U lanes a particle: quarter h of its table is lanes U h
+// .. U h + U - 1, each forming the terms of one entry of a chunk at a time,
+// and all U add them in table order, so each holds the quarter's sum; then
+// (q0 + q2) + (q1 + q3) in every lane.  A term left out is -0, which changes
+// no sum it is added to.
+
+// s and the U lanes' terms v (then w), lane by lane
+template <uint32_t U, int S = 0>
+__device__ __forceinline__ float group_add(float s, float v)
+{
+    s = s + group_value<U, S>(v);
+    if constexpr (S + 1 < (int)U) s = group_add<U, S + 1>(s, v);
+    return s;
+}
+template <uint32_t U, int S = 0>
+__device__ __forceinline__ float group_add(float s, float v, float w)
+{
+    s = (s + group_value<U, S>(v)) + group_value<U, S>(w);
+    if constexpr (S + 1 < (int)U) s = group_add<U, S + 1>(s, v, w);
+    return s;
+}
+template <uint32_t U, int S = 0>
+__device__ __forceinline__ float group_add(float s, float v, float w, float x)
+{
+    s = ((s + group_value<U, S>(v)) + group_value<U, S>(w)) + group_value<U, S>(x);
+    if constexpr (S + 1 < (int)U) s = group_add<U, S + 1>(s, v, w, x);
+    return s;
+}
+template <uint32_t U, int S = 0>
+__device__ __forceinline__ float group_fma(float s, float v, float w)
+{
+    s = __builtin_fmaf(group_value<U, S>(v), group_value<U, S>(w), s);
+    if constexpr (S + 1 < (int)U) s = group_fma<U, S + 1>(s, v, w);
+    return s;
+}
+
+// The same over sixteen lanes, lane l adding its terms to the sum of those
+// before it (every lane's values fetched at once would take 96 registers).
+__device__ __forceinline__ float row_add(float s, float v, float w)
+{
+    s = (s + v) + w;
+#pragma unroll
+    for (int l = 1; l < 16; l++)
+        s = (__int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(s), 0x111, 0xf, 0xf, true)) + v) + w;
+    return group_value<16, 15>(s);
+}
+
+// the quarters' sums q0..q3 as (q0 + q2) + (q1 + q3)
+template <uint32_t U>
+__device__ __forceinline__ float quarters_sum(float s)
+{
+    s = s + __shfl_xor(s, 2 * U, 64);
+    return s + __shfl_xor(s, U, 64);
+}
 
 // ---------------------------------------------------------------------------
 // Pins, walls and wall friction backwards, and the fluid sum's rho0 term,
@@ -287,14 +343,13 @@ __device__ __forceinline__ void adj_pre_one(const DevBuffers &b, const KConst &k
 }
 
 // dL/dl -> dL/dC = -lb / (D + eps), dL/dD = -lb l / (D + eps); rho0 terms.
-// Four lanes per particle: lane hh sums lb over quarter hh of the table (its
-// chunks 4m + hh), then lb = (q0 + q2) + (q1 + q3), and lane 0 finishes.
-template <bool UNIFORM>
+// Lane 0 of a particle finishes.
+template <bool UNIFORM, uint32_t U>
 __global__ __launch_bounds__(kAdjBlock) void adj_lambda_k(DevBuffers b, KConst k, AdjBuffers a, uint32_t n)
 {
-    const uint32_t i = xcd_block() * (kAdjBlock / 4) + (threadIdx.x >> 2);
-    const uint32_t hh = threadIdx.x & 3u;
-    if (i >= n) return;  // the four lanes of a particle leave together
+    const uint32_t i = xcd_block() * (kAdjBlock / (4u * U)) + threadIdx.x / (4u * U);
+    const uint32_t lane = threadIdx.x % (4u * U);
+    if (i >= n) return;  // the lanes of a particle leave together
     // every per-particle load goes out before the first wait (lane 0's
     // finish would otherwise wait on three more after the sum)
     const float4 mi = a.M[i];
@@ -305,7 +360,7 @@ __global__ __launch_bounds__(kAdjBlock) void adj_lambda_k(DevBuffers b, KConst k
     const float rhoi = a.rho[i];
     float r = a.r0b[i];
     if (!UNIFORM && phi != PS_PHASE_FLUID) {
-        if (!hh) {
+        if (!lane) {
             a.MC[i] = make_float4(mi.x, mi.y, mi.z, 0.0f);
             a.KV[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
@@ -314,36 +369,37 @@ __global__ __launch_bounds__(kAdjBlock) void adj_lambda_k(DevBuffers b, KConst k
     const float mu[3] = {mi.x, mi.y, mi.z};
     const float ir0 = mi.w;
     float lb = 0.0f;
-    auto body = [&](const float4 &pj, const float4 &mj, float wj, int32_t phj) {
-        if (wj == 0.0f) return;
+    auto body = [&](const float4 &pj, const float4 &mj, float wj, int32_t phj, bool used) {
+        float own = -0.0f, other = -0.0f;
         const float dv[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
         const float r2 = dist2(dv[0], dv[1], dv[2]);
-        if (!(r2 < k.h2)) return;
-        float g[3];
-        adj_gamma(k, dv, r2, g);
-        lb = lb + dot3(mu, g);
-        if (phj == PS_PHASE_FLUID) {
-            // G(-d) = -G(d) exactly (rounding is symmetric); the degenerate
-            // direction is the same for both
-            const bool deg = r2 < kDegenerateR2;
-            const float gj[3] = {deg ? g[0] : -g[0], deg ? g[1] : -g[1], deg ? g[2] : -g[2]};
-            const float muj[3] = {mj.x, mj.y, mj.z};
-            lb = lb + dot3(muj, gj);
+        if (used && wj != 0.0f && r2 < k.h2) {
+            float g[3];
+            adj_gamma(k, dv, r2, g);
+            own = dot3(mu, g);
+            if (phj == PS_PHASE_FLUID) {
+                // G(-d) = -G(d) exactly (rounding is symmetric); the
+                // degenerate direction is the same for both
+                const bool deg = r2 < kDegenerateR2;
+                const float gj[3] = {deg ? g[0] : -g[0], deg ? g[1] : -g[1], deg ? g[2] : -g[2]};
+                const float muj[3] = {mj.x, mj.y, mj.z};
+                other = dot3(muj, gj);
+            }
         }
+        lb = group_add<U>(lb, own, other);
     };
+    constexpr uint32_t kFlight = U == 4 ? 2 : 4;
     if (UNIFORM) {
-        for_neighbors_strided_chunked(
-            b, i, c, hh, 4u, [&](uint32_t j) { return GLam{a.Pit[j], a.M[j]}; },
-            [&](uint32_t, const GLam &d) { body(d.p, d.m, 1.0f, PS_PHASE_FLUID); });
+        for_neighbors_quarter<U, kFlight>(
+            b, i, c, lane / U, lane % U, [&](uint32_t j) { return GLam{a.Pit[j], a.M[j]}; },
+            [&](const GLam &d, bool used) { body(d.p, d.m, 1.0f, PS_PHASE_FLUID, used); });
     } else {
-        for_neighbors_strided_chunked(
-            b, i, c, hh, 4u, [&](uint32_t j) { return GLamAttr{a.Pit[j], a.M[j], a.AB[j]}; },
-            [&](uint32_t, const GLamAttr &d) { body(d.p, d.m, d.a.w, d.a.phase); });
+        for_neighbors_quarter<U, kFlight>(
+            b, i, c, lane / U, lane % U, [&](uint32_t j) { return GLamAttr{a.Pit[j], a.M[j], a.AB[j]}; },
+            [&](const GLamAttr &d, bool used) { body(d.p, d.m, d.a.w, d.a.phase, used); });
     }
-    lb = lb + __shfl_xor(lb, 2, 64);  // lanes 0 and 1: q0 + q2, q1 + q3
-    const float lo = __shfl_xor(lb, 1, 64);
-    if (hh) return;
-    lb = lb + lo;
+    lb = quarters_sum<U>(lb);
+    if (lane) return;
     const float den = sd.w + k.relax;
     const float lam = pi.w;
     const float Cb = -(lb / den);
@@ -358,20 +414,50 @@ __global__ __launch_bounds__(kAdjBlock) void adj_lambda_k(DevBuffers b, KConst k
     a.KV[i] = make_float4(dk * sd.x, dk * sd.y, dk * sd.z, Db * (sk * sk));
 }
 
-// dL/dp before the iteration.  Four lanes per particle: lane hh sums the
-// pair and contact terms of quarter hh of the table (chunks hh, hh + 4, ...;
-// quarter 0 starts from dL/dy), then acc = (q0 + q2) + (q1 + q3), and lane 0
-// adds the distance constraints.
-template <bool UNIFORM>
-__global__ __launch_bounds__(kAdjBlock) void adj_position_k(DevBuffers b, KConst k, AdjBuffers a, uint32_t n)
+// dL/dp before the iteration: pair and contact terms (quarter 0 starts from
+// dL/dy), then the distance constraints, a lane each, 4 U at a time.
+template <bool UNIFORM, uint32_t U>
+__global__ __launch_bounds__(kAdjBlock, U == 4 ? 4 : 5) void adj_position_k(DevBuffers b, KConst k, AdjBuffers a, uint32_t n)
 {
-    const uint32_t p = xcd_block() * (kAdjBlock / 4) + (threadIdx.x >> 2);
-    const uint32_t hh = threadIdx.x & 3u;
-    if (p >= n) return;  // the four lanes of a particle leave together
+    const uint32_t p = xcd_block() * (kAdjBlock / (4u * U)) + threadIdx.x / (4u * U);
+    const uint32_t lane = threadIdx.x % (4u * U);
+    if (p >= n) return;  // the lanes of a particle leave together
     const float4 pp = a.Pit[p];
     const Attr ap = b.A[p];
     const float4 Yp = a.Y[p];
-    float acc[3] = {hh ? 0.0f : Yp.x, hh ? 0.0f : Yp.y, hh ? 0.0f : Yp.z};
+    // a constraint is a chain of loads (list, partner's slot, records); the
+    // lane's first kR go out together, ahead of the neighbours' where
+    // registers are not short (U = 4)
+    struct Link {
+        float4 l;
+        float3 p, y;
+        uint32_t occ;
+    };
+    uint32_t e0 = 0, e1 = 0;
+    constexpr uint32_t kLanes = 4u * U, kR = U == 1 ? 2 : 1;
+    Link ln[kR] = {};
+    if (a.dist) {
+        e0 = b.dist_off[ap.orig];
+        e1 = b.dist_off[ap.orig + 1];
+    }
+    auto links = [&](uint32_t base) {
+#pragma unroll
+        for (uint32_t r = 0; r < kR; r++) ln[r].l = b.links[min(base + kLanes * r + lane, e1 - 1u)];
+        uint32_t j[kR];
+#pragma unroll
+        for (uint32_t r = 0; r < kR; r++) {
+            j[r] = b.slot_of[__float_as_uint(ln[r].l.x)];
+            ln[r].occ = b.occ[__float_as_uint(ln[r].l.x)];
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < kR; r++) {
+            ln[r].p = reinterpret_cast<const float3 &>(a.Pit[j[r]]);
+            ln[r].y = reinterpret_cast<const float3 &>(a.Y[j[r]]);
+        }
+    };
+    if (U == 4 && e0 < e1) links(e0);
+    const bool q0 = lane < U;
+    float acc[3] = {q0 ? Yp.x : 0.0f, q0 ? Yp.y : 0.0f, q0 ? Yp.z : 0.0f};
     float ydp[3];
     yd_of(k, Yp, ydp);
     const bool pf = UNIFORM || ap.phase == PS_PHASE_FLUID;
@@ -381,138 +467,104 @@ __global__ __launch_bounds__(kAdjBlock) void adj_position_k(DevBuffers b, KConst
     const bool contacts = !UNIFORM && a.contacts;
     const float massp = adj_mass(k, ap.w, ap.phase);  // p as a neighbour of j
     auto body = [&](const float4 &pj, const float4 &mcj, const float4 &kvj, float wj, int32_t phj, uint32_t ncj,
-                    float massj) {
+                    float massj, bool used) {
         const float dv[3] = {pp.x - pj.x, pp.y - pj.y, pp.z - pj.z};
         const float r2 = dist2(dv[0], dv[1], dv[2]);
-        if (r2 < k.h2) {
-            // p owns the pair when fluid and j moves, j when fluid and p moves
-            const bool op = pf && wj != 0.0f;
-            const bool oj = (UNIFORM || phj == PS_PHASE_FLUID) && ap.w != 0.0f;
-            if (op || oj) adj_pair_sum(k, dv, r2, pp.w + pj.w, op, oj, mcp, mcj, kvp, kvj, massp, massj, acc);
-        }
-        if (contacts) {
-            // cloth contacts: p's own, then p as the partner of j's (for a
-            // non-fluid j, MC holds its masked dL/dy)
-            const float dj[3] = {-dv[0], -dv[1], -dv[2]};
-            float m[3];
-            if (adj_contact(k, ap.w, ap.phase, wj, phj, ncp, dv, ydp, m))
-                for (int q2 = 0; q2 < 3; q2++) acc[q2] = acc[q2] + m[q2];
-            const float ydj[3] = {mcj.x, mcj.y, mcj.z};
-            if (adj_contact(k, wj, phj, ap.w, ap.phase, ncj, dj, ydj, m))
-                for (int q2 = 0; q2 < 3; q2++) acc[q2] = acc[q2] - m[q2];
+        float m[3] = {-0.0f, -0.0f, -0.0f};
+        // p owns the pair when fluid and j moves, j when fluid and p moves
+        const bool op = pf && wj != 0.0f;
+        const bool oj = (UNIFORM || phj == PS_PHASE_FLUID) && ap.w != 0.0f;
+        if (used && r2 < k.h2 && (op || oj))
+            adj_pair_sum(k, dv, r2, pp.w + pj.w, op, oj, mcp, mcj, kvp, kvj, massp, massj, m);
+        // cloth contacts: p's own, then p as the partner of j's (for a
+        // non-fluid j, MC holds its masked dL/dy)
+        const float dj[3] = {-dv[0], -dv[1], -dv[2]};
+        const float ydj[3] = {mcj.x, mcj.y, mcj.z};
+        if constexpr (U == 1) {
+            for (int q2 = 0; q2 < 3; q2++) acc[q2] = acc[q2] + m[q2];
+            if (contacts) {
+                if (adj_contact(k, ap.w, ap.phase, wj, phj, ncp, dv, ydp, m))
+                    for (int q2 = 0; q2 < 3; q2++) acc[q2] = acc[q2] + m[q2];
+                if (adj_contact(k, wj, phj, ap.w, ap.phase, ncj, dj, ydj, m))
+                    for (int q2 = 0; q2 < 3; q2++) acc[q2] = acc[q2] - m[q2];
+            }
+        } else {
+            float mo[3] = {-0.0f, -0.0f, -0.0f}, mj[3] = {0.0f, 0.0f, 0.0f};
+            bool touch = false;
+            if (contacts && used) {
+                touch = adj_contact(k, ap.w, ap.phase, wj, phj, ncp, dv, ydp, mo);
+                touch = adj_contact(k, wj, phj, ap.w, ap.phase, ncj, dj, ydj, mj) || touch;
+            }
+            if (contacts && __any(touch))
+                for (int q2 = 0; q2 < 3; q2++) acc[q2] = group_add<U>(acc[q2], m[q2], mo[q2], -mj[q2]);
+            else
+                for (int q2 = 0; q2 < 3; q2++) acc[q2] = group_add<U>(acc[q2], m[q2]);
         }
     };
     const uint32_t c = b.ncnt[p];
-    // two records (48 or 64 bytes each) in flight per lane: four would hold
-    // the kernel to four wavefronts per SIMD
+    // two records (48 or 64 bytes each) in flight per lane: four would cost
+    // registers the waves need
+    constexpr uint32_t kFlight = 2;
     if (UNIFORM) {
-        for_neighbors_strided_pairs(
-            b, p, c, hh, 4u, [&](uint32_t j) { return GPos{a.Pit[j], a.MC[j], a.KV[j]}; },
-            [&](uint32_t, const GPos &d) { body(d.p, d.mc, d.kv, ap.w, PS_PHASE_FLUID, 0u, massp); });
+        for_neighbors_quarter<U, kFlight>(
+            b, p, c, lane / U, lane % U, [&](uint32_t j) { return GPos{a.Pit[j], a.MC[j], a.KV[j]}; },
+            [&](const GPos &d, bool used) { body(d.p, d.mc, d.kv, ap.w, PS_PHASE_FLUID, 0u, massp, used); });
     } else {
-        for_neighbors_strided_pairs(
-            b, p, c, hh, 4u, [&](uint32_t j) { return GPosAttr{a.Pit[j], a.MC[j], a.KV[j], a.AB[j]}; },
-            [&](uint32_t, const GPosAttr &d) { body(d.p, d.mc, d.kv, d.a.w, d.a.phase, d.a.nc, d.a.mass); });
+        for_neighbors_quarter<U, kFlight>(
+            b, p, c, lane / U, lane % U, [&](uint32_t j) { return GPosAttr{a.Pit[j], a.MC[j], a.KV[j], a.AB[j]}; },
+            [&](const GPosAttr &d, bool used) {
+                body(d.p, d.mc, d.kv, d.a.w, d.a.phase, d.a.nc, d.a.mass, used);
+            });
     }
-    {
-        // lanes 0 and 1 form q0 + q2 and q1 + q3, lane 0 their sum
-        for (int q2 = 0; q2 < 3; q2++) acc[q2] = acc[q2] + __shfl_xor(acc[q2], 2, 64);
-        float lo[3];
-        for (int q2 = 0; q2 < 3; q2++) lo[q2] = __shfl_xor(acc[q2], 1, 64);
-        for (int q2 = 0; q2 < 3; q2++) acc[q2] = acc[q2] + lo[q2];  // used in lane 0
-    }
+    for (int q2 = 0; q2 < 3; q2++) acc[q2] = quarters_sum<U>(acc[q2]);
     // distance constraints incident to p, in their order; for a constraint
     // whose first particle p is, also its dL/dstiffness (one writer per
     // constraint): T_a / st = -(w_a / (wsum occ_a)) (1 - L/r) d_ab, and T_b
-    // its mirror.  The particle's four lanes take four constraints at a
-    // time, kR such rounds at once: each constraint is a chain of dependent
-    // loads (index, pair, slot, records), and each level of the chain goes
-    // out for all kR rounds together.  Lane 0 adds the terms in constraint
-    // order.
-    if (a.dist) {
-        constexpr uint32_t kR = 3;
-        const uint32_t o = ap.orig;
-        const uint32_t e0 = b.dist_off[o], e1 = b.dist_off[o + 1];
-        const uint32_t quad = threadIdx.x & ~3u;
-        const float occo = (float)b.occ[o];
-        for (uint32_t base = e0; base < e1; base += 4u * kR) {  // the same trip count in the four lanes
-            uint32_t cid[kR], j[kR];
-            bool ok[kR];
-            uint2 pr[kR];
+    // its mirror.  Each lane forms one constraint's p term X and the negative
+    // of its j term, Z; all lanes add them in constraint order.
+    if (e0 < e1) {
+        if (U != 4) links(e0);
+        const float occo = (float)b.occ[ap.orig];
+        for (uint32_t base = e0;;) {  // the same trip count in the particle's lanes
 #pragma unroll
             for (uint32_t r = 0; r < kR; r++) {
-                const uint32_t e = base + 4u * r + hh;
-                ok[r] = e < e1;
-                cid[r] = b.dist_adj[ok[r] ? e : e0];
-            }
-#pragma unroll
-            for (uint32_t r = 0; r < kR; r++) pr[r] = b.dist_pairs[cid[r]];
-#pragma unroll
-            for (uint32_t r = 0; r < kR; r++) j[r] = b.slot_of[pr[r].x == o ? pr[r].y : pr[r].x];
-            float4 pj[kR], yj[kR];
-            float2 rs[kR];
-            Attr aj[kR];
-#pragma unroll
-            for (uint32_t r = 0; r < kR; r++) {
-                pj[r] = a.Pit[j[r]];
-                aj[r] = b.A[j[r]];
-                yj[r] = a.Y[j[r]];
-                rs[r] = b.dist_rs[cid[r]];
-            }
-            // each round's p term X and j term Z; fl bit 0: X is added,
-            // bit 1: Z is subtracted
-            float X[kR][3], Z[kR][3];
-            uint32_t fl[kR];
-#pragma unroll
-            for (uint32_t r = 0; r < kR; r++) {
-                fl[r] = 0;
-                for (int q2 = 0; q2 < 3; q2++) X[r][q2] = Z[r][q2] = 0.0f;
-                const float dv[3] = {pp.x - pj[r].x, pp.y - pj[r].y, pp.z - pj[r].z};
+                float X[3] = {-0.0f, -0.0f, -0.0f}, Z[3] = {-0.0f, -0.0f, -0.0f};
+                const uint32_t e = base + kLanes * r + lane;
+                const float wj = ln[r].l.w;
+                const float dv[3] = {pp.x - ln[r].p.x, pp.y - ln[r].p.y, pp.z - ln[r].p.z};
                 const float dist = sqrtf(((dv[0] * dv[0]) + (dv[1] * dv[1])) + (dv[2] * dv[2]));
-                const float wsum = ap.w + aj[r].w;
-                if (!ok[r] || dist < 1e-6f || wsum == 0.0f) continue;
-                const float L = rs[r].x, st = rs[r].y;
-                const float k1 = 1.0f - (L / dist), k2 = L / ((dist * dist) * dist);
-                const bool first = pr[r].x == o;  // d = p_a - p_b
-                float gs = 0.0f;
-                // M(d) = -(w st / (wsum occ)) [(1 - L/r) I + (L/r^3) d d^T]
-                if (ap.w != 0.0f) {
-                    const float cf = -(((ap.w * st) / wsum) / occo);
-                    const float dy = dot3(dv, ydp);
-                    for (int q2 = 0; q2 < 3; q2++) X[r][q2] = cf * ((k1 * ydp[q2]) + ((k2 * dy) * dv[q2]));
-                    fl[r] |= 1u;
-                    if (first) gs = gs - (((ap.w / wsum) / occo) * (k1 * dy));
-                }
-                if (aj[r].w != 0.0f) {
-                    float ydj[3];
-                    yd_of(k, yj[r], ydj);
-                    const float occj = (float)b.occ[aj[r].orig];
-                    const float cf = -(((aj[r].w * st) / wsum) / occj);
-                    const float dy = dot3(dv, ydj);
-                    for (int q2 = 0; q2 < 3; q2++) Z[r][q2] = cf * ((k1 * ydj[q2]) + ((k2 * dy) * dv[q2]));
-                    fl[r] |= 2u;
-                    if (first) gs = gs + (((aj[r].w / wsum) / occj) * (k1 * dy));
-                }
-                if (first) a.sb[cid[r]] = a.sb[cid[r]] + gs;
-            }
-#pragma unroll
-            for (uint32_t r = 0; r < kR; r++)
-                for (uint32_t l = 0; l < 4u; l++) {
-                    const int src = (int)(quad + l);
-                    const uint32_t fll = (uint32_t)__shfl((int)fl[r], src, 64);
-                    float Xl[3], Zl[3];
-                    for (int q2 = 0; q2 < 3; q2++) {
-                        Xl[q2] = __shfl(X[r][q2], src, 64);
-                        Zl[q2] = __shfl(Z[r][q2], src, 64);
+                const float wsum = ap.w + wj;
+                if (e < e1 && !(dist < 1e-6f || wsum == 0.0f)) {
+                    const float L = ln[r].l.y, st = ln[r].l.z;
+                    const float k1 = 1.0f - (L / dist), k2 = L / ((dist * dist) * dist);
+                    float gs = 0.0f;
+                    // M(d) = -(w st / (wsum occ)) [(1 - L/r) I + (L/r^3) d d^T]
+                    if (ap.w != 0.0f) {
+                        const float cf = -(((ap.w * st) / wsum) / occo);
+                        const float dy = dot3(dv, ydp);
+                        for (int q2 = 0; q2 < 3; q2++) X[q2] = cf * ((k1 * ydp[q2]) + ((k2 * dy) * dv[q2]));
+                        gs = gs - (((ap.w / wsum) / occo) * (k1 * dy));
                     }
-                    if (fll & 1u)
-                        for (int q2 = 0; q2 < 3; q2++) acc[q2] = acc[q2] + Xl[q2];
-                    if (fll & 2u)
-                        for (int q2 = 0; q2 < 3; q2++) acc[q2] = acc[q2] - Zl[q2];
+                    if (wj != 0.0f) {
+                        const float ydj[3] = {ln[r].y.x, ln[r].y.y, k.dims == 2u ? 0.0f : ln[r].y.z};
+                        const float cf = -(((wj * st) / wsum) / (float)ln[r].occ);
+                        const float dy = dot3(dv, ydj);
+                        for (int q2 = 0; q2 < 3; q2++) Z[q2] = -(cf * ((k1 * ydj[q2]) + ((k2 * dy) * dv[q2])));
+                        gs = gs + (((wj / wsum) / (float)ln[r].occ) * (k1 * dy));
+                    }
+                    // the first particle of the constraint (d = p_a - p_b)
+                    const uint32_t id = b.link_id[e];
+                    if (!(id & 1u)) a.sb[id >> 1] = a.sb[id >> 1] + gs;
                 }
+                for (int q2 = 0; q2 < 3; q2++)
+                    acc[q2] = U == 4 ? row_add(acc[q2], X[q2], Z[q2]) : group_add<kLanes>(acc[q2], X[q2], Z[q2]);
+            }
+            base += kLanes * kR;
+            if (base >= e1) break;
+            links(base);
         }
     }
-    if (hh) return;
+    if (lane) return;
     // the next iteration's pre-step (its records loaded here: held from the
     // start they would cost this kernel a wavefront per SIMD)
     if (a.clampn)
@@ -527,14 +579,13 @@ __global__ __launch_bounds__(kAdjBlock) void adj_position_k(DevBuffers b, KConst
 // dL/dS_i = (c/rho0_i) vbar_i / dt (in Y) and the rho0 term; adj_finalize_k
 // gathers dL/dp (the final iterate) and dL/dx*.
 
-template <bool UNIFORM>
+template <bool UNIFORM, uint32_t U>
 __global__ __launch_bounds__(kAdjBlock) void adj_xsph_k(DevBuffers b, KConst k, AdjBuffers a, uint32_t n,
                                                      float dt)
 {
-    // four lanes per particle: lane hh forms quarter hh of S, lane 0 finishes
-    const uint32_t i = xcd_block() * (kAdjBlock / 4) + (threadIdx.x >> 2);
-    const uint32_t hh = threadIdx.x & 3u;
-    if (i >= n) return;  // the four lanes of a particle leave together
+    const uint32_t i = xcd_block() * (kAdjBlock / (4u * U)) + threadIdx.x / (4u * U);
+    const uint32_t lane = threadIdx.x % (4u * U);  // lane 0 finishes
+    if (i >= n) return;  // the lanes of a particle leave together
     // the particle's own loads go out together
     const Attr ai = b.A[i];
     const float4 pi = b.P[i], xi = b.X[i];
@@ -548,52 +599,51 @@ __global__ __launch_bounds__(kAdjBlock) void adj_xsph_k(DevBuffers b, KConst k, 
         const float cr = k.xsph_c / ai.rho0;
         // S exactly as finalize_k forms it: four quarters of the table
         float Sm[3] = {0.0f, 0.0f, 0.0f};
-        auto body = [&](const float4 &pj, const float4 &xj, float wj) {
+        auto body = [&](const float4 &pj, const float4 &xj, float wj, bool used) {
             const float r2 = dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z);
-            if (!(r2 < k.h2)) return;
-            const float t = k.h2 - r2;
-            const float m = ((t * t) * t) * (1.0f / wj);
-            Sm[0] = __builtin_fmaf((pj.x - xj.x) - ui[0], m, Sm[0]);
-            Sm[1] = __builtin_fmaf((pj.y - xj.y) - ui[1], m, Sm[1]);
-            Sm[2] = __builtin_fmaf((pj.z - xj.z) - ui[2], m, Sm[2]);
+            float d[3] = {0.0f, 0.0f, 0.0f}, m = 0.0f;  // a sum that starts at +0 never is -0
+            if (used && r2 < k.h2) {
+                const float t = k.h2 - r2;
+                m = ((t * t) * t) * (1.0f / wj);
+                d[0] = (pj.x - xj.x) - ui[0];
+                d[1] = (pj.y - xj.y) - ui[1];
+                d[2] = (pj.z - xj.z) - ui[2];
+            }
+            for (int q = 0; q < 3; q++) Sm[q] = group_fma<U>(Sm[q], d[q], m);
         };
+        constexpr uint32_t kFlight = U == 4 ? 2 : 4;
         if (UNIFORM) {
-            for_neighbors_strided_chunked(
-                b, i, c, hh, 4u, [&](uint32_t j) { return PX{b.P[j], b.X[j]}; },
-                [&](uint32_t, const PX &d) { body(d.p, d.x, ai.w); });
+            for_neighbors_quarter<U, kFlight>(
+                b, i, c, lane / U, lane % U, [&](uint32_t j) { return PX{b.P[j], b.X[j]}; },
+                [&](const PX &d, bool used) { body(d.p, d.x, ai.w, used); });
         } else {
-            for_neighbors_strided_chunked(
-                b, i, c, hh, 4u, [&](uint32_t j) { return GXA{b.P[j], b.X[j], b.A[j]}; },
-                [&](uint32_t, const GXA &d) {
-                    if (d.a.phase == PS_PHASE_FLUID) body(d.p, d.x, d.a.w);
+            for_neighbors_quarter<U, kFlight>(
+                b, i, c, lane / U, lane % U, [&](uint32_t j) { return GXA{b.P[j], b.X[j], b.A[j]}; },
+                [&](const GXA &d, bool used) {
+                    body(d.p, d.x, d.a.w, used && d.a.phase == PS_PHASE_FLUID);
                 });
         }
-        // (q0 + q2) + (q1 + q3)
-        for (int q = 0; q < 3; q++) Sm[q] = Sm[q] + __shfl_xor(Sm[q], 2, 64);
-        float lo[3];
-        for (int q = 0; q < 3; q++) lo[q] = __shfl_xor(Sm[q], 1, 64);
-        if (hh) return;
-        const float S[3] = {k.poly6 * (Sm[0] + lo[0]), k.poly6 * (Sm[1] + lo[1]), k.poly6 * (Sm[2] + lo[2])};
+        for (int q = 0; q < 3; q++) Sm[q] = quarters_sum<U>(Sm[q]);
+        if (lane) return;
+        const float S[3] = {k.poly6 * Sm[0], k.poly6 * Sm[1], k.poly6 * Sm[2]};
         const float vS = dot3(vbn, S);
         r0 = r0 - (((k.xsph_c / (ai.rho0 * ai.rho0)) * vS) / dt);
         for (int q = 0; q < 3; q++) Sh[q] = (vbn[q] * cr) / dt;
     }
-    if (hh) return;
+    if (lane) return;
     a.r0b[i] = r0;
     a.wkb[i] = 0.0f;
     a.Y[i] = make_float4(Sh[0], Sh[1], Sh[2], 0.0f);
 }
 
-// Four lanes per particle: lane hh sums the pair terms of quarter hh of the
-// table (quarter 0 starts from dL/dx and dL/dv / dt), then
-// (q0 + q2) + (q1 + q3).
-template <bool UNIFORM>
+// Quarter 0 starts from dL/dx and dL/dv / dt.
+template <bool UNIFORM, uint32_t U>
 __global__ __launch_bounds__(kAdjBlock) void adj_finalize_k(DevBuffers b, KConst k, AdjBuffers a, uint32_t n,
                                                          float dt)
 {
-    const uint32_t p = xcd_block() * (kAdjBlock / 4) + (threadIdx.x >> 2);
-    const uint32_t hh = threadIdx.x & 3u;
-    if (p >= n) return;  // the four lanes of a particle leave together
+    const uint32_t p = xcd_block() * (kAdjBlock / (4u * U)) + threadIdx.x / (4u * U);
+    const uint32_t lane = threadIdx.x % (4u * U);
+    if (p >= n) return;  // the lanes of a particle leave together
     // the particle's own loads go out together (and the last iteration's
     // pre-step records)
     const Attr ap = b.A[p];
@@ -601,64 +651,65 @@ __global__ __launch_bounds__(kAdjBlock) void adj_finalize_k(DevBuffers b, KConst
     const float4 shp4 = a.Y[p];
     const uint32_t c = b.ncnt[p];
     AdjPreIn pre{};
-    if (a.clampn && hh == 0) pre = adj_pre_load(a, p);
+    if (a.clampn && lane == 0) pre = adj_pre_load(a, p);
     const float4 vb = a.gv[ap.orig], xb = a.gx[ap.orig];
     float ub[3] = {vb.x / dt, vb.y / dt, vb.z / dt};
     float acc[3] = {xb.x, xb.y, xb.z};
-    if (hh)
+    if (lane >= U)
         for (int q = 0; q < 3; q++) ub[q] = acc[q] = 0.0f;
     if (k.xsph_c != 0.0f && (UNIFORM || ap.phase == PS_PHASE_FLUID)) {
         const float up[3] = {pp.x - xp.x, pp.y - xp.y, pp.z - xp.z};
         const float Shp[3] = {shp4.x, shp4.y, shp4.z};
         const float mp = 1.0f / ap.w;
-        auto body = [&](const float4 &pj, const float4 &xj, const float4 &shj4, float wj) {
+        auto body = [&](const float4 &pj, const float4 &xj, const float4 &shj4, float wj, bool used) {
             const float dv[3] = {pp.x - pj.x, pp.y - pj.y, pp.z - pj.z};
             const float r2 = dist2(dv[0], dv[1], dv[2]);
-            if (!(r2 < k.h2)) return;
-            const float t = k.h2 - r2;
-            const float W = k.poly6 * ((t * t) * t);
-            float g6[3];
-            adj_grad_w6(k, dv, r2, g6);
-            const float uj[3] = {pj.x - xj.x, pj.y - xj.y, pj.z - xj.z};
-            const float Shj[3] = {shj4.x, shj4.y, shj4.z};
-            // p as owner: S_p += (u_j - u_p) m_j W; p as neighbour of j
-            const float mj = 1.0f / wj;
-            const float wb = mj * ((((uj[0] - up[0]) * Shp[0]) + ((uj[1] - up[1]) * Shp[1])) +
-                                   ((uj[2] - up[2]) * Shp[2]));
-            const float wb2 = mp * ((((up[0] - uj[0]) * Shj[0]) + ((up[1] - uj[1]) * Shj[1])) +
-                                    ((up[2] - uj[2]) * Shj[2]));
+            // u gains us, then ua, the gradient g1, then g2
+            float us[3] = {-0.0f, -0.0f, -0.0f}, ua[3] = {-0.0f, -0.0f, -0.0f};
+            float g1[3] = {-0.0f, -0.0f, -0.0f}, g2[3] = {-0.0f, -0.0f, -0.0f};
+            if (used && r2 < k.h2) {
+                const float t = k.h2 - r2;
+                const float W = k.poly6 * ((t * t) * t);
+                float g6[3];
+                adj_grad_w6(k, dv, r2, g6);
+                const float uj[3] = {pj.x - xj.x, pj.y - xj.y, pj.z - xj.z};
+                const float Shj[3] = {shj4.x, shj4.y, shj4.z};
+                // p as owner: S_p += (u_j - u_p) m_j W; p as neighbour of j
+                const float mj = 1.0f / wj;
+                const float wb = mj * ((((uj[0] - up[0]) * Shp[0]) + ((uj[1] - up[1]) * Shp[1])) +
+                                       ((uj[2] - up[2]) * Shp[2]));
+                const float wb2 = mp * ((((up[0] - uj[0]) * Shj[0]) + ((up[1] - uj[1]) * Shj[1])) +
+                                        ((up[2] - uj[2]) * Shj[2]));
+                for (int q2 = 0; q2 < 3; q2++) {
+                    us[q2] = -((mj * W) * Shp[q2]);
+                    ua[q2] = (mp * W) * Shj[q2];
+                    g1[q2] = wb * g6[q2];
+                    g2[q2] = wb2 * g6[q2];
+                }
+            }
             for (int q2 = 0; q2 < 3; q2++) {
-                ub[q2] = (ub[q2] - ((mj * W) * Shp[q2])) + ((mp * W) * Shj[q2]);
-                acc[q2] = (acc[q2] + (wb * g6[q2])) + (wb2 * g6[q2]);
+                ub[q2] = group_add<U>(ub[q2], us[q2], ua[q2]);
+                acc[q2] = group_add<U>(acc[q2], g1[q2], g2[q2]);
             }
         };
+        constexpr uint32_t kFlight = U == 4 ? 2 : 4;
         if (UNIFORM) {
-            for_neighbors_strided_chunked(
-                b, p, c, hh, 4u, [&](uint32_t j) { return GXY{b.P[j], b.X[j], a.Y[j]}; },
-                [&](uint32_t, const GXY &d) { body(d.p, d.x, d.y, ap.w); });
+            for_neighbors_quarter<U, kFlight>(
+                b, p, c, lane / U, lane % U, [&](uint32_t j) { return GXY{b.P[j], b.X[j], a.Y[j]}; },
+                [&](const GXY &d, bool used) { body(d.p, d.x, d.y, ap.w, used); });
         } else {
-            for_neighbors_strided_chunked(
-                b, p, c, hh, 4u, [&](uint32_t j) { return GXYA{b.P[j], b.X[j], a.Y[j], b.A[j]}; },
-                [&](uint32_t, const GXYA &d) {
-                    if (d.a.phase == PS_PHASE_FLUID) body(d.p, d.x, d.y, d.a.w);
+            for_neighbors_quarter<U, kFlight>(
+                b, p, c, lane / U, lane % U, [&](uint32_t j) { return GXYA{b.P[j], b.X[j], a.Y[j], b.A[j]}; },
+                [&](const GXYA &d, bool used) {
+                    body(d.p, d.x, d.y, d.a.w, used && d.a.phase == PS_PHASE_FLUID);
                 });
         }
     }
-    // lanes 0 and 1 form q0 + q2 and q1 + q3, lane 0 their sum
     for (int q = 0; q < 3; q++) {
-        ub[q] = ub[q] + __shfl_xor(ub[q], 2, 64);
-        acc[q] = acc[q] + __shfl_xor(acc[q], 2, 64);
+        ub[q] = quarters_sum<U>(ub[q]);
+        acc[q] = quarters_sum<U>(acc[q]);
     }
-    float lu[3], la[3];
-    for (int q = 0; q < 3; q++) {
-        lu[q] = __shfl_xor(ub[q], 1, 64);
-        la[q] = __shfl_xor(acc[q], 1, 64);
-    }
-    if (hh) return;
-    for (int q = 0; q < 3; q++) {
-        ub[q] = ub[q] + lu[q];
-        acc[q] = acc[q] + la[q];
-    }
+    if (lane) return;
     a.xsb[p] = make_float4(-ub[0], -ub[1], -ub[2], 0.0f);
     float g[3] = {acc[0] + ub[0], acc[1] + ub[1], acc[2] + ub[2]};
     if (a.clampn)
@@ -690,29 +741,46 @@ __global__ __launch_bounds__(kAdjBlock) void adj_predict_k(DevBuffers b, KConst 
 
 static inline uint32_t adj_blocks(uint32_t n) { return (n + kAdjBlock - 1) / kAdjBlock; }
 
+// Lanes a quarter: four while the particles are too few to fill the chip with
+// one (65,536 of them make four wavefronts a SIMD), one from there on, where
+// the four lanes' repeated sums and the 4 times as many wavefronts' own
+// records cost more than the shorter chains give.  adj_position_k, then
+// adj_lambda_k, with one lane and with four, in us: 5k particles 20.8 / 10.9,
+// 6.8 / 4.4; 12k 16.3 / 9.2, 6.6 / 5.0; 32k 18.4 / 15.3, 8.5 / 7.6; 50k 23.3 /
+// 21.7, 12.3 / 10.3; 82k 39.6 / 44.1, 15.5 / 15.6; 328k 81 / 126, 48 / 51.
+static constexpr uint32_t kAdjSpread = 65536;
+
 hipError_t launch_adj(hipStream_t st, AdjKernel which, const DevBuffers &b, const KConst &k,
                       const AdjBuffers &a, uint32_t count, float dt, bool uniform)
 {
     if (count == 0) return hipSuccess;
     const dim3 grid(adj_blocks(count)), block(kAdjBlock);
-    // four lanes per particle: kAdjBlock / 4 particles per block
-    const dim3 grid4((count + kAdjBlock / 4 - 1) / (kAdjBlock / 4));
-#define PS_ADJ_LAUNCH4(kern, ...)                                                                 \
+    // 4 U lanes per particle
+#define PS_ADJ_LAUNCH_U(kern, U, ...)                                                              \
     do {                                                                                           \
+        const dim3 g((count + kAdjBlock / (4 * U) - 1) / (kAdjBlock / (4 * U)));                   \
         if (uniform)                                                                               \
-            PS_LAUNCH(kern<true>, grid4, block, 0, st, __VA_ARGS__);                      \
+            PS_LAUNCH((kern<true, U>), g, block, 0, st, __VA_ARGS__);                              \
         else                                                                                       \
-            PS_LAUNCH(kern<false>, grid4, block, 0, st, __VA_ARGS__);                     \
+            PS_LAUNCH((kern<false, U>), g, block, 0, st, __VA_ARGS__);                             \
+    } while (0)
+#define PS_ADJ_LAUNCH(kern, ...)                                                                   \
+    do {                                                                                           \
+        if (count <= kAdjSpread)                                                                   \
+            PS_ADJ_LAUNCH_U(kern, 4, __VA_ARGS__);                                                 \
+        else                                                                                       \
+            PS_ADJ_LAUNCH_U(kern, 1, __VA_ARGS__);                                                 \
     } while (0)
     switch (which) {
-    case ADJ_XSPH: PS_ADJ_LAUNCH4(adj_xsph_k, b, k, a, count, dt); break;
-    case ADJ_FINALIZE: PS_ADJ_LAUNCH4(adj_finalize_k, b, k, a, count, dt); break;
-    case ADJ_LAMBDA: PS_ADJ_LAUNCH4(adj_lambda_k, b, k, a, count); break;
-    case ADJ_POSITION: PS_ADJ_LAUNCH4(adj_position_k, b, k, a, count); break;
+    case ADJ_XSPH: PS_ADJ_LAUNCH(adj_xsph_k, b, k, a, count, dt); break;
+    case ADJ_FINALIZE: PS_ADJ_LAUNCH(adj_finalize_k, b, k, a, count, dt); break;
+    case ADJ_LAMBDA: PS_ADJ_LAUNCH(adj_lambda_k, b, k, a, count); break;
+    case ADJ_POSITION: PS_ADJ_LAUNCH(adj_position_k, b, k, a, count); break;
     case ADJ_PREDICT: PS_LAUNCH(adj_predict_k, grid, block, 0, st, b, k, a, count, dt); break;
     default: return hipErrorInvalidValue;
     }
-#undef PS_ADJ_LAUNCH4
+#undef PS_ADJ_LAUNCH
+#undef PS_ADJ_LAUNCH_U
     return hipGetLastError();
 }
 

@@ -409,7 +409,7 @@ void free_all(ps_system *s)
     dev_free(b.A); dev_free(b.A2); dev_free(b.key); dev_free(b.key2); dev_free(b.rank);
     dev_free(b.tmp_orig); dev_free(b.slot_of); dev_free(b.mj); dev_free(b.phs); dev_free(b.cell_count); dev_free(b.cell_off);
     dev_free(b.scan_part); dev_free(b.nbr); dev_free(b.ncnt); dev_free(b.dist_off);
-    dev_free(b.dist_adj); dev_free(b.dist_pairs); dev_free(b.dist_rs); dev_free(b.occ);
+    dev_free(b.link_id); dev_free(b.occ);
     dev_free(b.pin_of); dev_free(b.pin_xyz); dev_free(b.body_off); dev_free(b.body_idx);
     dev_free(b.body_rest); dev_free(b.body_stiff); dev_free(b.body_mass); dev_free(b.body_q);
     dev_free(b.body_goal); dev_free(b.body_of); dev_free(b.member_of); dev_free(b.status);
@@ -419,7 +419,7 @@ void free_all(ps_system *s)
     dev_free(b.stage);
     dev_free(b.omark); dev_free(b.smark); dev_free(b.walk_rank); dev_free(b.link_rank);
     dev_free(b.walk_slot); dev_free(b.link_slot);
-    dev_free(b.link_off); dev_free(b.links); dev_free(b.link_own); dev_free(b.con_c); dev_free(b.con_d);
+    dev_free(b.link_ends); dev_free(b.links); dev_free(b.link_own); dev_free(b.con_c); dev_free(b.con_d);
     for (ps_system::Emitter &e : s->emitters) dev_free(e.mark);
     adj_free(s);
 }
@@ -806,7 +806,7 @@ int con_reserve(ps_system *s)
     int rc;
     for (uint32_t **p : {&b.walk_rank, &b.link_rank, &b.walk_slot, &b.link_slot})
         if (!*p && (rc = dev_alloc(s, p, s->cap))) return rc;
-    if (!b.link_off && (rc = dev_alloc(s, &b.link_off, (size_t)s->cap + 1))) return rc;
+    if (!b.link_ends && (rc = dev_alloc(s, &b.link_ends, s->cap))) return rc;
     if (!b.link_own && (rc = dev_alloc(s, &b.link_own, s->cap))) return rc;
     if (!b.con_c && (rc = dev_alloc(s, &b.con_c, s->cap))) return rc;
     if (!b.con_d && (rc = dev_alloc(s, &b.con_d, s->cap))) return rc;
@@ -848,35 +848,32 @@ int upload_constraints(ps_system *s, size_t c0)
     const size_t m = s->dist_rest.size();
     if (m > s->dist_cap) {
         size_t nc = m * 2;
-        dev_free(b.dist_adj);
-        dev_free(b.dist_pairs);
-        dev_free(b.dist_rs);
+        dev_free(b.link_id);
         dev_free(b.links);
         s->dist_cap = b.nlink = 0;
         int rc;
-        if ((rc = dev_alloc(s, &b.dist_adj, 2 * nc))) return rc;
-        if ((rc = dev_alloc(s, &b.dist_pairs, nc))) return rc;
-        if ((rc = dev_alloc(s, &b.dist_rs, nc))) return rc;
+        if ((rc = dev_alloc(s, &b.link_id, 2 * nc))) return rc;
         if ((rc = dev_alloc(s, &b.links, 2 * nc))) return rc;
         s->dist_cap = nc;
     }
-    std::vector<uint32_t> off(s->cap + 1, 0), adj(2 * m), fill(s->cap, 0);
-    for (size_t c = 0; c < m; c++) {
-        off[s->dist_pairs[2 * c] + 1]++;
-        off[s->dist_pairs[2 * c + 1] + 1]++;
-    }
+    // each particle's links, in constraint order
+    std::vector<uint32_t> off(s->cap + 1, 0), id(2 * m);
+    std::vector<float4> links(2 * m);
+    for (uint32_t o : s->dist_pairs) off[o + 1]++;
     for (uint32_t i = 0; i < s->cap; i++) off[i + 1] += off[i];
-    for (size_t c = 0; c < m; c++) {
-        uint32_t a = s->dist_pairs[2 * c], bb = s->dist_pairs[2 * c + 1];
-        adj[off[a] + fill[a]++] = (uint32_t)c;
-        adj[off[bb] + fill[bb]++] = (uint32_t)c;
+    // filled from the last constraint on: off[o + 1] counts down to where
+    // particle o's begin, and is moved to its place after
+    for (size_t e = 2 * m; e-- > 0;) {
+        const uint32_t c = (uint32_t)(e / 2), o = s->dist_pairs[e], other = s->dist_pairs[e ^ 1];
+        const uint32_t q = --off[o + 1];
+        float bits;
+        memcpy(&bits, &other, sizeof(bits));
+        id[q] = (uint32_t)e;
+        links[q] = make_float4(bits, s->dist_rest[c], s->dist_stiff[c], s->inv_mass[other]);
     }
-    std::vector<float> rs(2 * m);
-    for (size_t c = 0; c < m; c++) {
-        rs[2 * c] = s->dist_rest[c];
-        rs[2 * c + 1] = s->dist_stiff[c];
-    }
-    // the constraint blocks' copy: each linked particle's links in constraint order
+    off.erase(off.begin());
+    off.push_back((uint32_t)(2 * m));
+    // the constraint blocks' list of the particles that links move
     Touched touched;
     for (size_t e = 2 * c0; e < 2 * m; e++) {
         const uint32_t o = s->dist_pairs[e];
@@ -886,35 +883,21 @@ int upload_constraints(ps_system *s, size_t c0)
         s->link_rank[o] = (uint32_t)s->linked.size();
         s->linked.push_back(o);
     }
-    std::vector<uint32_t> link_off(1, 0);
-    std::vector<float4> links;
-    links.reserve(2 * m);
-    for (uint32_t o : s->linked) {
-        for (uint32_t q = off[o]; q < off[o + 1]; q++) {
-            const uint32_t c = adj[q], first = s->dist_pairs[2 * c];
-            const uint32_t other = first == o ? s->dist_pairs[2 * c + 1] : first;
-            float bits;
-            memcpy(&bits, &other, sizeof(bits));
-            links.push_back(make_float4(bits, s->dist_rest[c], s->dist_stiff[c], s->inv_mass[other]));
-        }
-        link_off.push_back((uint32_t)links.size());
-    }
+    std::vector<uint2> ends;
+    ends.reserve(s->linked.size());
+    for (uint32_t o : s->linked) ends.push_back(make_uint2(off[o], off[o + 1]));
     HIP_TRY(s, hipMemcpy(b.dist_off, off.data(), sizeof(uint32_t) * off.size(), hipMemcpyHostToDevice));
     HIP_TRY(s, touched.upload(b.occ, s->occ));
     HIP_TRY(s, touched.upload(b.omark, s->mark));
     HIP_TRY(s, touched.upload(b.link_rank, s->link_rank));
     if (int rc = upload_link_own(s)) return rc;
-    if (!s->linked.empty()) {
-        HIP_TRY(s, hipMemcpy(b.link_off, link_off.data(), sizeof(uint32_t) * link_off.size(), hipMemcpyHostToDevice));
+    if (!ends.empty())
+        HIP_TRY(s, hipMemcpy(b.link_ends, ends.data(), sizeof(uint2) * ends.size(), hipMemcpyHostToDevice));
+    if (m) {
+        HIP_TRY(s, hipMemcpy(b.link_id, id.data(), sizeof(uint32_t) * id.size(), hipMemcpyHostToDevice));
         HIP_TRY(s, hipMemcpy(b.links, links.data(), sizeof(float4) * links.size(), hipMemcpyHostToDevice));
     }
-    b.nlink = (uint32_t)s->linked.size();
-    if (m) {
-        HIP_TRY(s, hipMemcpy(b.dist_adj, adj.data(), sizeof(uint32_t) * adj.size(), hipMemcpyHostToDevice));
-        HIP_TRY(s, hipMemcpy(b.dist_pairs, s->dist_pairs.data(), sizeof(uint32_t) * 2 * m,
-                             hipMemcpyHostToDevice));
-        HIP_TRY(s, hipMemcpy(b.dist_rs, rs.data(), sizeof(float) * 2 * m, hipMemcpyHostToDevice));
-    }
+    b.nlink = (uint32_t)ends.size();
     return PS_OK;
 }
 

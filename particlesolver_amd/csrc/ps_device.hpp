@@ -279,35 +279,63 @@ __device__ __forceinline__ void for_neighbors_strided_chunked(const DevBuffers &
     }
 }
 
-// As for_neighbors_strided_chunked with two records in flight instead of
-// four: the gathers of a chunk's entries 2 and 3 go out once entries 0 and
-// 1 are done.  For records so large (tens of bytes) that four of them in
-// registers would cost a wavefront per SIMD.
-template <typename G, typename Fn>
-__device__ __forceinline__ void for_neighbors_strided_pairs(const DevBuffers &b, uint32_t i, uint32_t c,
-                                                            uint32_t first, uint32_t stride, G gather,
-                                                            Fn fn)
+// The value of lane S of each four, and of lane L of each sixteen.  (Every
+// lane read from must be active.)
+template <int S>
+__device__ __forceinline__ uint32_t quad_value(uint32_t v)
 {
-    const uint32_t nch = (c + 3u) >> 2;  // chunks in use
-    if (first >= nch) return;
-    const uint4 *nb = nbr_lane(b, i);
-    uint4 jj = nb[(size_t)first * 64];
-    for (uint32_t m = first; m < nch; m += stride) {
-        const uint4 jn = nb[(size_t)(m + stride < nch ? m + stride : m) * 64];
-        const uint32_t q = m << 2;
-        {
-            const auto d0 = gather(jj.x);
-            const auto d1 = gather(jj.y);
-            fn(jj.x, d0);
-            if (q + 1 < c) fn(jj.y, d1);
-        }
-        if (q + 2 < c) {
-            const auto d2 = gather(jj.z);
-            const auto d3 = gather(jj.w);
-            fn(jj.z, d2);
-            if (q + 3 < c) fn(jj.w, d3);
-        }
-        jj = jn;
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, S * 0x55, 0xf, 0xf, true);
+}
+template <int S>
+__device__ __forceinline__ float quad_value(float v)
+{
+    return __uint_as_float(quad_value<S>(__float_as_uint(v)));
+}
+
+// The value of lane S of each U lanes (U = 1, 4 or 16).
+template <uint32_t U, int S>
+__device__ __forceinline__ float group_value(float v)
+{
+    if constexpr (U == 1)
+        return v;
+    else if constexpr (U == 4)
+        return quad_value<S>(v);
+    else
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + S, 0xf, 0xf, true));
+}
+
+// Quarter h of particle i's first c neighbours (its chunks h, h + 4, ...) by
+// U lanes (1 or 4): fn(record, in use) for entry U s + u of a chunk in
+// lane u, s = 0, 1, ..., with D records in flight and the entries after them.
+// An entry past the table's end reads particle i's record and is not in use.
+// The U lanes make the same calls.  (One lane loading a chunk's four entries
+// with one 16-byte load was slower: the reverse kernels took 52, 62 and 70 us
+// instead of 48, 54 and 66 at 328k particles.)
+template <uint32_t U, uint32_t D, typename G, typename Fn>
+__device__ __forceinline__ void for_neighbors_quarter(const DevBuffers &b, uint32_t i, uint32_t c, uint32_t h,
+                                                      uint32_t u, G gather, Fn fn)
+{
+    if (4u * h >= c) return;
+    const uint32_t *nb = reinterpret_cast<const uint32_t *>(nbr_lane(b, i));
+    constexpr uint32_t kS = 4u / U;  // steps a chunk
+    // where step t begins in the table
+    auto begin = [&](uint32_t t) { return 4u * (h + 4u * (t / kS)) + U * (t % kS); };
+    auto entry = [&](uint32_t t) {
+        const uint32_t q = begin(t) + u;
+        return q < c ? nb[(size_t)(q >> 2) * 256 + (q & 3u)] : i;
+    };
+    uint32_t j[D];
+#pragma unroll
+    for (uint32_t e = 0; e < D; e++) j[e] = entry(e);
+    for (uint32_t t = 0; begin(t) < c; t += D) {
+        decltype(gather(0u)) d[D];
+#pragma unroll
+        for (uint32_t e = 0; e < D; e++) d[e] = gather(j[e]);
+#pragma unroll
+        for (uint32_t e = 0; e < D; e++) j[e] = entry(t + D + e);
+#pragma unroll
+        for (uint32_t e = 0; e < D; e++)
+            if (begin(t + e) < c) fn(d[e], begin(t + e) + u < c);
     }
 }
 

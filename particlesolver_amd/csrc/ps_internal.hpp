@@ -155,7 +155,8 @@ struct DevBuffers {
     // links (partner index, rest, stiffness, the partner's w) and their own w
     // and incidence count; and per slot of one of them its corrections of the
     // iteration
-    uint32_t *walk_rank, *link_rank, *walk_slot, *link_slot, *link_off;
+    uint32_t *walk_rank, *link_rank, *walk_slot, *link_slot;
+    uint2 *link_ends;
     float4 *links;
     float2 *link_own;
     float4 *con_c, *con_d;
@@ -174,9 +175,7 @@ struct DevBuffers {
     uint32_t kq;  // max_neighbors / 4
     // distance constraints (insertion-index CSR)
     uint32_t *dist_off;    // max_particles + 1
-    uint32_t *dist_adj;    // 2*m: constraint ids
-    uint2 *dist_pairs;     // m
-    float2 *dist_rs;       // m: (rest, stiffness)
+    uint32_t *link_id;     // 2*m: 2 * constraint + (1 for its second particle)
     uint32_t *occ;         // per particle incidence count (distance + pins)
     // pins
     uint32_t *pin_of;      // per particle: pin + 1 (0 = none)

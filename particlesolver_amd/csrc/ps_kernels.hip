@@ -1201,18 +1201,6 @@ __device__ __forceinline__ void shape_body(const DevBuffers &b, uint32_t bd)
 // ensemble of 2.6M with 128 ropes 118 + 187 (solve), 121 + 142; 7k mixed
 // 5.2 + 9.1 + 12.5, 11.3 + 6.9; cloth over a pool, 82k, 10 + 24, 12 + 11.
 
-// the value of lane S of each four
-template <int S>
-__device__ __forceinline__ uint32_t quad_value(uint32_t v)
-{
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, S * 0x55, 0xf, 0xf, false);
-}
-template <int S>
-__device__ __forceinline__ float quad_value(float v)
-{
-    return __uint_as_float(quad_value<S>(__float_as_uint(v)));
-}
-
 // a7: particle contacts + friction (collideD, integration_kernel.cuh:358-462).
 // The corrections are summed in the two halves of the table, each in table
 // order, then added half 0 + half 1 (the oracle's order).  Eight lanes a
@@ -1394,7 +1382,8 @@ __device__ __forceinline__ void constrain_contacts(const DevBuffers &b, const KC
 __device__ __forceinline__ void constrain_links(const DevBuffers &b, uint32_t q, uint32_t g)
 {
     const uint32_t i = b.link_slot[q];
-    const uint32_t a0 = b.link_off[q], a1 = b.link_off[q + 1];
+    const uint2 ends = b.link_ends[q];
+    const uint32_t a0 = ends.x, a1 = ends.y;
     const float2 own = b.link_own[q];  // its inverse mass and incidence count
     const float wi = own.x;
     const float4 p = b.P[i];
