@@ -177,7 +177,7 @@ hipError_t grid_run(hipStream_t st, const GridK &g, uint32_t cells, uint32_t n, 
     hipLaunchKernelGGL(grid_fill_k, dim3(grid_blocks(cells)), t, 0, st, w.cnt, cells, 0u);
     if (n > 0) hipLaunchKernelGGL(grid_hash_k, dim3(grid_blocks(n)), t, 0, st, pos, n, g, w.key, w.rank, w.cnt);
     // the scan kernels of the grid build read cell_count / scan_part and
-    // write cell_off (and clear the counts again)
+    // write cell_off
     DevBuffers view{};
     view.cell_count = w.cnt;
     view.cell_off = w.off;

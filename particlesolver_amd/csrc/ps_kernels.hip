@@ -157,18 +157,11 @@ __global__ __launch_bounds__(kMaxBlock) void predict_hash_k(DevBuffers b, KConst
 // ---------------------------------------------------------------------------
 // a4 part 1: exclusive scan of the per-cell counts into cell offsets
 // (cell c = sorted slots [off[c], off[c+1]); the reference's cellStart/End,
-// reorderDataAndFindCellStartD integration_kernel.cuh:229-299), two passes
-// over tiles of 4096 cells; the counts are cleared for the next build.
-
-__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t *lds4)
-{
-    v = wave_sum(v);
-    const uint32_t w = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) lds4[w] = v;
-    __syncthreads();
-    return lds4[0] + lds4[1] + lds4[2] + lds4[3];
-}
+// reorderDataAndFindCellStartD integration_kernel.cuh:229-299), over tiles of
+// 4096 cells, a block of 1024 threads each.  A block needs the sum of the
+// tiles before its own: of few tiles it adds up the counts themselves, of
+// more it reads their sums, which scan_partials_k forms before.  The counts
+// stay (a block may still read them): the scatter clears those it finds.
 
 __global__ __launch_bounds__(kBlock) void scan_partials_k(const uint32_t *cnt, uint32_t *part,
                                                           uint32_t C)
@@ -181,72 +174,79 @@ __global__ __launch_bounds__(kBlock) void scan_partials_k(const uint32_t *cnt, u
         uint32_t c = base + q * kBlock + threadIdx.x;
         if (c < C) sum += cnt[c];
     }
-    sum = block_sum(sum, lds4);
-    if (threadIdx.x == 0) part[blockIdx.x] = sum;
+    sum = wave_sum(sum);
+    if ((threadIdx.x & 63u) == 0) lds4[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x] = lds4[0] + lds4[1] + lds4[2] + lds4[3];
 }
 
-__global__ __launch_bounds__(kBlock) void scan_final_k(uint32_t *cnt, const uint32_t *part,
-                                                       uint32_t *off, uint32_t C)
+// The tiles up to which the sums are formed from the counts: the last of 32
+// blocks reads 32 tiles of 16 KB from the L2, eight loads in flight, which
+// costs less than a launch: one tile 1.7 us (two launches of 256 threads: 6.7),
+// 8 tiles 5.3 (10.7), 25 tiles 7.4 (9.6).  With 256 tiles the second launch
+// is 5.0 us (6.1 with 256 threads, 16 cells each, through LDS).
+static constexpr uint32_t kScanDirect = 32;
+
+template <bool DIRECT>
+__global__ __launch_bounds__(kScanTile / 4) void scan_k(const uint32_t *cnt, const uint32_t *part, uint32_t *off,
+                                                        uint32_t C)
 {
-    __shared__ uint32_t tile[kScanTile + kScanTile / 16];
-    __shared__ uint32_t lds4[4];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t base = blockIdx.x * kScanTile;
+    constexpr uint32_t kThreads = kScanTile / 4, kWaves = kThreads / 64;
+    __shared__ uint32_t wtot[kWaves], ptot[kWaves];
+    const uint32_t tid = threadIdx.x, w = tid >> 6;
+    const uint32_t c = blockIdx.x * kScanTile + 4u * tid;
+    const bool whole = c < C && C - c >= 4u;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (whole) {
+        v = *reinterpret_cast<const uint4 *>(cnt + c);
+    } else if (c < C) {
+        v.x = cnt[c];
+        if (C - c > 1u) v.y = cnt[c + 1];
+        if (C - c > 2u) v.z = cnt[c + 2];
+    }
     uint32_t pre = 0;
-    for (uint32_t t = tid; t < blockIdx.x; t += kBlock) pre += part[t];
-    pre = block_sum(pre, lds4);
-    // coalesced load (and clear) into LDS; padded index avoids bank conflicts
-#pragma unroll
-    for (uint32_t q = 0; q < kScanPerThread; q++) {
-        uint32_t idx = q * kBlock + tid;
-        uint32_t c = base + idx;
-        uint32_t v = 0;
-        if (c < C) {
-            v = cnt[c];
-            cnt[c] = 0;
+    if (DIRECT) {
+#pragma unroll 8
+        for (uint32_t t = 0; t < blockIdx.x; t++) {
+            const uint4 u = *reinterpret_cast<const uint4 *>(cnt + t * kScanTile + 4u * tid);
+            pre += (u.x + u.y) + (u.z + u.w);
         }
-        tile[idx + (idx >> 4)] = v;
+    } else {
+        for (uint32_t t = tid; t < blockIdx.x; t += kThreads) pre += part[t];
+    }
+    const uint32_t local = (v.x + v.y) + (v.z + v.w);
+    const uint32_t incl = wave_incl_scan(local);
+    pre = wave_sum(pre);
+    if ((tid & 63u) == 63u) {
+        wtot[w] = incl;
+        ptot[w] = pre;
     }
     __syncthreads();
-    uint32_t v[kScanPerThread];
-    uint32_t local = 0;
+    uint32_t run = incl - local;
 #pragma unroll
-    for (uint32_t q = 0; q < kScanPerThread; q++) {
-        uint32_t idx = tid * kScanPerThread + q;
-        v[q] = tile[idx + (idx >> 4)];
-        local += v[q];
+    for (uint32_t q = 0; q < kWaves; q++) run += ptot[q] + (q < w ? wtot[q] : 0u);
+    const uint4 o = make_uint4(run, run + v.x, run + v.x + v.y, run + v.x + v.y + v.z);
+    if (whole) {
+        *reinterpret_cast<uint4 *>(off + c) = o;
+    } else if (c < C) {
+        off[c] = o.x;
+        if (C - c > 1u) off[c + 1] = o.y;
+        if (C - c > 2u) off[c + 2] = o.z;
     }
-    // block exclusive scan of the per-thread totals
-    uint32_t incl = wave_incl_scan(local);
-    const uint32_t w = tid >> 6;
-    __shared__ uint32_t wtot[4];
-    if ((tid & 63) == 63) wtot[w] = incl;
-    __syncthreads();
-    uint32_t wpre = 0;
-    for (uint32_t q = 0; q < w; q++) wpre += wtot[q];
-    uint32_t run = pre + wpre + (incl - local);
-#pragma unroll
-    for (uint32_t q = 0; q < kScanPerThread; q++) {
-        uint32_t idx = tid * kScanPerThread + q;
-        tile[idx + (idx >> 4)] = run;
-        run += v[q];
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t q = 0; q < kScanPerThread; q++) {
-        uint32_t idx = q * kBlock + tid;
-        uint32_t c = base + idx;
-        if (c < C) off[c] = tile[idx + (idx >> 4)];
-    }
-    if (blockIdx.x == gridDim.x - 1 && tid == kBlock - 1) off[C] = run;
+    if (blockIdx.x == gridDim.x - 1 && tid == kThreads - 1) off[C] = run + local;
 }
 
-// a4 part 2: provisional placement by arrival rank (insertion indices only)
+// a4 part 2: provisional placement by arrival rank (insertion indices only).
+// The counts are cleared for the next build here, where nothing reads them:
+// by the first particle of each run of equal keys in a wavefront.
 __global__ __launch_bounds__(kBlock) void scatter_k(DevBuffers b, uint32_t n)
 {
     const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
     if (s >= n) return;
-    const uint32_t t = b.cell_off[b.key[s]] + b.rank[s];
+    const uint32_t key = b.key[s];
+    const uint32_t prev = __shfl_up(key, 1, 64);
+    if ((threadIdx.x & 63u) == 0u || key != prev) b.cell_count[key] = 0;
+    const uint32_t t = b.cell_off[key] + b.rank[s];
     if (t < n)
         b.tmp_orig[t] = b.A[s].orig;
     else
@@ -2079,12 +2079,15 @@ hipError_t launch_predict_hash(hipStream_t st, const DevBuffers &b, const KConst
 hipError_t launch_scan(hipStream_t st, const DevBuffers &b, uint32_t num_cells)
 {
     const uint32_t tiles = scan_tiles(num_cells);
-    hipLaunchKernelGGL(scan_partials_k, dim3(tiles), dim3(kBlock), 0, st, b.cell_count,
-                       b.scan_part, num_cells);
+    const dim3 t(kScanTile / 4);
+    if (tiles <= kScanDirect) {
+        hipLaunchKernelGGL(scan_k<true>, dim3(tiles), t, 0, st, b.cell_count, b.scan_part, b.cell_off, num_cells);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(scan_partials_k, dim3(tiles), dim3(kBlock), 0, st, b.cell_count, b.scan_part, num_cells);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(scan_final_k, dim3(tiles), dim3(kBlock), 0, st, b.cell_count, b.scan_part,
-                       b.cell_off, num_cells);
+    hipLaunchKernelGGL(scan_k<false>, dim3(tiles), t, 0, st, b.cell_count, b.scan_part, b.cell_off, num_cells);
     return hipGetLastError();
 }
 
