@@ -2737,6 +2737,8 @@ int ps_autotune(ps_system *s, float dt, uint32_t substeps, uint32_t *blocks_out)
         if ((rc = timing_collect(s))) { cleanup(); return rc; }
         memcpy(ms0, s->total_ms, sizeof(ms0));
         memcpy(l0, s->launches, sizeof(l0));
+        // the trials launch their substeps themselves (substeps_of): a replayed
+        // graph holds the block sizes and the staging it was captured with
         for (int k : kTunable) {
             if (g_tune.count({k, bucket, feat})) continue;
             uint32_t best = s->block[k];
@@ -2744,11 +2746,11 @@ int ps_autotune(ps_system *s, float dt, uint32_t substeps, uint32_t *blocks_out)
             for (uint32_t bs : kCandidates) {
                 s->block[k] = bs;
                 s->timing = 0;
-                if ((rc = ps_step(s, dt, 1))) break;  // warm-up of this shape
+                if ((rc = substeps_of(s, dt, 1))) break;  // warm-up of this shape
                 s->timing = 1u << k;
                 s->total_ms[k] = 0.0;
                 s->launches[k] = 0;
-                if ((rc = ps_step(s, dt, substeps))) break;
+                if ((rc = substeps_of(s, dt, substeps))) break;
                 if ((rc = timing_collect(s))) break;
                 const double ms = s->launches[k] ? s->total_ms[k] / (double)s->launches[k] : 1e30;
                 if (ms < best_ms) {
@@ -2771,9 +2773,9 @@ int ps_autotune(ps_system *s, float dt, uint32_t substeps, uint32_t *blocks_out)
                 const int choice = round & 1;
                 s->stage_choice = choice;
                 s->timing = 0;
-                if ((rc = ps_step(s, dt, 1))) break;  // warm-up of this choice
+                if ((rc = substeps_of(s, dt, 1))) break;  // warm-up of this choice
                 e = hipEventRecord(e0, s->stream);
-                if (e == hipSuccess && !(rc = ps_step(s, dt, substeps))) {
+                if (e == hipSuccess && !(rc = substeps_of(s, dt, substeps))) {
                     e = hipEventRecord(e1, s->stream);
                     if (e == hipSuccess) e = hipEventSynchronize(e1);
                     float ms = 0.0f;
