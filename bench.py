@@ -94,10 +94,10 @@ def parse():
     return ap.parse_args()
 
 
-KERNEL_OF = {"predict_hash_k": "predict_hash", "scan_partials_k": "scan", "scan_final_k": "scan",
+KERNEL_OF = {"predict_hash_k": "predict_hash", "scan_partials_k": "scan", "scan_k": "scan",
              "scatter_k": "scatter", "reorder_k": "reorder", "neighbors_k": "neighbors",
-             "neighbors_staged_k": "neighbors",
-             "lambda_k": "lambda", "solve_k": "solve", "shape_k": "shape",
+             "neighbors_staged_k": "neighbors", "neighbors_split_k": "neighbors",
+             "lambda_k": "lambda", "solve_k": "solve",
              "finalize_k": "finalize"}
 
 
@@ -278,7 +278,7 @@ def trace_report(stats_csv, trace_csv, log):
     warm, steps = line["warmup"], line["steps"]
     out += ["", "Per-dispatch means over the bench's timed window (substeps %d-%d) from the same "
             "trace, and the bench line this run printed:" % (warm + 1, warm + steps), ""]
-    for name, per in (("solve_k", 4), ("lambda_k", 4), ("shape_k", 4), ("neighbors_", 1),
+    for name, per in (("solve_k", 4), ("lambda_k", 4), ("neighbors_", 1),
                       ("finalize_k", 1), ("reorder_k", 1), ("predict_hash_k", 1)):
         ds = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
               for r in trace if name in r["Kernel_Name"]]
@@ -492,19 +492,18 @@ def copy_calibration(mib):
     print("copy calibration: 3 x %d bytes" % n, file=sys.stderr)
 
 
-def mixed_solve_bytes(K, n, n_nonfluid, n_cloth, n_links, n_rigid):
+def mixed_solve_bytes(K, n, n_nonfluid, n_cloth, n_rigid):
     """Algorithmic bytes of one solve launch on the mixed scene: every
     particle's iterate 16 + attributes 16 + count 4 + K indices + result 16;
-    the contact phases' start position 16 (friction and walls); per cloth
-    particle its constraint range 8 and incidence count 4; per link its
-    pair 8 and (rest, stiffness) 8, gathered from both ends with the id 4
-    and the partner's slot 4 (48 per link); per body member its body, member
-    index and goal 24.  Neighbour records count inside the own reads."""
-    return ((52.0 + 4.0 * K) * n + 16.0 * n_nonfluid + 12.0 * n_cloth + 48.0 * n_links
-            + 24.0 * n_rigid)
+    the contact phases' start position 16 (friction and walls) and contact
+    correction 16; per cloth particle its links' correction 16; per body
+    member its body, member index and goal 24.  Neighbour records count
+    inside the own reads, the constraints' terms with the lambda launch that
+    forms them."""
+    return (52.0 + 4.0 * K) * n + 32.0 * n_nonfluid + 16.0 * n_cloth + 24.0 * n_rigid
 
 
-MIXED_TIMED = ("lambda", "solve", "shape", "neighbors", "finalize")
+MIXED_TIMED = ("lambda", "solve", "neighbors", "finalize")
 
 
 def mixed_main(args):
@@ -559,7 +558,7 @@ def mixed_main(args):
             kernels[name] = {"ms_total": round(ms, 4), "launches": launches,
                              "us_per_launch": round(1000.0 * ms / launches, 3)}
     if "solve" in kernels:
-        b = mixed_solve_bytes(K, N, N - n_fluid, n_cloth, n_links, n_rigid)
+        b = mixed_solve_bytes(K, N, N - n_fluid, n_cloth, n_rigid)
         ach = b / (kernels["solve"]["us_per_launch"] * 1e-6) / 1e9
         roof = {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": None, "kernel": "solve",

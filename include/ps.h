@@ -492,7 +492,7 @@ typedef enum ps_kernel_id {
     PS_K_NEIGHBORS,
     PS_K_LAMBDA,
     PS_K_SOLVE,
-    PS_K_SHAPE,
+    PS_K_SHAPE,         /* no launches: shape matching is part of lambda's */
     PS_K_FINALIZE,
     /* reverse pass (ps_step_backward) */
     PS_K_ADJ_XSPH,
