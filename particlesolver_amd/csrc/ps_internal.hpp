@@ -160,7 +160,10 @@ struct DevBuffers {
     float4 *links;
     float2 *link_own;
     float4 *con_c, *con_d;
-    uint32_t nwalk, nlink, nbody, con_blocks;
+    uint32_t nwalk, nlink, nbody;
+    // a launch's constraint blocks (launch_lambda): the contacts' and the
+    // links' of all, the first and the number in this launch
+    uint32_t con_walks, con_links, con_first, con_blocks;
     SceneDev *scenes;
     // grid
     uint32_t *cell_count;  // num_cells, zero between builds

@@ -22,6 +22,7 @@
 // contiguous range of sorted particles, keeping a spatial region's
 // neighbour data inside one XCD's L2.
 
+#include "ps_blocks.hpp"
 #include "ps_device.hpp"
 
 namespace ps {
@@ -1415,31 +1416,23 @@ __device__ __forceinline__ void constrain_links(const DevBuffers &b, uint32_t q,
     if (!g) b.con_d[i] = make_float4(cx / own.y, cy / own.y, cz / own.y, 0.0f);
 }
 
-// Block bid of the constraint blocks: contacts (eight lanes a particle;
-// lds holds their lists, cap entries a lane), links (four lanes), bodies (a
-// wavefront), the longest chains first.
-__host__ __device__ __forceinline__ uint32_t con_parts(const DevBuffers &b, uint32_t threads, uint32_t &walks, uint32_t &links)
-{
-    walks = (8u * b.nwalk + threads - 1u) / threads;
-    links = (4u * b.nlink + threads - 1u) / threads;
-    return walks + links + (64u * b.nbody + threads - 1u) / threads;
-}
-
+// Block bid of the constraint blocks (con_parts): contacts (lds holds their
+// lists, cap entries a lane), links, bodies, the longest chains first.
 __device__ __forceinline__ void constraint_block(const DevBuffers &b, const KConst &k, uint32_t bid, uint32_t *lds,
                                                  uint32_t cap)
 {
-    uint32_t walks, links;
-    con_parts(b, blockDim.x, walks, links);
-    if (bid < walks) {
+    // the first item of the block, counted in items: bid times the threads
+    // may be past 32 bits
+    if (bid < b.con_walks) {
         // a half's list is its four lanes' share
-        const uint32_t q = (bid * blockDim.x + threadIdx.x) >> 3;
+        const uint32_t q = bid * (blockDim.x >> 3) + (threadIdx.x >> 3);
         if (q < b.nwalk)
             constrain_contacts(b, k, q, threadIdx.x & 7u, lds + (threadIdx.x & ~3u) * cap, 4u * cap);
-    } else if (bid < walks + links) {
-        const uint32_t q = ((bid - walks) * blockDim.x + threadIdx.x) >> 2;
+    } else if (bid - b.con_walks < b.con_links) {
+        const uint32_t q = (bid - b.con_walks) * (blockDim.x >> 2) + (threadIdx.x >> 2);
         if (q < b.nlink) constrain_links(b, q, threadIdx.x & 3u);
     } else {
-        const uint32_t bd = ((bid - walks - links) * blockDim.x + threadIdx.x) >> 6;
+        const uint32_t bd = (bid - b.con_walks - b.con_links) * (blockDim.x >> 6) + (threadIdx.x >> 6);
         if (bd < b.nbody) shape_body(b, bd);
     }
 }
@@ -1459,7 +1452,7 @@ __device__ __forceinline__ void constraint_block(const DevBuffers &b, const KCon
 
 // TAPE (reverse-pass recording): also store S, D and rho per particle.
 // A scene that is not a uniform fluid: the first con_blocks blocks (a multiple
-// of the XCDs) are its constraints' (constraint_block).  Six wavefronts a
+// of the XCDs) are its constraints' from con_first on (constraint_block).  Six wavefronts a
 // SIMD (80 VGPRs) are what three staged blocks a CU take.
 template <bool UNIFORM, bool STAGED, bool TAPE = false>
 __global__ __launch_bounds__(kMaxBlock, UNIFORM ? 1 : 6) void lambda_k(DevBuffers b, KConst k, uint32_t n, float mu)
@@ -1479,10 +1472,10 @@ __global__ __launch_bounds__(kMaxBlock, UNIFORM ? 1 : 6) void lambda_k(DevBuffer
     } else {
         if (blockIdx.x < b.con_blocks) {
             if (STAGED)
-                constraint_block(b, k, blockIdx.x, reinterpret_cast<uint32_t *>(lds4),
+                constraint_block(b, k, b.con_first + blockIdx.x, reinterpret_cast<uint32_t *>(lds4),
                                  4u * kStageSlots / (2u * kStageUnit));
             else
-                constraint_block(b, k, blockIdx.x, contact_lds, kContactList);
+                constraint_block(b, k, b.con_first + blockIdx.x, contact_lds, kContactList);
             return;
         }
         unit = xcd_block(blockIdx.x - b.con_blocks, gridDim.x - b.con_blocks);
@@ -2148,23 +2141,31 @@ hipError_t launch_lambda(hipStream_t st, const DevBuffers &b0, const KConst &k, 
             PS_LAUNCH((lambda_k<true, false>), g, t, 0, st, b0, k, n, mu);
         return hipGetLastError();
     }
-    // the constraint blocks first, in whole turns of the XCDs
+    // the constraint blocks first, as many launches of them alone as it takes
+    // until the rest fits in one with the fluid's
     DevBuffers b = b0;
-    uint32_t walks, links;
-    b.con_blocks = (con_parts(b, threads, walks, links) + 7u) & ~7u;
-    const dim3 g(b.con_blocks + blocks);
+    const ConParts parts = con_parts(b.nwalk, b.nlink, b.nbody, threads);
+    b.con_walks = parts.walks;
+    b.con_links = parts.links;
     // contact lists of the global-slot variants (the staged ones' share the
     // staged cells' LDS)
     const size_t cl = b.nwalk ? sizeof(uint32_t) * kContactList * bs : 0;
-    if (b.tape_lq && b.staging)
-        PS_LAUNCH((lambda_k<false, true, true>), g, t, 0, st, b, k, n, mu);
-    else if (b.tape_lq)
-        PS_LAUNCH((lambda_k<false, false, true>), g, t, cl, st, b, k, n, mu);
-    else if (b.staging)
-        PS_LAUNCH((lambda_k<false, true>), g, t, 0, st, b, k, n, mu);
-    else
-        PS_LAUNCH((lambda_k<false, false>), g, t, cl, st, b, k, n, mu);
-    return hipGetLastError();
+    for (;;) {
+        const ConLaunch part = con_launch(parts.all, b.con_first, blocks, threads);
+        b.con_blocks = part.blocks;
+        const dim3 g(part.blocks + (part.last ? blocks : 0u));
+        if (b.tape_lq && b.staging)
+            PS_LAUNCH((lambda_k<false, true, true>), g, t, 0, st, b, k, n, mu);
+        else if (b.tape_lq)
+            PS_LAUNCH((lambda_k<false, false, true>), g, t, cl, st, b, k, n, mu);
+        else if (b.staging)
+            PS_LAUNCH((lambda_k<false, true>), g, t, 0, st, b, k, n, mu);
+        else
+            PS_LAUNCH((lambda_k<false, false>), g, t, cl, st, b, k, n, mu);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || part.last) return e;
+        b.con_first += part.blocks;
+    }
 }
 
 // NC: tensile exponent known at compile time (4, as in the reference's
