@@ -86,6 +86,7 @@ struct ps_system {
     std::vector<StepGraph> sgraphs;
     float sg_dt = 0.0f;
     uint32_t sg_sub = 0, sg_calls = 0;
+    bool sg_off = false;  // a capture failed: launch until the scene changes (drop_graph)
     // substep state
     uint32_t it_sub = 0;    // iterations done in the open substep
     int stage = 0;          // 1 between predict and end
@@ -431,6 +432,7 @@ void drop_graph(ps_system *s)
     for (ps_system::StepGraph &g : s->sgraphs) (void)hipGraphExecDestroy(g.exec);
     s->sgraphs.clear();
     s->sg_calls = 0;
+    s->sg_off = false;
 }
 
 // ---- timing -------------------------------------------------------------
@@ -1847,9 +1849,9 @@ int capture_substeps(ps_system *s, float dt, uint32_t substeps, hipGraphExec_t *
     const uint64_t sub0 = s->substeps, it0 = s->iters;
     const bool hashed = s->hashed, valid = s->nbr_valid, bnd = s->cr_bnd_done;
     const float dt0 = s->dt;
+    HIP_TRY(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
     const uint32_t timing = s->timing;
     s->timing = 0;  // no event records inside the graph
-    HIP_TRY(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
     const int rc = substeps_of(s, dt, substeps);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(s->stream, &g);
@@ -1892,7 +1894,9 @@ bool same_buffers(DevBuffers a, DevBuffers c)
 // a row captures the next ones, one graph for each arrangement its buffers
 // rotate through (a graph bakes in the pointers it was captured with), which
 // a capture repeats at most kGraphMost times; a call of another dt or
-// length, or any change to the scene (drop_graph), starts over.  Scenes past
+// length, or any change to the scene (drop_graph), starts over.  Where a
+// capture fails (no memory for another graph) the calls launch their substeps
+// as before, until the scene changes.  Scenes past
 // kGraphParticles keep the GPU busy longer than their launches take (131,072
 // particles: 90 us a substep for 35 us of launches).
 constexpr uint32_t kGraphParticles = 65536, kGraphSubsteps = 8, kGraphAfter = 16, kGraphMost = 12;
@@ -1900,7 +1904,7 @@ constexpr uint32_t kGraphParticles = 65536, kGraphSubsteps = 8, kGraphAfter = 16
 // 1: the call's substeps were enqueued; 0: not replayed; < 0: an error
 int step_replayed(ps_system *s, float dt, uint32_t substeps)
 {
-    if (s->n > kGraphParticles || substeps == 0 || substeps > kGraphSubsteps || s->timing ||
+    if (s->n > kGraphParticles || substeps == 0 || substeps > kGraphSubsteps || s->timing || s->sg_off ||
         !s->emitters.empty() || !s->femitters.empty())
         return 0;
     if (s->sg_dt != dt || s->sg_sub != substeps) {
@@ -1921,7 +1925,15 @@ int step_replayed(ps_system *s, float dt, uint32_t substeps)
         if (s->sgraphs.size() >= kGraphMost) return 0;
         ps_system::StepGraph g{};
         g.before = s->b;
-        if (int rc = capture_substeps(s, dt, substeps, &g.exec, &g.after)) return rc;
+        const std::string err = s->err;
+        if (capture_substeps(s, dt, substeps, &g.exec, &g.after)) {
+            // the handle is as it was before: the call launches its substeps,
+            // and if these fail too it reports that
+            (void)hipGetLastError();
+            s->err = err;
+            s->sg_off = true;
+            return 0;
+        }
         s->sgraphs.push_back(g);
         use = &s->sgraphs.back();
     }
