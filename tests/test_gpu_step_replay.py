@@ -88,3 +88,34 @@ def test_two_handles_and_the_2d_solver(gpu_available):
                 refs[1].step(sc.dt, 2)
         same(a, refs[0], "first handle")
         same(b, refs[1], "second handle")
+
+
+@pytest.mark.parametrize("change", ["dt", "length", "params", "tuning", "graph"])
+def test_graphs_let_go_of_while_a_replay_runs(gpu_available, change):
+    """A replayed call is followed at once, with no wait, by one that lets go
+    of the graphs, and the next capture destroys them."""
+    sc = scenes.dam_break(14, 12, 13, max_neighbors=64)
+    ref = load_scene(sc, "f32")
+    with System(sc.params) as g:
+        sc.load_into(g)
+        for block in range(10):
+            dt, sub = sc.dt, 1
+            if change == "dt":
+                dt = sc.dt * (1.0 if block % 2 else 0.75)
+            if change == "length":
+                sub = 1 + block % 2
+            for _ in range(21):
+                g.step(dt, sub)
+                ref.step(dt, sub)
+            if change == "params":
+                g.set_params(sc.params)
+            if change == "tuning":
+                g.set_tuning({"lambda": 64 * (1 + block % 4)})
+            if change == "graph":
+                g.step_graph(0.5 * sc.dt, 4)
+                ref.step(0.5 * sc.dt, 4)
+        same(g, ref, change)
+        g.synchronize()
+        g.step(sc.dt, 1)
+        ref.step(sc.dt, 1)
+        same(g, ref, change + ", after a wait")
