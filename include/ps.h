@@ -365,8 +365,19 @@ int ps_set_velocities(ps_system *sys, uint32_t first, uint32_t n, const float *v
 /* ParticleSystem::update (gpu/src/particlesystem.cpp:144-246) for
  * `substeps` substeps of dt each: predict, grid, neighbours, `iterations`
  * Jacobi iterations, velocity + XSPH.  No dt clamp (the reference clamps to
- * 0.05, :149).  Asynchronous. */
+ * 0.05, :149).  Asynchronous.
+ * A handle of up to 65,536 particles (without emitters, and while no kernel
+ * is timed) that has made the same call, dt and up to 8 substeps alike, 16
+ * times in a row captures the next ones in HIP graphs, one per arrangement of
+ * its buffers (two to six as a rule), and replays them from then on: less
+ * host time a call, the same results.  A capturing call takes 0.1 to 0.7 ms
+ * more once.  Another dt or length, or a change to the scene, its parameters
+ * or tuning, starts the count over; where a capture fails the substeps are
+ * launched. */
 int ps_step(ps_system *sys, float dt, uint32_t substeps);
+/* How many step graphs the handle holds now, and how many ps_step calls a
+ * graph has served (either may be NULL). */
+int ps_step_replays(const ps_system *sys, uint32_t *graphs, uint64_t *calls);
 
 /* The same substep in its stages, for callers that interleave work and for
  * stage-level parity tests:

@@ -167,6 +167,7 @@ PROTOTYPES = {
     "ps_add_rigid_bodies": (_int, [_P, _u32, _P, _P, _P, ctypes.POINTER(_u32)]),
     "ps_set_velocities": (_int, [_P, _u32, _u32, _P]),
     "ps_step": (_int, [_P, _f32, _u32]),
+    "ps_step_replays": (_int, [_P, ctypes.POINTER(_u32), ctypes.POINTER(ctypes.c_uint64)]),
     "ps_substep_begin": (_int, [_P, _f32]),
     "ps_substep_iterate": (_int, [_P]),
     "ps_substep_end": (_int, [_P]),
@@ -473,6 +474,12 @@ class System:
     # -- stepping
     def step(self, dt, substeps=1):
         self._check(self.lib.ps_step(self.h, dt, substeps))
+
+    def step_replays(self):
+        """ps_step_replays: (step graphs held, step calls served by one)"""
+        g, c = ctypes.c_uint32(), ctypes.c_uint64()
+        self._check(self.lib.ps_step_replays(self.h, ctypes.byref(g), ctypes.byref(c)))
+        return g.value, c.value
 
     def step_graph(self, dt, substeps):
         self._check(self.lib.ps_step_graph(self.h, dt, substeps))

@@ -88,6 +88,7 @@ struct ps_system {
     std::vector<StepGraph> sgraphs;
     float sg_dt = 0.0f;
     uint32_t sg_sub = 0, sg_calls = 0;
+    uint64_t sg_replayed = 0;  // calls a graph has served
     bool sg_off = false;  // a capture failed: launch until the scene changes (drop_graph)
     // substep state
     uint32_t it_sub = 0;    // iterations done in the open substep
@@ -1968,6 +1969,7 @@ int step_replayed(ps_system *s, float dt, uint32_t substeps)
     s->iters += (uint64_t)substeps * s->prm.iterations;
     s->hashed = false;
     s->nbr_valid = !s->cpuref;
+    s->sg_replayed++;
     return 1;
 }
 
@@ -1984,6 +1986,14 @@ int ps_step(ps_system *s, float dt, uint32_t substeps)
         if (int rc = emission_check(s, dt, substeps)) return rc;
     const int rc = step_replayed(s, dt, substeps);
     return rc ? (rc < 0 ? rc : (int)PS_OK) : substeps_of(s, dt, substeps);
+}
+
+int ps_step_replays(const ps_system *s, uint32_t *graphs, uint64_t *calls)
+{
+    if (!s) return fail(nullptr, PS_ERR_INVALID_ARGUMENT, "system is NULL");
+    if (graphs) *graphs = (uint32_t)s->sgraphs.size();
+    if (calls) *calls = s->sg_replayed;
+    return PS_OK;
 }
 
 int ps_step_graph(ps_system *s, float dt, uint32_t substeps)

@@ -2,7 +2,11 @@
 per arrangement its buffers rotate through).  Against the FP32 oracle, bit for
 bit, over enough calls that every arrangement is captured and replayed several
 times, with eager work (other step lengths, another dt, changed parameters, a
-graph of ps_step_graph, velocities set, export) between."""
+graph of ps_step_graph, velocities set, export) between; the library's count of
+replayed calls says that they were."""
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 
@@ -33,6 +37,7 @@ def test_replayed_steps_bitexact(gpu_available, iterations, substeps):
                 assert_bitexact(buf.numpy(np.float32, (sc.n, 4))[:, :3], ref.positions(), "export after %d" % call)
         same(g, ref, "replayed")
         assert g.status().substeps == 44 * substeps and g.status().iterations == 44 * substeps * iterations
+        assert g.step_replays()[0] > 0 and g.step_replays()[1] == 44 - 16
 
 
 def test_eager_work_between_replays(gpu_available):
@@ -49,7 +54,9 @@ def test_eager_work_between_replays(gpu_available):
             for _ in range(26):
                 both(lambda s: s.step(sc.dt, 1))
             same(g, ref, "block %d" % block)
+            assert g.step_replays()[0] > 0 and g.step_replays()[1] == 10 * (block + 1)
             both(lambda s: s.step(sc.dt, 2))          # another length starts over
+            assert g.step_replays() == (0, 10 * (block + 1))
             both(lambda s: s.step(0.75 * sc.dt, 1))   # and another dt
             g.step_graph(sc.dt, 12)
             ref.step(sc.dt, 12)
@@ -67,8 +74,10 @@ def test_eager_work_between_replays(gpu_available):
         p.gravity[:] = (1.0, -5.0, 0.0)
         for _ in range(20):
             both(lambda s: s.step(sc.dt, 1))
+        assert g.step_replays()[0] > 0
         g.set_params(p)
         ref.set_params(p)
+        assert g.step_replays()[0] == 0
         for _ in range(24):
             both(lambda s: s.step(sc.dt, 1))
         same(g, ref, "after set_params")
@@ -88,6 +97,96 @@ def test_two_handles_and_the_2d_solver(gpu_available):
                 refs[1].step(sc.dt, 2)
         same(a, refs[0], "first handle")
         same(b, refs[1], "second handle")
+        assert a.step_replays()[1] == 40 - 16 and b.step_replays()[1] == 20 - 16
+
+
+def replay_bitexact(sc, calls, substeps=1):
+    ref = load_scene(sc, "f32")
+    with System(sc.params) as g:
+        sc.load_into(g)
+        for _ in range(calls):
+            g.step(sc.dt, substeps)
+            ref.step(sc.dt, substeps)
+        same(g, ref, "%d calls" % calls)
+        assert g.status().flags == ref.status().flags
+        return g.step_replays()
+
+
+@pytest.mark.parametrize("flags", [0, capi.PS_FLAG_NO_LDS_STAGING, capi.PS_FLAG_REBUILD_EVERY_ITERATION,
+                                   capi.PS_FLAG_SLEEPING])
+@pytest.mark.parametrize("iterations", [3, 4])
+def test_bodies_and_contacts_replayed(gpu_available, flags, iterations):
+    """Cloth and rigid cubes (whose rotations carry over from one replay to
+    the next) falling on two fluids."""
+    sc = scenes.mixed(cloth_n=16, cubes=(2, 1, 2), fluid=(8, 6, 6), box=(5.0, 8.0, 5.0), iterations=iterations)
+    sc.params = sc.params.copy()
+    sc.params.flags |= flags
+    graphs, replayed = replay_bitexact(sc, 48)
+    assert graphs > 0 and replayed == 48 - 16
+
+
+@pytest.mark.parametrize("dims,replays", [((64, 16, 64), True), ((65537, 1, 1), False)])
+def test_largest_replayed_scene(gpu_available, dims, replays):
+    sc = scenes.dam_break(*dims, max_neighbors=64, iterations=2)
+    graphs, replayed = replay_bitexact(sc, 22)
+    assert (graphs > 0, replayed) == ((True, 6) if replays else (False, 0))
+
+
+def test_batch_replayed(gpu_available):
+    b = scenes.ensemble(nscenes=3, nmin=300, nmax=2500)
+    with System(b.params, b.descs) as g, System(b.params, b.descs) as ref:
+        b.load_into(g)
+        b.load_into(ref)
+        for _ in range(40):
+            g.step(b.dt, 1)
+            ref.begin(b.dt)
+            for _ in range(b.params.iterations):
+                ref.iterate()
+            ref.end()
+        same(g, ref, "batch")
+        assert g.step_replays()[1] == 24 and ref.step_replays() == (0, 0)
+
+
+def test_threads_step_while_another_allocates_and_waits(gpu_available):
+    """Handles in threads of their own reach their captures while the main
+    thread allocates, frees and waits for the device."""
+    sc = scenes.dam_break(12, 10, 11, max_neighbors=64)
+    ref = load_scene(sc, "f32")
+    for _ in range(60):
+        ref.step(sc.dt, 1)
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    handles, failures = [System(sc.params) for _ in range(4)], []
+
+    def work(g):
+        try:
+            for _ in range(60):
+                g.step(sc.dt, 1)
+            g.synchronize()
+        except Exception as e:
+            failures.append(e)
+
+    try:
+        for g in handles:
+            sc.load_into(g)
+        threads = [threading.Thread(target=work, args=(g,)) for g in handles]
+        for t in threads:
+            t.start()
+        rounds = 0
+        while any(t.is_alive() for t in threads) or rounds < 20:
+            p = ctypes.c_void_p()
+            assert hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(1 << 20)) == 0
+            assert hip.hipDeviceSynchronize() == 0
+            assert hip.hipFree(p) == 0
+            rounds += 1
+        for t in threads:
+            t.join()
+        assert not failures, failures
+        for g in handles:
+            same(g, ref, "a thread's handle")
+            assert g.step_replays()[1] == 60 - 16
+    finally:
+        for g in handles:
+            g.close()
 
 
 @pytest.mark.parametrize("change", ["dt", "length", "params", "tuning", "graph"])
