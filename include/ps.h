@@ -372,8 +372,8 @@ int ps_set_velocities(ps_system *sys, uint32_t first, uint32_t n, const float *v
  * its buffers (two to six as a rule), and replays them from then on: less
  * host time a call, the same results.  A capturing call takes 0.1 to 0.7 ms
  * more once.  Another dt or length, or a change to the scene, its parameters
- * or tuning, starts the count over; where a capture fails the substeps are
- * launched. */
+ * or tuning, starts the count over; where a capture fails, or the process
+ * holds 1,024 such graphs already, the substeps are launched. */
 int ps_step(ps_system *sys, float dt, uint32_t substeps);
 /* How many step graphs the handle holds now, and how many ps_step calls a
  * graph has served (either may be NULL). */

@@ -11,6 +11,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <string>
 #include <vector>
@@ -73,6 +74,7 @@ struct ps_system {
     uint32_t last_scene = 0;
     // graphs let go of whose last launch may still be running on `stream`
     std::vector<hipGraphExec_t> retired;
+    uint32_t retired_steps = 0;  // of them, graphs of ps_step
     // captured substep graph (ps_step_graph)
     hipGraphExec_t gexec = nullptr;
     DevBuffers g_before;
@@ -428,6 +430,14 @@ void free_all(ps_system *s)
     adj_free(s);
 }
 
+// Graphs of ps_step in the process, replaced ones not yet destroyed among
+// them.  Each holds about 1.5 MiB of device memory (14 launches), so a
+// program of thousands of small handles would lose gigabytes to them: past
+// kGraphsInAll a handle launches, and captures once others have given theirs
+// back.
+constexpr uint32_t kGraphsInAll = 1024;
+std::atomic<uint32_t> g_step_graphs{0};
+
 // Graphs are let go of by calls that do not wait for the GPU (another dt,
 // ps_set_params), and the last launch of one may still be running then.  They
 // are destroyed once the stream has been waited for: by ps_synchronize and
@@ -439,12 +449,23 @@ void free_all(ps_system *s)
 void destroy_retired(ps_system *s)  // nothing runs on the stream
 {
     for (hipGraphExec_t g : s->retired) (void)hipGraphExecDestroy(g);
+    g_step_graphs -= s->retired_steps;
+    s->retired_steps = 0;
     s->retired.clear();
+}
+
+int wait_for_retired(ps_system *s)
+{
+    if (s->retired.empty()) return PS_OK;
+    HIP_TRY(s, hipStreamSynchronize(s->stream));
+    destroy_retired(s);
+    return PS_OK;
 }
 
 void drop_step_graphs(ps_system *s)
 {
     for (ps_system::StepGraph &g : s->sgraphs) s->retired.push_back(g.exec);
+    s->retired_steps += (uint32_t)s->sgraphs.size();
     s->sgraphs.clear();
     s->sg_calls = 0;
 }
@@ -1872,10 +1893,7 @@ int capture_substeps(ps_system *s, float dt, uint32_t substeps, hipGraphExec_t *
     const uint64_t sub0 = s->substeps, it0 = s->iters;
     const bool hashed = s->hashed, valid = s->nbr_valid, bnd = s->cr_bnd_done;
     const float dt0 = s->dt;
-    if (!s->retired.empty()) {
-        HIP_TRY(s, hipStreamSynchronize(s->stream));
-        destroy_retired(s);
-    }
+    if (int rc = wait_for_retired(s)) return rc;
     HIP_TRY(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
     const uint32_t timing = s->timing;
     s->timing = 0;  // no event records inside the graph
@@ -1948,6 +1966,11 @@ int step_replayed(ps_system *s, float dt, uint32_t substeps)
         if (same_buffers(g.before, s->b)) use = &g;
     if (!use) {
         if (s->sgraphs.size() >= kGraphMost) return 0;
+        if (int rc = wait_for_retired(s)) return rc;  // they count
+        if (g_step_graphs.fetch_add(1) >= kGraphsInAll) {
+            g_step_graphs--;
+            return 0;
+        }
         ps_system::StepGraph g{};
         g.before = s->b;
         const std::string err = s->err;
@@ -1955,6 +1978,7 @@ int step_replayed(ps_system *s, float dt, uint32_t substeps)
             // the handle is as it was before: the call launches its substeps,
             // and if these fail too it reports that
             (void)hipGetLastError();
+            g_step_graphs--;
             s->err = err;
             s->sg_off = true;
             return 0;

@@ -218,3 +218,32 @@ def test_graphs_let_go_of_while_a_replay_runs(gpu_available, change):
         g.step(sc.dt, 1)
         ref.step(sc.dt, 1)
         same(g, ref, change + ", after a wait")
+
+
+def test_graphs_of_a_process_are_bounded(gpu_available):
+    """More handles than the process's 1,024 step graphs go round: the last
+    ones launch, and capture once others have closed."""
+    sc = scenes.dam_break(3, 2, 2, max_neighbors=32)
+    ref = load_scene(sc, "f32")
+    handles = []
+    try:
+        for _ in range(300):
+            handles.append(System(sc.params))
+            sc.load_into(handles[-1])
+            for _ in range(24):
+                handles[-1].step(sc.dt, 1)
+        held = [g.step_replays()[0] for g in handles]
+        assert sum(held) == 1024 and held[0] > 0 and held[-1] == 0, held
+        ref.step(sc.dt, 24)
+        for g in (handles[0], handles[-1]):
+            same(g, ref, "24 calls")
+        for g in handles[:10]:
+            g.close()
+        for _ in range(8):
+            handles[-1].step(sc.dt, 1)
+        ref.step(sc.dt, 8)
+        same(handles[-1], ref, "32 calls")
+        assert handles[-1].step_replays()[0] > 0
+    finally:
+        for g in handles:
+            g.close()
