@@ -58,6 +58,7 @@ struct ps_system {
     // the particles that links move (w != 0), ranked as they got their first
     // link, and per insertion index the rank
     std::vector<uint32_t> linked, link_rank;
+    size_t walk_cap = 0, link_cap = 0;  // entries of the lists by rank
     bool any_solid_phase = false;  // SOLID or RIGID particles present
     // host copies of the constraint sets (insertion indices)
     std::vector<uint32_t> dist_pairs;
@@ -843,18 +844,50 @@ int check_sys(ps_system *s)
     return PS_OK;
 }
 
-// Room for the constraint blocks' lists and results, made when the first
-// particle that needs them is added.
-int con_reserve(ps_system *s)
+// Room for the constraint blocks of `need` contact walkers: a rank per
+// insertion index and a result per slot from the first walker on, a slot per
+// walker.  The stream is idle and no graph holds the lists.
+int walk_reserve(ps_system *s, size_t need)
 {
     DevBuffers &b = s->b;
     int rc;
-    for (uint32_t **p : {&b.walk_rank, &b.link_rank, &b.walk_slot, &b.link_slot})
-        if (!*p && (rc = dev_alloc(s, p, s->cap))) return rc;
-    if (!b.link_ends && (rc = dev_alloc(s, &b.link_ends, s->cap))) return rc;
-    if (!b.link_own && (rc = dev_alloc(s, &b.link_own, s->cap))) return rc;
+    if (!b.walk_rank && (rc = dev_alloc(s, &b.walk_rank, s->cap))) return rc;
     if (!b.con_c && (rc = dev_alloc(s, &b.con_c, s->cap))) return rc;
+    if (need <= s->walk_cap) return PS_OK;
+    const size_t cap = std::min<size_t>(s->cap, std::max(need, 2 * s->walk_cap));
+    uint32_t *slot = nullptr;
+    if ((rc = dev_alloc(s, &slot, cap))) return rc;
+    dev_free(b.walk_slot);
+    b.walk_slot = slot;  // written by every sort
+    s->walk_cap = cap;
+    return PS_OK;
+}
+
+// the same for `need` linked particles (link_ends and link_own are uploaded
+// whole after it)
+int link_reserve(ps_system *s, size_t need)
+{
+    DevBuffers &b = s->b;
+    int rc;
+    if (!b.link_rank && (rc = dev_alloc(s, &b.link_rank, s->cap))) return rc;
     if (!b.con_d && (rc = dev_alloc(s, &b.con_d, s->cap))) return rc;
+    if (need <= s->link_cap) return PS_OK;
+    const size_t cap = std::min<size_t>(s->cap, std::max(need, 2 * s->link_cap));
+    uint32_t *slot = nullptr;
+    uint2 *ends = nullptr;
+    float2 *own = nullptr;
+    if ((rc = dev_alloc(s, &slot, cap)) || (rc = dev_alloc(s, &ends, cap)) || (rc = dev_alloc(s, &own, cap))) {
+        dev_free(slot);
+        dev_free(ends);
+        return rc;
+    }
+    dev_free(b.link_slot);
+    dev_free(b.link_ends);
+    dev_free(b.link_own);
+    b.link_slot = slot;
+    b.link_ends = ends;
+    b.link_own = own;
+    s->link_cap = cap;
     return PS_OK;
 }
 
@@ -928,6 +961,7 @@ int upload_constraints(ps_system *s, size_t c0)
         s->link_rank[o] = (uint32_t)s->linked.size();
         s->linked.push_back(o);
     }
+    if (int rc = link_reserve(s, s->linked.size())) return rc;
     std::vector<uint2> ends;
     ends.reserve(s->linked.size());
     for (uint32_t o : s->linked) ends.push_back(make_uint2(off[o], off[o + 1]));
@@ -1520,9 +1554,10 @@ static int add_particles_impl(ps_system *s, uint32_t scene, uint32_t n, const fl
     const size_t o = s->n;
     DevBuffers &b = s->b;
     if (s->cpuref) nwalk = 0;
-    if (nwalk)
-        if (int rc = con_reserve(s)) return rc;
     HIP_TRY(s, hipStreamSynchronize(s->stream));
+    drop_graph(s);
+    if (nwalk)
+        if (int rc = walk_reserve(s, nwalk)) return rc;
     if (nwalk) HIP_TRY(s, hipMemcpy(b.walk_rank + o, walk.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
     HIP_TRY(s, hipMemcpy(b.X + o, X.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
     // the iterate starts equal to the positions (lambda 0)
@@ -1546,7 +1581,6 @@ static int add_particles_impl(ps_system *s, uint32_t scene, uint32_t n, const fl
     }
     s->scene_count[scene] += n;
     s->last_scene = scene;
-    drop_graph(s);
     if (first_out) *first_out = s->n;
     s->n += n;
     s->uniform = uni;
@@ -1581,7 +1615,6 @@ int ps_add_distance_constraints(ps_system *s, uint32_t m, const uint32_t *pairs,
     HIP_TRY(s, hipStreamSynchronize(s->stream));
     drop_graph(s);
     if (int rc = enable_slot_tracking(s)) return rc;
-    if (int rc = con_reserve(s)) return rc;
     const size_t m0 = s->dist_rest.size();
     for (uint32_t k = 0; k < m; k++) {
         s->dist_pairs.push_back(pairs[2 * k]);
