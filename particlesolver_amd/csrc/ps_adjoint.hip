@@ -85,13 +85,6 @@ __device__ __forceinline__ bool adj_contact(const KConst &k, float wi, int32_t p
     return true;
 }
 
-__device__ __forceinline__ void load3(const float4 &v, float *o)
-{
-    o[0] = v.x;
-    o[1] = v.y;
-    o[2] = v.z;
-}
-
 // masked dL/dy of particle i as the Jacobian uses it (z dropped in 2D)
 __device__ __forceinline__ void yd_of(const KConst &k, const float4 &Y, float *yd)
 {

@@ -172,7 +172,6 @@ struct ps_system {
         uint32_t *nc = nullptr;
         float *r0b = nullptr, *wkb = nullptr, *drho = nullptr, *dwk = nullptr, *sb = nullptr;
     } adj;
-    bool adj_active = false;  // inside ps_step_backward: neighbours stay global
 };
 
 namespace {
@@ -2471,10 +2470,8 @@ int ps_step_backward(ps_system *s, float dt, uint32_t substeps, uint32_t checkpo
     }
     const uint32_t K = checkpoint_every >= substeps ? 0u : checkpoint_every;
     drop_graph(s);
-    s->adj_active = true;
     const int rc = step_backward_impl(s, dt, substeps, K, dl_dx, dl_dv, dl_dx0, dl_dv0, dl_drho0,
                                       dl_dstiffness, dl_dmu_k);
-    s->adj_active = false;
     // a failure can leave reverse work queued: let it drain before the
     // workspace is reused
     if (rc && s->rstream) (void)hipStreamSynchronize(s->rstream);

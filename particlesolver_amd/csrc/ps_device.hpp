@@ -151,64 +151,19 @@ __device__ __forceinline__ void for_staged_half_plain(const DevBuffers &b, uint3
             fn((uint32_t)reinterpret_cast<const uint16_t *>(nbr16_chunk(b, i, q >> 2))[q & 3u]);
 }
 
-// Visit the first c neighbours of particle i in table order, calling
-// fn(j, gather(j)) for each.  Software-pipelined: while chunk m is being
-// processed, the four gathers of chunk m+1 and the index load of chunk m+2
-// are already in flight.  The loop is unrolled over two chunks whose record
-// sets swap roles, so no records are copied between registers.  Every entry
-// of a chunk at or below the last one is a valid slot (the builder pads the
-// last chunk with the particle's own slot, or with the sentinel record in a
-// staged unit), so all loads are unconditional; only fn is guarded.
-template <typename G, typename Fn>
-__device__ __forceinline__ void for_neighbors(const DevBuffers &b, uint32_t i, uint32_t c, G gather,
-                                              Fn fn)
-{
-    if (c == 0) return;
-    const uint4 *nb = nbr_lane(b, i);
-    const uint32_t last = (c - 1) >> 2;
-    auto chunk = [&](uint32_t m) { return nb[(size_t)min(m, last) * 64]; };
-    auto visit = [&](const uint4 &jj, uint32_t q, const auto &d0, const auto &d1, const auto &d2,
-                     const auto &d3) {
-        fn(jj.x, d0);
-        if (q + 1 < c) fn(jj.y, d1);
-        if (q + 2 < c) fn(jj.z, d2);
-        if (q + 3 < c) fn(jj.w, d3);
-    };
-    uint4 ja = nb[0];
-    uint4 jb = chunk(1);
-    auto a0 = gather(ja.x);
-    auto a1 = gather(ja.y);
-    auto a2 = gather(ja.z);
-    auto a3 = gather(ja.w);
-    for (uint32_t m = 0;; m += 2) {
-        // records of chunk m are in a*; chunk m+1 goes in flight
-        const uint4 jc = chunk(m + 2);
-        auto b0 = gather(jb.x);
-        auto b1 = gather(jb.y);
-        auto b2 = gather(jb.z);
-        auto b3 = gather(jb.w);
-        visit(ja, m << 2, a0, a1, a2, a3);
-        if (m + 1 > last) break;
-        // chunk m+2 goes in flight into a*; chunk m+1 is processed
-        const uint4 jd = chunk(m + 3);
-        a0 = gather(jc.x);
-        a1 = gather(jc.y);
-        a2 = gather(jc.z);
-        a3 = gather(jc.w);
-        visit(jb, (m + 1) << 2, b0, b1, b2, b3);
-        if (m + 2 > last) break;
-        ja = jc;
-        jb = jd;
-    }
-}
-
 // The fluid sums (density, λ's gradient sums, the Δp sum) are formed in two
 // halves, h = 0 over the table's chunks 0, 2, 4, ... and h = 1 over chunks
 // 1, 3, 5, ..., each in table order, and then added as half 0 + half 1.  The
 // staged kernels give each half its own lane (two lanes per particle, twice
 // the wavefronts for the same LDS); the others visit both halves in turn.
 // Visits the entries of half h of particle i's first c neighbours (global
-// slots), pipelined as for_neighbors.
+// slots) in table order, calling fn(j, gather(j)) for each.
+// Software-pipelined: while chunk m of the half is processed, the four gathers
+// of chunk m + 1 and the index load of chunk m + 2 are already in flight.  The
+// loop is unrolled over two chunks whose record sets swap roles, so no records
+// are copied between registers.  Every entry of a chunk at or below the last
+// one is a valid slot (the builder pads the last chunk with the particle's
+// own), so all loads are unconditional; only fn is guarded.
 template <typename G, typename Fn>
 __device__ __forceinline__ void for_neighbors_half(const DevBuffers &b, uint32_t i, uint32_t c, uint32_t h,
                                                    G gather, Fn fn)
@@ -352,7 +307,7 @@ __device__ __forceinline__ void for_neighbors_half_plain(const DevBuffers &b, ui
         }
 }
 
-// Both halves in one pass, as for_neighbors: fn0 gets the entries of the
+// Both halves in one pass, pipelined as for_neighbors_half: fn0 gets the entries of the
 // even chunks (half 0), fn1 those of the odd chunks (half 1), each half in
 // table order.  The pipelined loop's two record sets hold an even and an
 // odd chunk, so the half of every call is fixed where it is made.
@@ -398,11 +353,6 @@ __device__ __forceinline__ void for_neighbors_split(const DevBuffers &b, uint32_
     }
 }
 
-struct PA {
-    float4 p;
-    Attr a;
-};
-
 struct PX {
     float4 p, x;
 };
@@ -412,12 +362,6 @@ struct PM {
     float4 p;
     float m;
 };
-
-// entry q of particle i (single-entry access for the less travelled loops)
-__device__ __forceinline__ uint32_t nbr_at(const DevBuffers &b, uint32_t i, uint32_t q)
-{
-    return reinterpret_cast<const uint32_t *>(nbr_lane(b, i) + (size_t)(q >> 2) * 64)[q & 3u];
-}
 
 // ---------------------------------------------------------------------------
 // Pair arithmetic shared with the CPU oracle: squared distances and sums use
