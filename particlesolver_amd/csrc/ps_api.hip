@@ -594,8 +594,7 @@ int stage_sort(ps_system *s)
 // Neighbour cells can be staged in LDS (in a batch, the units that lie in
 // one scene), unless the caller turned it off by flag; the autotuner may
 // turn it off too.  (Staged XSPH takes the fluid mass as a constant: with
-// fluid masses that differ, finalize gathers from global memory through
-// the units' chunk tables.)
+// fluid masses that differ, finalize stages each slot's mass as well.)
 bool can_stage(const ps_system *s) { return !s->cpuref && !(s->prm.flags & PS_FLAG_NO_LDS_STAGING); }
 
 bool staging_ok(const ps_system *s) { return can_stage(s) && s->stage_choice != 0; }
@@ -1962,20 +1961,24 @@ bool same_buffers(DevBuffers a, DevBuffers c)
     return memcmp(&a, &c, sizeof(DevBuffers)) == 0;
 }
 
-// A small scene's substeps replayed from graphs.  The launches of a substep
-// of 2,048 particles (15, at 2.3 us each) take the host longer than the GPU
-// needs for them once several handles step at a time: with three handles in
-// turn a substep and two exports took 64 us, replayed 34 (7,096 particles of
-// a mixed scene 81 -> 56, 17,391 of fluid 107 -> 72 for two substeps).  A
-// handle that makes the same call kGraphAfter times in
-// a row captures the next ones, one graph for each arrangement its buffers
-// rotate through (a graph bakes in the pointers it was captured with), which
-// a capture repeats at most kGraphMost times; a call of another dt or
-// length, or any change to the scene (drop_graph), starts over.  Where a
-// capture fails (no memory for another graph) the calls launch their substeps
-// as before, until the scene changes.  Scenes past
-// kGraphParticles keep the GPU busy longer than their launches take (131,072
-// particles: 90 us a substep for 35 us of launches).
+// A small scene's substeps replayed from graphs.  What a replay saves is the
+// host's time for the launches (14 a substep of 2,048 particles, 42 us with
+// two exports, replayed 18), so it shows where the host is what the GPU waits
+// for: three handles stepped and exported in turn took 57 us a pass, replayed
+// 38 (7,096 particles of a mixed scene 57 -> 45; two substeps of 17,391, not
+// exported, 97 -> 66).  One handle alone is bound by its chain of kernels: 83 -> 80
+// us, 123 -> 123, 188 -> 185.
+// A handle that makes the same call kGraphAfter times in a row captures the
+// next ones, one graph for each arrangement its buffers rotate through (a
+// graph bakes in the pointers it was captured with), which a capture repeats
+// at most kGraphMost times; a call of another dt or length, or any change to
+// the scene (drop_graph), starts over.  A capturing call takes 75 to 700 us
+// (launched it took 42 to 110), four in a row as a rule: a program whose dt
+// changes every 20 calls pays about what the launches would have cost, 60
+// against 59 us a call.  Where a capture fails (no memory for another graph)
+// the calls launch their substeps as before, until the scene changes.  Scenes
+// past kGraphParticles keep the GPU busy longer than their launches take
+// (131,072 particles: 88 us a substep for 33 us of launches).
 constexpr uint32_t kGraphParticles = 65536, kGraphSubsteps = 8, kGraphAfter = 16, kGraphMost = 12;
 
 // 1: the call's substeps were enqueued; 0: not replayed; < 0: an error

@@ -890,8 +890,8 @@ __global__ __launch_bounds__(kStageUnit) void neighbors_staged_k(DevBuffers b, K
 
 // The search of a few units, bound by its chain of dependent loads: each
 // unit's particles go to four blocks (each plans the unit for itself), four
-// lanes a particle, lane g over the stencil rows from kRowOf(g) to
-// kRowOf(g + 1).  A lane reads its rows' ranges and the first eight
+// lanes a particle, lane g over the stencil rows from row_of(g) to
+// row_of(g + 1).  A lane reads its rows' ranges and the first eight
 // candidates before the plan, which only the entries need, and from then on
 // the next eight while it tests eight.  A lane's accepted entries go to its
 // list in LDS; the lists of a particle, in lane order, are its table, written
@@ -900,8 +900,13 @@ __global__ __launch_bounds__(kStageUnit) void neighbors_staged_k(DevBuffers b, K
 // With one lane a particle the nine rows follow one another, each waiting
 // for its range and its slots: 20.8 us at 2,048 particles (8 units), now 14.1;
 // 26.3 -> 17.7 at 7,096 of a mixed scene (28 units).  Every lane's loads are
-// its own, so the line lies where the chip begins to fill: at 17,391
-// particles (68 units) 31.5 us against 33.7, at 131,072 (512) 111 against 44.
+// its own, so the gain ends where the chip begins to fill.  Split against one
+// lane after 60 to 80 substeps, in us: 32 units 34.9 / 35.7, 48 35.5 / 35.5, 49
+// 34.1 / 35.0, 55 (mixed) 37.2 / 34.8, 61 (cloth over a pool) 33.6 / 33.8, 64
+// 35.1 / 34.8, 66 (a filled tank) 39.4 / 37.6, 68 38.2 / 36.3, 71 (mixed) 39.4 /
+// 36.6, 96 37.3 / 34.8, 128 37.4 / 34.9, and at 512 111 / 44.  From 32 to 64
+// units it depends on the scene; the line is the last count measured where no
+// scene lost by it.
 
 constexpr uint32_t kNbrParts = 4;                  // blocks per unit
 constexpr uint32_t kNbrOwn = kStageUnit / kNbrParts;
