@@ -36,19 +36,25 @@ TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "traffic_dam_break_1M.md")
 ROOF_KERNELS = ("lambda", "solve")
 TIMING_PERIOD = 7
 
-# Algorithmic bytes per particle per launch, K = neighbour-table length.
-# Each array read once and written once; neighbour positions are counted
-# inside the own-position read.
+# Algorithmic bytes per particle per launch, K = neighbour-table length, e =
+# bytes of a table entry (entry_bytes).  Each array read once and written
+# once; neighbour positions are counted inside the own-position read.
 ALGO_BYTES = {
     # own x,y,z 12 + rho0 4 + count 4 + K indices + lambda out 4
-    "lambda": lambda K: 24.0 + 4.0 * K,
+    "lambda": lambda K, e: 24.0 + e * K,
     # own x,y,z,lambda 16 + rho0 4 + insertion index 4 + count 4 + K indices + x,y,z out 12
-    "solve": lambda K: 40.0 + 4.0 * K,
+    "solve": lambda K, e: 40.0 + e * K,
     # x,y,z 12 + cell key 4 + K indices out + count out 4 (+ cell offsets, ~C/N)
-    "neighbors": lambda K: 20.0 + 4.0 * K,
+    "neighbors": lambda K, e: 20.0 + e * K,
     # p, x*: 24 + rho0 4 + count 4 + K indices + v out 12
-    "finalize": lambda K: 44.0 + 4.0 * K,
+    "finalize": lambda K, e: 44.0 + e * K,
 }
+
+
+def entry_bytes(st):
+    """Mean bytes of a neighbour-table entry under status st: 2 in a staged
+    unit (indices into its LDS), 4 in any other (slots)."""
+    return 4.0 - 2.0 * (st.staged_units / st.units if st.units else 0.0)
 
 
 def parse():
@@ -131,6 +137,7 @@ def traffic_report(fetch_csv, write_csv, log):
         if l.startswith("{") and '"metric"' in l:
             line = json.loads(l)
     N, K = line["config"]["particles"], line["config"]["mean_neighbors"]
+    e = line["roofline"]["entry_bytes"]
     if "adjoint" in line or "batched" in line:
         raise SystemExit("traffic report: the counted run must use --no-adjoint --no-batched (the "
                          "reverse-pass and ensemble workloads launch the same kernels on other scenes)")
@@ -160,14 +167,14 @@ def traffic_report(fetch_csv, write_csv, log):
            "same runs reads FETCH_SIZE %.1f KiB and WRITE_SIZE %.1f KiB for %.1f KiB moved each "
            "way, so FETCH_SIZE is scaled by %.4f and WRITE_SIZE by %.4f."
            % (cal, sum(fcopy) / len(fcopy), sum(wcopy) / len(wcopy), ref_kib, f_scale, w_scale),
-           "N = %d particles, mean neighbour-table length K = %.2f." % (N, K), "",
+           "N = %d particles, mean neighbour-table length K = %.2f, %.2f bytes an entry." % (N, K, e), "",
            "| kernel | FETCH KiB | WRITE KiB | traffic MB/launch | algorithmic MB/launch | traffic / algorithmic |",
            "|---|---:|---:|---:|---:|---:|"]
     table = {}
     for k in sorted(set(fetch) | set(write), key=lambda k: -(fetch.get(k, 0) * f_scale + write.get(k, 0))):
         t = (fetch.get(k, 0.0) * f_scale + write.get(k, 0.0) * w_scale) * 1024.0
         table[k] = int(t)
-        algo = ALGO_BYTES[k](K) * N if k in ALGO_BYTES else None
+        algo = ALGO_BYTES[k](K, e) * N if k in ALGO_BYTES else None
         out.append("| %s | %.1f | %.1f | %.1f | %s | %s |" % (
             k, fetch.get(k, 0.0), write.get(k, 0.0), t / 1e6,
             "%.1f" % (algo / 1e6) if algo else "-", "%.2f" % (t / algo) if algo else "-"))
@@ -492,15 +499,16 @@ def copy_calibration(mib):
     print("copy calibration: 3 x %d bytes" % n, file=sys.stderr)
 
 
-def mixed_solve_bytes(K, n, n_nonfluid, n_cloth, n_rigid):
+def mixed_solve_bytes(K, e, n, n_nonfluid, n_cloth, n_rigid):
     """Algorithmic bytes of one solve launch on the mixed scene: every
-    particle's iterate 16 + attributes 16 + count 4 + K indices + result 16;
+    particle's iterate 16 + attributes 16 + count 4 + K indices of e bytes +
+    result 16;
     the contact phases' start position 16 (friction and walls) and contact
     correction 16; per cloth particle its links' correction 16; per body
     member its body, member index and goal 24.  Neighbour records count
     inside the own reads, the constraints' terms with the lambda launch that
     forms them."""
-    return (52.0 + 4.0 * K) * n + 32.0 * n_nonfluid + 16.0 * n_cloth + 24.0 * n_rigid
+    return (52.0 + e * K) * n + 32.0 * n_nonfluid + 16.0 * n_cloth + 24.0 * n_rigid
 
 
 MIXED_TIMED = ("lambda", "solve", "neighbors", "finalize")
@@ -558,11 +566,12 @@ def mixed_main(args):
             kernels[name] = {"ms_total": round(ms, 4), "launches": launches,
                              "us_per_launch": round(1000.0 * ms / launches, 3)}
     if "solve" in kernels:
-        b = mixed_solve_bytes(K, N, N - n_fluid, n_cloth, n_rigid)
+        e = entry_bytes(st)
+        b = mixed_solve_bytes(K, e, N, N - n_fluid, n_cloth, n_rigid)
         ach = b / (kernels["solve"]["us_per_launch"] * 1e-6) / 1e9
         roof = {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": None, "kernel": "solve",
-                "algo_bytes_per_launch": int(b), "K": round(K, 2)}
+                "algo_bytes_per_launch": int(b), "K": round(K, 2), "entry_bytes": round(e, 3)}
         kernels["solve"]["algo_GBs"] = round(ach, 1)
     cpu = None
     if not args.no_cpu:
@@ -986,13 +995,14 @@ def main():
         timed = {k: v for k, v in kernels.items() if k in ALGO_BYTES}
         dom = max(timed, key=lambda k: timed[k]["ms_total"])
         per_launch_s = timed[dom]["us_per_launch"] * 1e-6
-        bytes_per_launch = ALGO_BYTES[dom](K) * N
+        e = entry_bytes(st)
+        bytes_per_launch = ALGO_BYTES[dom](K, e) * N
         achieved = bytes_per_launch / per_launch_s / 1e9
         roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": quoted_traffic(dom, N),
                 "kernel": dom, "algo_bytes_per_launch": int(bytes_per_launch),
-                "K": round(K, 2)}
+                "K": round(K, 2), "entry_bytes": round(e, 3)}
         # the same launches against the FP32 vector peak (algorithmic flops)
         flops = ALGO_FLOPS_PER_PAIR[dom] * K * N
         tf = flops / per_launch_s / 1e12
@@ -1001,7 +1011,7 @@ def main():
                         "frac": round(tf / FP32_VECTOR_PEAK_TFLOPS, 4)}
         for k in kernels:
             if k in ALGO_BYTES:
-                b = ALGO_BYTES[k](K) * N
+                b = ALGO_BYTES[k](K, e) * N
                 kernels[k]["algo_GBs"] = round(b / (kernels[k]["us_per_launch"] * 1e-6) / 1e9, 1)
 
     if roof is not None:
