@@ -190,7 +190,7 @@ SIMDS, CLOCK_GHZ, VALU_CYCLES = 1024, 2.4, 4.0
 def counter_report(a_csv, b_csv, log):
     """Markdown summary of two rocprofv3 --pmc passes of SQ counters over
     this script (printed to stdout): per kernel, the counts per wavefront and
-    the VALU issue floor, INSTS_VALU x 4 cycles / (1024 SIMDs x 2.4 GHz),
+    the VALU issue time, INSTS_VALU x 4 cycles / (1024 SIMDs x 2.4 GHz),
     against the dispatch's own duration in the same runs."""
     rows = {}
     for f in (a_csv, b_csv):
@@ -215,18 +215,19 @@ def counter_report(a_csv, b_csv, log):
            "Commands (repository root on the GPU host as R, MI355X):", "", "```",
            "cd /tmp && export TMPDIR=/tmp",
            cmd % ("SQ_WAVES SQ_INSTS_VALU SQ_INSTS_SALU SQ_INSTS_LDS SQ_LDS_BANK_CONFLICT SQ_WAIT_INST_LDS "
-                  "SQ_ACTIVE_INST_VALU SQ_WAVE_CYCLES", "A", "A", "A"),
+                  "SQ_ACTIVE_INST_VALU SQ_WAVE_CYCLES GRBM_GUI_ACTIVE", "A", "A", "A"),
            cmd % ("SQ_BUSY_CYCLES SQ_WAIT_INST_ANY SQ_ACTIVE_INST_LDS SQ_ACTIVE_INST_ANY SQ_ACTIVE_INST_SCA "
                   "SQ_WAIT_ANY SQ_INSTS_SMEM SQ_INSTS_VMEM_RD", "B", "B", "B"),
            "cd $R && python3 bench.py --counter-report gpurun_out/pmcA/pmcA_counter_collection.csv "
            "gpurun_out/pmcB/pmcB_counter_collection.csv gpurun_out/pmcA.log", "```", "",
            "13 substeps from rest (K = %.2f neighbours per particle). Counts are means per dispatch divided "
-           "by SQ_WAVES. The VALU floor is the time to issue the dispatch's VALU instructions at one "
-           "wave64 instruction per SIMD every %d cycles on all %d SIMDs at %.1f GHz (FP32 without packed "
-           "math); a kernel whose duration is close to it is VALU-issue-bound. Durations are the "
-           "dispatches' own under the counters (kernels run one at a time)." % (K, VALU_CYCLES, SIMDS, CLOCK_GHZ),
+           "by SQ_WAVES. The issue time is that of the dispatch's VALU instructions at one wave64 "
+           "instruction per SIMD every %d cycles on all %d SIMDs at %.1f GHz (FP32 without packed math). A "
+           "kernel whose duration is close to it is bound by VALU issue. It is no floor: the neighbour build "
+           "takes less than it, so some instructions issue faster than that. Durations are the dispatches' own "
+           "under the counters (kernels run one at a time)." % (K, VALU_CYCLES, SIMDS, CLOCK_GHZ),
            "", "| kernel | waves | VALU / wave | SALU / wave | LDS / wave | VMEM rd / wave | "
-           "LDS bank conflict cycles / wave | mean us | VALU floor us | floor / duration |",
+           "LDS bank conflict cycles / wave | mean us | VALU issue us | issue / duration |",
            "|---|---:|---:|---:|---:|---:|---:|---:|---:|---:|"]
     for k, d in sorted(rows.items(), key=lambda kv: -sum(kv[1]["dur"])):
         c = {n: sum(v) / len(v) for n, v in d["c"].items()}
@@ -234,10 +235,10 @@ def counter_report(a_csv, b_csv, log):
         if w <= 0:
             continue
         dur = sum(d["dur"]) / len(d["dur"])
-        floor = c.get("SQ_INSTS_VALU", 0.0) * VALU_CYCLES / (SIMDS * CLOCK_GHZ * 1e3)
+        issue = c.get("SQ_INSTS_VALU", 0.0) * VALU_CYCLES / (SIMDS * CLOCK_GHZ * 1e3)
         out.append("| `%s` | %.0f | %.1f | %.1f | %.1f | %.1f | %.1f | %.1f | %.1f | %.2f |" % (
             k, w, c.get("SQ_INSTS_VALU", 0) / w, c.get("SQ_INSTS_SALU", 0) / w, c.get("SQ_INSTS_LDS", 0) / w,
-            c.get("SQ_INSTS_VMEM_RD", 0) / w, c.get("SQ_LDS_BANK_CONFLICT", 0) / w, dur, floor, floor / dur))
+            c.get("SQ_INSTS_VMEM_RD", 0) / w, c.get("SQ_LDS_BANK_CONFLICT", 0) / w, dur, issue, issue / dur))
     print("\n".join(out))
 
 
