@@ -14,6 +14,7 @@
 #include <atomic>
 #include <map>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "ps_internal.hpp"
@@ -1955,6 +1956,7 @@ int capture_substeps(ps_system *s, float dt, uint32_t substeps, hipGraphExec_t *
 
 // the same buffers in the same places; the staging mode is whatever the
 // last neighbour build chose
+static_assert(std::has_unique_object_representations_v<DevBuffers>, "DevBuffers are compared as bytes");
 bool same_buffers(DevBuffers a, DevBuffers c)
 {
     a.staging = c.staging = 0;

@@ -28,6 +28,13 @@ constexpr ConParts con_parts(uint32_t nwalk, uint32_t nlink, uint32_t nbody, uin
     return ConParts{w, l, (w + l + item_blocks(nbody, 64u, threads) + 7u) & ~7u};
 }
 
+// What a lambda launch is told of them (an argument of its own: the buffers go
+// to every kernel): the walkers' and the links' of all, the first of this
+// launch and how many.
+struct ConBlocks {
+    uint32_t walks, links, first, blocks;
+};
+
 // A launch holds fewer than 2^32 threads.  Of `all` constraint blocks and
 // `fluid` blocks after them, those from `first` on: the next launch's
 // constraint blocks, and whether the fluid's are in it (then it is the last).

@@ -140,7 +140,6 @@ struct DevBuffers {
     uint32_t *tmp_orig;    // insertion index by provisional sorted slot
     uint32_t *slot_of;     // insertion index -> current slot (kept only while
                            // track_slots: distance constraints or bodies exist)
-    uint32_t track_slots;
     uint32_t *sid, *sid2;  // scene of each slot (batches only)
     float *mj;             // per slot, written by the sort for scenes that are not
                            // a uniform fluid: the particle's density mass as a
@@ -160,10 +159,6 @@ struct DevBuffers {
     float4 *links;
     float2 *link_own;
     float4 *con_c, *con_d;
-    uint32_t nwalk, nlink, nbody;
-    // a launch's constraint blocks (launch_lambda): the contacts' and the
-    // links' of all, the first and the number in this launch
-    uint32_t con_walks, con_links, con_first, con_blocks;
     SceneDev *scenes;
     // grid
     uint32_t *cell_count;  // num_cells, zero between builds
@@ -175,7 +170,6 @@ struct DevBuffers {
     uint32_t *ncnt;
     uint32_t *nbr_glob;    // recording a substep for the reverse pass with staging:
                            // the same table with global slots (else null)
-    uint32_t kq;  // max_neighbors / 4
     // distance constraints (insertion-index CSR)
     uint32_t *dist_off;    // max_particles + 1
     uint32_t *link_id;     // 2*m: 2 * constraint + (1 for its second particle)
@@ -196,7 +190,11 @@ struct DevBuffers {
     DevStatus *status;
     // LDS staging of neighbour cells: one descriptor per unit
     StageDesc *stage;
+    // no padding between them: step graphs are told apart by the bytes
     uint32_t staging;      // 1: the last neighbour build staged its units
+    uint32_t kq;           // max_neighbors / 4
+    uint32_t track_slots;
+    uint32_t nwalk, nlink, nbody;
     // adjoint recompute only (else null): per particle, the coordinates the
     // walls and pins set and the wall-friction branch (walls() bits)
     uint8_t *clamp_rec;

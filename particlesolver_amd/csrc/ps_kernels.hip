@@ -1423,21 +1423,22 @@ __device__ __forceinline__ void constrain_links(const DevBuffers &b, uint32_t q,
 
 // Block bid of the constraint blocks (con_parts): contacts (lds holds their
 // lists, cap entries a lane), links, bodies, the longest chains first.
-__device__ __forceinline__ void constraint_block(const DevBuffers &b, const KConst &k, uint32_t bid, uint32_t *lds,
-                                                 uint32_t cap)
+__device__ __forceinline__ void constraint_block(const DevBuffers &b, const KConst &k, const ConBlocks &con,
+                                                 uint32_t *lds, uint32_t cap)
 {
+    const uint32_t bid = con.first + blockIdx.x;
     // the first item of the block, counted in items: bid times the threads
     // may be past 32 bits
-    if (bid < b.con_walks) {
+    if (bid < con.walks) {
         // a half's list is its four lanes' share
         const uint32_t q = bid * (blockDim.x >> 3) + (threadIdx.x >> 3);
         if (q < b.nwalk)
             constrain_contacts(b, k, q, threadIdx.x & 7u, lds + (threadIdx.x & ~3u) * cap, 4u * cap);
-    } else if (bid - b.con_walks < b.con_links) {
-        const uint32_t q = (bid - b.con_walks) * (blockDim.x >> 2) + (threadIdx.x >> 2);
+    } else if (bid - con.walks < con.links) {
+        const uint32_t q = (bid - con.walks) * (blockDim.x >> 2) + (threadIdx.x >> 2);
         if (q < b.nlink) constrain_links(b, q, threadIdx.x & 3u);
     } else {
-        const uint32_t bd = (bid - b.con_walks - b.con_links) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+        const uint32_t bd = (bid - con.walks - con.links) * (blockDim.x >> 6) + (threadIdx.x >> 6);
         if (bd < b.nbody) shape_body(b, bd);
     }
 }
@@ -1456,11 +1457,12 @@ __device__ __forceinline__ void constraint_block(const DevBuffers &b, const KCon
 // UNIFORM: every particle is fluid with inverse mass wu (no Attr gathers).
 
 // TAPE (reverse-pass recording): also store S, D and rho per particle.
-// A scene that is not a uniform fluid: the first con_blocks blocks (a multiple
-// of the XCDs) are its constraints' from con_first on (constraint_block).  Six wavefronts a
+// A scene that is not a uniform fluid: the first con.blocks blocks (a multiple
+// of the XCDs) are its constraints' from con.first on (constraint_block).  Six wavefronts a
 // SIMD (80 VGPRs) are what three staged blocks a CU take.
 template <bool UNIFORM, bool STAGED, bool TAPE = false>
-__global__ __launch_bounds__(kMaxBlock, UNIFORM ? 1 : 6) void lambda_k(DevBuffers b, KConst k, uint32_t n, float mu)
+__global__ __launch_bounds__(kMaxBlock, UNIFORM ? 1 : 6) void lambda_k(DevBuffers b, KConst k, uint32_t n, float mu,
+                                                                       ConBlocks con)
 {
     // staged: a uniform fluid stages neighbour positions only, 12 bytes
     // per slot (36 KB, so four blocks fit in a CU's LDS where 16-byte slots
@@ -1475,15 +1477,14 @@ __global__ __launch_bounds__(kMaxBlock, UNIFORM ? 1 : 6) void lambda_k(DevBuffer
     if constexpr (UNIFORM) {
         unit = xcd_block();
     } else {
-        if (blockIdx.x < b.con_blocks) {
+        if (blockIdx.x < con.blocks) {
             if (STAGED)
-                constraint_block(b, k, b.con_first + blockIdx.x, reinterpret_cast<uint32_t *>(lds4),
-                                 4u * kStageSlots / (2u * kStageUnit));
+                constraint_block(b, k, con, reinterpret_cast<uint32_t *>(lds4), 4u * kStageSlots / (2u * kStageUnit));
             else
-                constraint_block(b, k, b.con_first + blockIdx.x, contact_lds, kContactList);
+                constraint_block(b, k, con, contact_lds, kContactList);
             return;
         }
-        unit = xcd_block(blockIdx.x - b.con_blocks, gridDim.x - b.con_blocks);
+        unit = xcd_block(blockIdx.x - con.blocks, gridDim.x - con.blocks);
     }
     const uint32_t hh = STAGED ? (threadIdx.x & 1u) : 0u;
     const uint32_t i = STAGED ? unit * kStageUnit + (threadIdx.x >> 1) : unit * blockDim.x + threadIdx.x;
@@ -2125,51 +2126,51 @@ hipError_t launch_neighbors(hipStream_t st, const DevBuffers &b, const KConst &k
     return hipGetLastError();
 }
 
-hipError_t launch_lambda(hipStream_t st, const DevBuffers &b0, const KConst &k, uint32_t n,
+hipError_t launch_lambda(hipStream_t st, const DevBuffers &b, const KConst &k, uint32_t n,
                          bool uniform, float wu, uint32_t bs)
 {
     if (n == 0) return hipSuccess;
     const float mu = 1.0f / wu;
     // staged: two lanes per particle
-    const uint32_t threads = b0.staging ? 2u * kStageUnit : bs;
-    const uint32_t blocks = blocks_for(n, b0.staging ? kStageUnit : bs);
+    const uint32_t threads = b.staging ? 2u * kStageUnit : bs;
+    const uint32_t blocks = blocks_for(n, b.staging ? kStageUnit : bs);
     const dim3 t(threads);
+    ConBlocks con{};
     if (uniform) {
         const dim3 g(blocks);
-        if (b0.tape_lq && b0.staging)  // recording for the reverse pass
-            PS_LAUNCH((lambda_k<true, true, true>), g, t, 0, st, b0, k, n, mu);
-        else if (b0.tape_lq)
-            PS_LAUNCH((lambda_k<true, false, true>), g, t, 0, st, b0, k, n, mu);
-        else if (b0.staging)
-            PS_LAUNCH((lambda_k<true, true>), g, t, 0, st, b0, k, n, mu);
+        if (b.tape_lq && b.staging)  // recording for the reverse pass
+            PS_LAUNCH((lambda_k<true, true, true>), g, t, 0, st, b, k, n, mu, con);
+        else if (b.tape_lq)
+            PS_LAUNCH((lambda_k<true, false, true>), g, t, 0, st, b, k, n, mu, con);
+        else if (b.staging)
+            PS_LAUNCH((lambda_k<true, true>), g, t, 0, st, b, k, n, mu, con);
         else
-            PS_LAUNCH((lambda_k<true, false>), g, t, 0, st, b0, k, n, mu);
+            PS_LAUNCH((lambda_k<true, false>), g, t, 0, st, b, k, n, mu, con);
         return hipGetLastError();
     }
     // the constraint blocks first, as many launches of them alone as it takes
     // until the rest fits in one with the fluid's
-    DevBuffers b = b0;
     const ConParts parts = con_parts(b.nwalk, b.nlink, b.nbody, threads);
-    b.con_walks = parts.walks;
-    b.con_links = parts.links;
+    con.walks = parts.walks;
+    con.links = parts.links;
     // contact lists of the global-slot variants (the staged ones' share the
     // staged cells' LDS)
     const size_t cl = b.nwalk ? sizeof(uint32_t) * kContactList * bs : 0;
     for (;;) {
-        const ConLaunch part = con_launch(parts.all, b.con_first, blocks, threads);
-        b.con_blocks = part.blocks;
+        const ConLaunch part = con_launch(parts.all, con.first, blocks, threads);
+        con.blocks = part.blocks;
         const dim3 g(part.blocks + (part.last ? blocks : 0u));
         if (b.tape_lq && b.staging)
-            PS_LAUNCH((lambda_k<false, true, true>), g, t, 0, st, b, k, n, mu);
+            PS_LAUNCH((lambda_k<false, true, true>), g, t, 0, st, b, k, n, mu, con);
         else if (b.tape_lq)
-            PS_LAUNCH((lambda_k<false, false, true>), g, t, cl, st, b, k, n, mu);
+            PS_LAUNCH((lambda_k<false, false, true>), g, t, cl, st, b, k, n, mu, con);
         else if (b.staging)
-            PS_LAUNCH((lambda_k<false, true>), g, t, 0, st, b, k, n, mu);
+            PS_LAUNCH((lambda_k<false, true>), g, t, 0, st, b, k, n, mu, con);
         else
-            PS_LAUNCH((lambda_k<false, false>), g, t, cl, st, b, k, n, mu);
+            PS_LAUNCH((lambda_k<false, false>), g, t, cl, st, b, k, n, mu, con);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess || part.last) return e;
-        b.con_first += part.blocks;
+        con.first += part.blocks;
     }
 }
 
