@@ -153,15 +153,15 @@ def traffic_report(fetch_csv, write_csv, log):
     out = ["# HBM traffic per launch, 1M-particle dam break", "",
            "Commands (repository root on the GPU host, R = its absolute path):", "",
            "    cd /tmp && export TMPDIR=/tmp",
-           "    rocprofv3 --pmc FETCH_SIZE --output-format csv -d $R/gpurun_out/pmc_fetch -o fetch "
+           "    rocprofv3 --pmc FETCH_SIZE --output-format csv -d $R/out/pmc_fetch -o fetch "
            "-- python3 $R/bench.py --steps 5 --warmup 2 --no-cpu --no-adjoint --no-batched --breakdown 0 "
-           "--copy-calibration 512 > $R/gpurun_out/pmc_fetch.log 2>&1",
-           "    rocprofv3 --pmc WRITE_SIZE --output-format csv -d $R/gpurun_out/pmc_write -o write "
+           "--copy-calibration 512 > $R/out/pmc_fetch.log 2>&1",
+           "    rocprofv3 --pmc WRITE_SIZE --output-format csv -d $R/out/pmc_write -o write "
            "-- python3 $R/bench.py --steps 5 --warmup 2 --no-cpu --no-adjoint --no-batched --breakdown 0 "
-           "--copy-calibration 512 > $R/gpurun_out/pmc_write.log 2>&1",
+           "--copy-calibration 512 > $R/out/pmc_write.log 2>&1",
            "    cd $R && python3 bench.py --traffic-report "
-           "gpurun_out/pmc_fetch/fetch_counter_collection.csv "
-           "gpurun_out/pmc_write/write_counter_collection.csv gpurun_out/pmc_fetch.log", "",
+           "out/pmc_fetch/fetch_counter_collection.csv "
+           "out/pmc_write/write_counter_collection.csv out/pmc_fetch.log", "",
            "Counters: rocprofv3 FETCH_SIZE and WRITE_SIZE (KiB per dispatch), one run each.",
            "Calibration: the runtime copy kernel of a %d-byte hipMemcpy (device to device) in the "
            "same runs reads FETCH_SIZE %.1f KiB and WRITE_SIZE %.1f KiB for %.1f KiB moved each "
@@ -208,9 +208,9 @@ def counter_report(a_csv, b_csv, log):
         if l.startswith("{") and '"metric"' in l:
             line = json.loads(l)
     K = line["config"]["mean_neighbors"]
-    cmd = ("timeout -s KILL 150 rocprofv3 --pmc %s --output-format csv -d $R/gpurun_out/pmc%s -o pmc%s -- "
+    cmd = ("timeout -s KILL 150 rocprofv3 --pmc %s --output-format csv -d $R/out/pmc%s -o pmc%s -- "
            "python3 $R/bench.py --steps 10 --warmup 3 --no-cpu --no-adjoint --no-batched --breakdown 0 "
-           "> $R/gpurun_out/pmc%s.log 2>&1")
+           "> $R/out/pmc%s.log 2>&1")
     out = ["# SQ counters per wavefront: 1,048,576-particle PBF dam break", "",
            "Commands (repository root on the GPU host as R, MI355X):", "", "```",
            "cd /tmp && export TMPDIR=/tmp",
@@ -218,8 +218,8 @@ def counter_report(a_csv, b_csv, log):
                   "SQ_ACTIVE_INST_VALU SQ_WAVE_CYCLES GRBM_GUI_ACTIVE", "A", "A", "A"),
            cmd % ("SQ_BUSY_CYCLES SQ_WAIT_INST_ANY SQ_ACTIVE_INST_LDS SQ_ACTIVE_INST_ANY SQ_ACTIVE_INST_SCA "
                   "SQ_WAIT_ANY SQ_INSTS_SMEM SQ_INSTS_VMEM_RD", "B", "B", "B"),
-           "cd $R && python3 bench.py --counter-report gpurun_out/pmcA/pmcA_counter_collection.csv "
-           "gpurun_out/pmcB/pmcB_counter_collection.csv gpurun_out/pmcA.log", "```", "",
+           "cd $R && python3 bench.py --counter-report out/pmcA/pmcA_counter_collection.csv "
+           "out/pmcB/pmcB_counter_collection.csv out/pmcA.log", "```", "",
            "13 substeps from rest (K = %.2f neighbours per particle). Counts are means per dispatch divided "
            "by SQ_WAVES. The issue time is that of the dispatch's VALU instructions at one wave64 "
            "instruction per SIMD every %d cycles on all %d SIMDs at %.1f GHz (FP32 without packed math). A "
@@ -274,9 +274,9 @@ def trace_report(stats_csv, trace_csv, log):
     out = ["# Kernel durations: %s (rocprofv3 kernel trace)" % title, "",
            "Commands (repository root on the GPU host as R, MI355X):", "", "```",
            "cd /tmp && export TMPDIR=/tmp && rocprofv3 --kernel-trace --stats --output-format csv "
-           "-d /tmp/%s -o kt -- python3 $R/bench.py %s > $R/gpurun_out/%s.log 2>&1" % (d, run, d),
+           "-d /tmp/%s -o kt -- python3 $R/bench.py %s > $R/out/%s.log 2>&1" % (d, run, d),
            "cd $R && python3 bench.py --trace-report /tmp/%s/kt_kernel_stats.csv "
-           "/tmp/%s/kt_kernel_trace.csv gpurun_out/%s.log" % (d, d, d), "```", "", what,
+           "/tmp/%s/kt_kernel_trace.csv out/%s.log" % (d, d, d), "```", "", what,
            "", "| kernel | calls | avg us | min us | max us | share |", "|---|---|---|---|---|---|"]
     for r in sorted(rows, key=lambda r: -float(r["TotalDurationNs"])):
         out.append("| `%s` | %s | %.1f | %.1f | %.1f | %.1f %% |" % (
@@ -313,9 +313,9 @@ def _trace_report_ensemble(rows, tot, line, trace_csv):
            "Commands (repository root on the GPU host as R, MI355X):", "", "```",
            "cd /tmp && export TMPDIR=/tmp && rocprofv3 --kernel-trace --stats --output-format csv "
            "-d /tmp/kte -o kte -- python3 $R/bench.py --workload ensemble --steps %d "
-           "> $R/gpurun_out/kte.log 2>&1" % c["timed_substeps"],
+           "> $R/out/kte.log 2>&1" % c["timed_substeps"],
            "cd $R && python3 bench.py --trace-report /tmp/kte/kte_kernel_stats.csv "
-           "/tmp/kte/kte_kernel_trace.csv gpurun_out/kte.log", "```", "",
+           "/tmp/kte/kte_kernel_trace.csv out/kte.log", "```", "",
            "%s. One handle steps all scenes with one launch per stage, %d substeps per captured "
            "graph: one warm-up replay, then %d timed replays. Then the same scenes as %d separate "
            "handles, twice issued back to back and once one after another (the rows below "
@@ -381,9 +381,9 @@ def _trace_report_adjoint(rows, tot, line):
            "Commands (repository root on the GPU host as R, MI355X):", "", "```",
            "cd /tmp && export TMPDIR=/tmp && rocprofv3 --kernel-trace --stats --output-format csv "
            "-d /tmp/kta -o kta -- python3 $R/bench.py --workload adjoint_cloth_pool --no-cpu "
-           "> $R/gpurun_out/kta.log 2>&1",
+           "> $R/out/kta.log 2>&1",
            "cd $R && python3 bench.py --trace-report /tmp/kta/kta_kernel_stats.csv "
-           "/tmp/kta/kta_kernel_trace.csv gpurun_out/kta.log", "```", "",
+           "/tmp/kta/kta_kernel_trace.csv out/kta.log", "```", "",
            "%s. The run holds one forward pass for the target (perturbed parameters), warm-up, "
            "one timed forward pass, four reverse passes (two with checkpoints every %d "
            "substeps, two with the whole horizon on tape) and one more with events on every "

@@ -501,7 +501,8 @@ typedef enum ps_kernel_id {
     PS_K_SCATTER,
     PS_K_REORDER,
     PS_K_NEIGHBORS,
-    PS_K_LAMBDA,
+    PS_K_LAMBDA,        /* in a scene that is not a uniform fluid with the blocks of
+                         * its contacts, distance constraints and bodies */
     PS_K_SOLVE,
     PS_K_SHAPE,         /* no launches: shape matching is part of lambda's */
     PS_K_FINALIZE,
